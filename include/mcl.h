@@ -123,9 +123,12 @@ int         mcl_cluster_limits(const void* ctx, int32_t* max_electrons, int32_t*
  *                     searched by the whole wave, up to four at a time, up
  *                     to this many, lane-parallel beyond (default 32, at
  *                     most 64).
- *   "lookahead_max"   with at most this many live electrons in a cluster, the
- *                     wave tests the next 64 steps at once and skips those in
- *                     which no electron can fire (default 8; 0 turns it off).
+ *   "lookahead_max" (default 8), "fixed_thresholds" and "quiet_window" (0 or 1,
+ *                     default 1): accepted, checked and read back for programs and
+ *                     tables that set them, with no effect: they chose between ways
+ *                     of skipping steps in which no electron fires, and every
+ *                     fixed-dt launch now simulates only the steps in which one
+ *                     does (first-fire windows).
  *   "waves_per_cluster" wavefronts per fixed-dt cluster: 1, 2, 4 or 8 (the waves
  *                     split the cluster's 64-electron rows, at most 64 rows a
  *                     wave, so clusters above 4096 electrons take at least the
@@ -136,18 +139,6 @@ int         mcl_cluster_limits(const void* ctx, int32_t* max_electrons, int32_t*
  *                     cluster's holes in the global-memory form (results
  *                     identical, slower); 0 (default): only clusters that do
  *                     not fit LDS.
- *   "fixed_thresholds" 1 (default): a fixed-dt launch (or size class) with an
- *                     isothermal one-localisation-channel run takes the kernels
- *                     that keep each electron's fire threshold in its w slot;
- *                     0: the kernels that compute it from w every step (results
- *                     identical; ramped and two-channel launches always take
- *                     those).
- *   "quiet_window"    1 (default): fixed-dt launches (or size classes) with a
- *                     ramped run take the kernels with the quiet window: after
- *                     two steps in which no electron fired, the steps left in
- *                     the Philox block (up to three) are tested at once and
- *                     skipped together when no electron fires in them; 0: the
- *                     kernels without it (results identical).
  * No counterpart in the reference (it has no kernels); the autotuner
  * (mcluminescence_amd/autotune.py) sets them. */
 int         mcl_tune_set(void* ctx, const char* key, double value);

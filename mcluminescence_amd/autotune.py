@@ -7,8 +7,6 @@ The kernels' results do not depend on the tuning knobs (mcl_tune_set):
   wave_search_max  queue length up to which a step's nearest-hole searches run
                    wave-cooperatively (four electrons at a time) rather than
                    lane-parallel
-  lookahead_max    live electrons up to which a cluster tests 64 steps at once and
-                   skips the quiet ones
   persist_frac     persistent workgroups per size class, as a fraction of what
                    fits on the device at once (load balance against contention
                    between concurrently running class kernels)
@@ -36,7 +34,7 @@ TABLE = Path(__file__).resolve().parent / "tuning" / "table.json"
 DEFAULTS = {"holes_per_cell": 2.0, "persist_frac": 1.0, "wave_search_max": 32.0,
             "lookahead_max": 8.0, "waves_per_cluster": 0.0}
 SPACE = {"holes_per_cell": [2.0, 2.5, 3.0, 4.0], "persist_frac": [1.0, 2.0],
-         "wave_search_max": [8.0, 32.0, 64.0], "lookahead_max": [0.0, 4.0, 8.0, 32.0],
+         "wave_search_max": [8.0, 32.0, 64.0], "lookahead_max": [8.0],
          "waves_per_cluster": [0.0, 1.0]}
 
 

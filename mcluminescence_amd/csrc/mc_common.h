@@ -88,15 +88,15 @@ __device__ __forceinline__ uint64_t block_search_lane(const Grid& g, float x, fl
               cz = cell_of(z, g.inv_cell, G);
     const int x0 = max(cx - RAD, 0), x1 = min(cx + RAD, G - 1);
     uint64_t key = ~0ull;
-#pragma unroll
+    // (a loop: unrolled, its nine copies at every call are most of a kernel's code)
+#pragma unroll 1
     for (int k = 0; k < W * W; ++k) {
         const int zz = cz + k / W - RAD, yy = cy + k % W - RAD;
-        int s = 0, e = 0;
-        if ((unsigned)zz < (unsigned)G && (unsigned)yy < (unsigned)G) {
-            const int base = (zz * G + yy) * G;
-            s = (int)g.cstart[base + x0];
-            e = (int)g.cstart[base + x1 + 1];
-        }
+        // rows outside the grid are empty: the reads go to the nearest row inside
+        const bool in = (unsigned)zz < (unsigned)G && (unsigned)yy < (unsigned)G;
+        const int base = (min(max(zz, 0), G - 1) * G + min(max(yy, 0), G - 1)) * G;
+        const int s = (int)g.cstart[base + x0], s1 = (int)g.cstart[base + x1 + 1];
+        const int e = in ? s1 : s;
         evals += (uint64_t)(e - s);
         for (int i0 = s; i0 < e; i0 += kChunk) {
             float4 hv[kChunk];
@@ -203,44 +203,51 @@ __device__ __forceinline__ uint64_t block_search_rows(const Grid& g, int nb, flo
     const int q = lane & 15;
     const bool act = (lane >> 4) < nb;
     int s[9], e[9];
-    int longest = 0;
-    if (act) {
-        const Block k(g, x, y, z);
-        const int cz = cell_of(z, g.inv_cell, G), cy = cell_of(y, g.inv_cell, G);
-        int total = 0;
+    int longest = 0, total = 0;
+    const Block k(g, x, y, z);
+    const int cz = cell_of(z, g.inv_cell, G), cy = cell_of(y, g.inv_cell, G);
+    // (z, y) row r of the unclamped block; rows outside the grid, and all rows of a lane
+    // row without an electron, are empty (their reads go to the nearest row inside).
+    // No branches, so that the 18 cell starts and then the 9 holes are in flight
+    // together: inside `if`s each would wait for the one before.
 #pragma unroll
-        for (int r = 0; r < 9; ++r) {
-            // (z, y) row r of the unclamped block; rows outside the grid are empty
-            const int zz = cz - 1 + r / 3, yy = cy - 1 + r % 3;
-            s[r] = 0;
-            e[r] = 0;
-            if ((unsigned)zz < (unsigned)G && (unsigned)yy < (unsigned)G) {
-                const int base = (zz * G + yy) * G;
-                s[r] = (int)g.cstart[base + k.x0];
-                e[r] = (int)g.cstart[base + k.x1 + 1];
-            }
-            total += e[r] - s[r];
-            longest = max(longest, e[r] - s[r]);
-        }
-        if (q == 0) evals += (uint64_t)total;      // summed over lanes at the end
-    } else {
-#pragma unroll
-        for (int r = 0; r < 9; ++r) s[r] = e[r] = 0;
+    for (int r = 0; r < 9; ++r) {
+        const int zz = cz - 1 + r / 3, yy = cy - 1 + r % 3;
+        const int base = (min(max(zz, 0), G - 1) * G + min(max(yy, 0), G - 1)) * G;
+        s[r] = (int)g.cstart[base + k.x0];
+        e[r] = (int)g.cstart[base + k.x1 + 1];
     }
+#pragma unroll
+    for (int r = 0; r < 9; ++r) {
+        const int zz = cz - 1 + r / 3, yy = cy - 1 + r % 3;
+        const bool in = act && (unsigned)zz < (unsigned)G && (unsigned)yy < (unsigned)G;
+        e[r] = in ? e[r] : s[r];
+        total += e[r] - s[r];
+        longest = max(longest, e[r] - s[r]);
+    }
+    evals += q == 0 ? (uint64_t)total : 0ull;          // summed over lanes at the end
     uint64_t key = ~0ull;
+    float4 hv[9];
+    // (a range's first slot is within the hole array's capacity, empty ranges included)
+#pragma unroll
+    for (int r = 0; r < 9; ++r) hv[r] = g.hole[s[r] + q < e[r] ? s[r] + q : s[r]];
 #pragma unroll
     for (int r = 0; r < 9; ++r) {
         const int slot = s[r] + q;
-        if (slot < e[r]) {
-            const uint64_t k = key_of(g.hole[slot], x, y, z, slot);
-            key = k < key ? k : key;
-        }
+        uint64_t k2 = key_of(hv[r], x, y, z, slot);
+        k2 = slot < e[r] ? k2 : ~0ull;
+        key = k2 < key ? k2 : key;
     }
     if (ballot(longest > 16) != 0) {
+#pragma unroll 1
         for (int r = 0; r < 9; ++r) {
-            for (int slot = s[r] + q + 16; slot < e[r]; slot += 16) {
-                const uint64_t k = key_of(g.hole[slot], x, y, z, slot);
-                key = k < key ? k : key;
+            const int zz = cz - 1 + r / 3, yy = cy - 1 + r % 3;
+            if (!act || (unsigned)zz >= (unsigned)G || (unsigned)yy >= (unsigned)G) continue;
+            const int base = (zz * G + yy) * G;
+            const int e2 = (int)g.cstart[base + k.x1 + 1];
+            for (int slot = (int)g.cstart[base + k.x0] + q + 16; slot < e2; slot += 16) {
+                const uint64_t k2 = key_of(g.hole[slot], x, y, z, slot);
+                key = k2 < key ? k2 : key;
             }
         }
     }
@@ -260,10 +267,56 @@ __device__ __forceinline__ uint64_t full_scan_wave(const Grid& g, float x, float
     return wave_min_u64(key);
 }
 
+// Nearest live hole of one electron (x, y, z wave-uniform) whose 3x3x3 block was
+// inconclusive, by the whole wave.  WIDE: blocks of 5 and 9 cells an axis while they
+// leave out most of the grid, each accepted by the same test as the 3x3x3 block,
+// then every hole.  A block's (z, y) rows of cells are contiguous slot ranges; a row is
+// split over two lanes (5 cells) or three (9 cells), each fetching four holes a trip.
+// Not WIDE: every hole at once (kernels for small grids, without the blocks' code).
+template <bool WIDE>
+__device__ __forceinline__ uint64_t far_search_wave(const Grid& g, float x, float y, float z, int lane,
+                                                    uint64_t& evals)
+{
+    const int G = g.G;
+    for (int R = 2; WIDE && R <= 4 && 4 * R + 1 <= G; R += 2) {
+        const int cx = cell_of(x, g.inv_cell, G), cy = cell_of(y, g.inv_cell, G),
+                  cz = cell_of(z, g.inv_cell, G);
+        const int x0 = max(cx - R, 0), x1 = min(cx + R, G - 1);
+        const int y0 = max(cy - R, 0), y1 = min(cy + R, G - 1);
+        const int z0 = max(cz - R, 0), z1 = min(cz + R, G - 1);
+        const int ny = y1 - y0 + 1, parts = R == 2 ? 2 : 3;
+        const int items = (z1 - z0 + 1) * ny * parts;
+        uint64_t key = ~0ull;
+        for (int i = lane; i < items; i += kWave) {
+            const int row = i / parts, part = i - row * parts;
+            const int zz = z0 + row / ny, yy = y0 + row % ny;
+            const int base = (zz * G + yy) * G;
+            const int s = (int)g.cstart[base + x0], e = (int)g.cstart[base + x1 + 1];
+            if (part == 0) evals += (uint64_t)(e - s);
+            for (int i0 = s + part; i0 < e; i0 += 4 * parts) {
+                float4 hv[4];
+#pragma unroll
+                for (int t = 0; t < 4; ++t) hv[t] = g.hole[min(i0 + t * parts, e - 1)];
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const uint64_t k = key_of(hv[t], x, y, z, min(i0 + t * parts, e - 1));
+                    key = k < key ? k : key;
+                }
+            }
+        }
+        key = wave_min_u64(key);
+        const float gap = fminf(face_gap(x, x0, x1, G, g.cell),
+                                fminf(face_gap(y, y0, y1, G, g.cell), face_gap(z, z0, z1, G, g.cell)));
+        if (block_conclusive(__uint_as_float((uint32_t)(key >> 32)), gap, g.cell)) return key;
+    }
+    return full_scan_wave(g, x, y, z, lane, evals);
+}
+
 // Nearest live hole for every active lane's electron: 3x3x3 block search per
-// lane, then one wave-wide full scan per lane whose block was inconclusive.  (A
+// lane, then one wave-wide search per lane whose block was inconclusive.  (A
 // lane-private 5x5x5 level in between measured slower: it is divergent, so one
 // open lane makes the wave pay 25 serialized LDS round trips.)
+template <bool WIDE>
 __device__ __forceinline__ uint64_t nn_resolve(const Grid& g, bool act, float x, float y, float z,
                                                int lane, uint64_t& evals)
 {
@@ -275,10 +328,107 @@ __device__ __forceinline__ uint64_t nn_resolve(const Grid& g, bool act, float x,
         const int l = __builtin_ctzll(fb);
         fb &= fb - 1;
         const float fx = lane_value(x, l), fy = lane_value(y, l), fz = lane_value(z, l);
-        const uint64_t k = full_scan_wave(g, fx, fy, fz, lane, evals);
+        const uint64_t k = far_search_wave<WIDE>(g, fx, fy, fz, lane, evals);
         if (lane == l) key = k;
     }
     return key;
+}
+
+// Nearest live holes for the electrons of the lanes in mask (act: the lane is one of
+// them; x, y, z its electron's coordinates), each lane's key in key.  Up to
+// wave_search_max electrons are searched by the whole wave, up to four at a time;
+// beyond, lane-parallel.  A batch of one, two or four gives each electron 64, 32 or
+// 16 lanes; its 3x3x3 block is at most 9 contiguous slot ranges (one per (z, y) row of
+// cells), each shared by 7, 3 or 1 of those lanes, which fetch four holes a trip.
+// (Every lane taking a slot of every range instead, nine range bounds and nine
+// holes a lane, was 550 instructions a batch against 320: the bounds of one range
+// cost as much as three holes.)
+template <bool WIDE>
+__device__ __forceinline__ void search_lanes(const Grid& g, uint64_t mask, bool act, float x, float y,
+                                             float z, int wave_search_max, int lane, uint64_t& key,
+                                             uint64_t& evals)
+{
+    if (__popcll(mask) > wave_search_max) {
+        const uint64_t k = nn_resolve<WIDE>(g, act, x, y, z, lane, evals);
+        if (act) key = k;
+        return;
+    }
+    const int G = g.G;
+    while (mask != 0) {
+        int b[kSearchBatch];
+        int nb = 0;
+#pragma unroll
+        for (int i = 0; i < kSearchBatch; ++i) {       // (a missing one repeats the first)
+            b[i] = mask != 0 ? (int)__builtin_ctzll(mask) : b[0];
+            nb += mask != 0 ? 1 : 0;
+            mask = mask != 0 ? mask & (mask - 1) : 0;
+        }
+        const int log_l = nb == 1 ? 6 : nb == 2 ? 5 : 4;          // log2 lanes of an electron
+        const int parts = nb == 1 ? 7 : nb == 2 ? 3 : 1;          // lanes of a range
+        const int e = lane >> log_l, l = lane & ((1 << log_l) - 1);
+        const int j = nb == 1 ? (l * 37) >> 8 : nb == 2 ? (l * 11) >> 5 : l;   // l / parts
+        const float qx = e == 0 ? lane_value(x, b[0]) : e == 1 ? lane_value(x, b[1])
+                       : e == 2 ? lane_value(x, b[2]) : lane_value(x, b[3]);
+        const float qy = e == 0 ? lane_value(y, b[0]) : e == 1 ? lane_value(y, b[1])
+                       : e == 2 ? lane_value(y, b[2]) : lane_value(y, b[3]);
+        const float qz = e == 0 ? lane_value(z, b[0]) : e == 1 ? lane_value(z, b[1])
+                       : e == 2 ? lane_value(z, b[2]) : lane_value(z, b[3]);
+        const int cx = cell_of(qx, g.inv_cell, G), cy = cell_of(qy, g.inv_cell, G),
+                  cz = cell_of(qz, g.inv_cell, G);
+        const int x0 = max(cx - 1, 0), x1 = min(cx + 1, G - 1);
+        const int jz = (j * 11) >> 5, zz = cz - 1 + jz, yy = cy - 1 + (j - 3 * jz);
+        // range j of the unclamped block; ranges outside the grid are empty
+        uint64_t k = ~0ull;
+        if (j < 9 && (unsigned)zz < (unsigned)G && (unsigned)yy < (unsigned)G) {
+            const int base = (zz * G + yy) * G;
+            const int s0 = (int)g.cstart[base + x0], end = (int)g.cstart[base + x1 + 1];
+            const int part = l - j * parts;
+            if (part == 0 && e < nb) evals += (uint64_t)(end - s0);   // summed over lanes at the end
+            for (int i0 = s0 + part; i0 < end; i0 += 4 * parts) {
+                float4 hv[4];
+#pragma unroll
+                for (int t = 0; t < 4; ++t) hv[t] = g.hole[min(i0 + t * parts, end - 1)];
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const uint64_t kt = key_of(hv[t], qx, qy, qz, min(i0 + t * parts, end - 1));
+                    k = kt < k ? kt : k;
+                }
+            }
+        }
+        k = row_min_u64(k);
+        const int y0 = max(cy - 1, 0), y1 = min(cy + 1, G - 1);
+        const int z0 = max(cz - 1, 0), z1 = min(cz + 1, G - 1);
+        const bool whole = x0 == 0 && y0 == 0 && z0 == 0 && x1 == G - 1 && y1 == G - 1 && z1 == G - 1;
+        const float gap = fminf(face_gap(qx, x0, x1, G, g.cell),
+                                fminf(face_gap(qy, y0, y1, G, g.cell), face_gap(qz, z0, z1, G, g.cell)));
+        // the rows of 16 lanes of each electron combined
+        uint64_t kr[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            kr[i] = ((uint64_t)lane_value((uint32_t)(k >> 32), 16 * i) << 32) |
+                    lane_value((uint32_t)k, 16 * i);
+        if (nb <= 2) {
+            kr[0] = kr[1] < kr[0] ? kr[1] : kr[0];
+            kr[1] = kr[3] < kr[2] ? kr[3] : kr[2];
+            if (nb == 1) kr[0] = kr[1] < kr[0] ? kr[1] : kr[0];
+        }
+        const uint64_t own = e == 0 ? kr[0] : e == 1 ? kr[1] : e == 2 ? kr[2] : kr[3];
+        const bool ok = e >= nb || whole ||
+                        block_conclusive(__uint_as_float((uint32_t)(own >> 32)), gap, g.cell);
+        uint64_t open = ballot(l == 0 && !ok);
+#pragma unroll
+        for (int i = kSearchBatch - 1; i >= 0; --i)     // (the first last: it repeats)
+            if (lane == b[i]) key = i < nb ? kr[i] : kr[0];
+        // electrons whose block was inconclusive
+        while (open != 0) {
+            const int lo = (int)__builtin_ctzll(open);
+            open &= open - 1;
+            const uint64_t kf = far_search_wave<WIDE>(g, lane_value(qx, lo), lane_value(qy, lo),
+                                                      lane_value(qz, lo), lane, evals);
+            const int i = lo >> log_l;
+            if (lane == (i == 0 ? b[0] : i == 1 ? b[1] : i == 2 ? b[2] : b[3])) key = kf;
+        }
+    }
 }
 
 // Inclusive prefix sum of a float64 value over the 64 lanes (all active), in a
@@ -337,29 +487,6 @@ __device__ __forceinline__ float w_of(uint32_t d2bits, float alpha_f)
     return exp_own(-(alpha_f * __builtin_sqrtf(__uint_as_float(d2bits))));
 }
 
-// What a cluster keeps in an electron's w slot: w itself, or (fixed) the fire
-// threshold of x = fma(bdt, w, xA) as its 32-bit pattern, 0xFFFFFFFF for "always"
-// (no other threshold reaches it: p < 1 in float32 gives at most 2^32 - 256), for
-// runs in which that threshold is constant while w is (isothermal, one
-// localisation channel).  The step then reads the threshold instead of taking
-// exp of every electron's x again.
-struct WSlot {
-    bool fixed;
-    float bdt, xA;
-    __device__ __forceinline__ float of(float w) const
-    {
-        if (!fixed) return w;
-        const FireThr t = fire_threshold(__builtin_fmaf(bdt, w, xA));
-        return __uint_as_float(t.always ? 0xFFFFFFFFu : t.thr);
-    }
-};
-
-__device__ __forceinline__ FireThr slot_threshold(float v)
-{
-    const uint32_t b = __float_as_uint(v);
-    return FireThr{b, b == 0xFFFFFFFFu};
-}
-
 __device__ __forceinline__ void nn_from_key(uint64_t key, float alpha_f, uint32_t& slot, float& w)
 {
     const uint32_t d2bits = (uint32_t)(key >> 32);
@@ -394,13 +521,12 @@ __device__ __forceinline__ uint64_t rows_any(uint64_t bits, int rows)
 // the cell prefix, the scatter (slots within a cell in hole-index order) and the
 // shift are wave 0's, between the workgroup's barriers.  Shared by the fixed-dt
 // and event kernels.
-template <int NW>
+template <int NW, bool WIDE>
 __device__ __forceinline__ Grid setup_cluster_t(const RunDesc& R, const ElectronGen& egen,
                                                 float4* hole, uint32_t* cstart, uint32_t* est,
                                                 float* ew, uint32_t prun, uint32_t psim,
                                                 uint32_t k0, uint32_t k1, int tid,
-                                                uint64_t& dist_evals,
-                                                const WSlot& ws = WSlot{false, 0.0f, 0.0f})
+                                                uint64_t& dist_evals)
 {
     constexpr int NT = NW * kWave;
     const int lane = NW == 1 ? tid : (tid & (kWave - 1));
@@ -470,13 +596,13 @@ __device__ __forceinline__ Grid setup_cluster_t(const RunDesc& R, const Electron
         const bool act = e < n_e0;
         float x = 0.0f, y = 0.0f, z = 0.0f;
         if (act) egen.xyz((uint32_t)e, x, y, z);
-        const uint64_t key = nn_resolve(grid, act, x, y, z, lane, dist_evals);
+        const uint64_t key = nn_resolve<WIDE>(grid, act, x, y, z, lane, dist_evals);
         if (act) {
             uint32_t slot;
             float w;
             nn_from_key(key, alpha_f, slot, w);
             est[e] = (slot << 16) | (uint32_t)e;
-            ew[e] = ws.of(w);
+            ew[e] = w;
         }
     }
     __syncthreads();
@@ -484,24 +610,25 @@ __device__ __forceinline__ Grid setup_cluster_t(const RunDesc& R, const Electron
     return grid;
 }
 
+template <bool WIDE>
 __device__ __forceinline__ Grid setup_cluster(const RunDesc& R, const ElectronGen& egen,
                                               float4* hole, uint32_t* cstart, uint32_t* est,
                                               float* ew, uint32_t prun, uint32_t psim,
                                               uint32_t k0, uint32_t k1, int lane,
                                               uint64_t& dist_evals)
 {
-    return setup_cluster_t<1>(R, egen, hole, cstart, est, ew, prun, psim, k0, k1, lane, dist_evals);
+    return setup_cluster_t<1, WIDE>(R, egen, hole, cstart, est, ew, prun, psim, k0, k1, lane, dist_evals);
 }
 
 // New nearest holes for the queued electrons rq[0..nq) ((slot << 16) | index):
 // wave-cooperative searches, kSearchBatch electrons at a time, while the queue
 // is short (at most wave_search_max), lane-parallel otherwise; writes est and ew
-// of their slots (ew as ws keeps it).
+// of their slots.
+template <bool WIDE>
 __device__ __forceinline__ void search_queue_nn(const Grid& grid, const ElectronGen& egen,
                                                 uint32_t* est, float* ew, const uint32_t* rq,
                                                 int nq, int wave_search_max, float alpha_f,
-                                                int lane, uint64_t& dist_evals,
-                                                const WSlot& ws = WSlot{false, 0.0f, 0.0f})
+                                                int lane, uint64_t& dist_evals)
 {
     if (nq <= wave_search_max) {
         for (int i0 = 0; i0 < nq; i0 += kSearchBatch) {
@@ -513,13 +640,13 @@ __device__ __forceinline__ void search_queue_nn(const Grid& grid, const Electron
                 egen.xyz(qq & 0xFFFFu, qx, qy, qz);
                 bool ok = true;
                 uint64_t key = block_search_wave(grid, qx, qy, qz, lane, ok, dist_evals);
-                if (!ok) key = full_scan_wave(grid, qx, qy, qz, lane, dist_evals);
+                if (!ok) key = far_search_wave<WIDE>(grid, qx, qy, qz, lane, dist_evals);
                 if (lane == 0) {
                     uint32_t slot;
                     float w;
                     nn_from_key(key, alpha_f, slot, w);
                     est[qq >> 16] = (slot << 16) | (qq & 0xFFFFu);
-                    ew[qq >> 16] = ws.of(w);
+                    ew[qq >> 16] = w;
                 }
                 continue;
             }
@@ -541,7 +668,7 @@ __device__ __forceinline__ void search_queue_nn(const Grid& grid, const Electron
             while (fb != 0) {
                 const int l = __builtin_ctzll(fb);
                 fb &= fb - 1;
-                const uint64_t k = full_scan_wave(grid, lane_value(qx, l), lane_value(qy, l),
+                const uint64_t k = far_search_wave<WIDE>(grid, lane_value(qx, l), lane_value(qy, l),
                                                   lane_value(qz, l), lane, dist_evals);
                 if ((lane >> 4) == (l >> 4)) key = k;
             }
@@ -550,7 +677,7 @@ __device__ __forceinline__ void search_queue_nn(const Grid& grid, const Electron
                 float w;
                 nn_from_key(key, alpha_f, slot, w);
                 est[qq >> 16] = (slot << 16) | (qq & 0xFFFFu);
-                ew[qq >> 16] = ws.of(w);
+                ew[qq >> 16] = w;
             }
         }
         return;
@@ -562,13 +689,13 @@ __device__ __forceinline__ void search_queue_nn(const Grid& grid, const Electron
         const uint32_t o = q & 0xFFFFu;
         float x = 0.0f, y = 0.0f, z = 0.0f;
         if (act) egen.xyz(o, x, y, z);
-        const uint64_t key = nn_resolve(grid, act, x, y, z, lane, dist_evals);
+        const uint64_t key = nn_resolve<WIDE>(grid, act, x, y, z, lane, dist_evals);
         if (act) {
             uint32_t slot;
             float w;
             nn_from_key(key, alpha_f, slot, w);
             est[q >> 16] = (slot << 16) | o;
-            ew[q >> 16] = ws.of(w);
+            ew[q >> 16] = w;
         }
     }
 }

@@ -121,7 +121,7 @@ __device__ __forceinline__ void run_cluster_event(const EventArgs& a, const int 
     const ElectronGen egen{prun, psim | MCL_TAG_GEOM_E, k0, k1, R.side_nm};
 
     uint64_t dist_evals = 0;
-    const Grid grid = setup_cluster(R, egen, hole, cstart, est, ew, prun, psim, k0, k1, lane,
+    const Grid grid = setup_cluster<GM>(R, egen, hole, cstart, est, ew, prun, psim, k0, k1, lane,
                                     dist_evals);
     const float alpha_f = (float)R.alpha_nm;
 
@@ -340,7 +340,7 @@ __device__ __forceinline__ void run_cluster_event(const EventArgs& a, const int 
             w_valid = false;
             event_fence<GM>();
             if (nq > 0) {
-                search_queue_nn(grid, egen, est, ew, rq, nq, a.wave_search_max, alpha_f, lane,
+                search_queue_nn<GM>(grid, egen, est, ew, rq, nq, a.wave_search_max, alpha_f, lane,
                                 dist_evals);
                 event_fence<GM>();
             }

@@ -4,46 +4,72 @@
 //
 // Replaces the run x sim x step loop of simulate.py:36-92 (Box / Physics /
 // TLTrapSim: engine.py:44-188, tl_trap_lab.py:24-60).  One workgroup of NW
-// wavefronts (1, 2, 4 or 8) owns one cluster; everything the step touches lives in LDS:
+// wavefronts (1, 2, 4 or 8) owns one cluster; everything it touches lives in LDS:
 //
 //   hole       [h_cap]   16-byte records {x, y, z, meta}, float32 nm, sorted by
 //                        grid cell; meta = (claiming electron << 16) | original
 //                        hole index; a removed hole keeps its slot with x = 3e38
 //   cstart     [g_cap]   first sorted slot of each cell, cstart[G^3] = n_h
-//   est        [e_cap]   compacted live electrons: (nearest hole slot << 16) | electron index
-//   ew         [e_cap]   compacted w = exp(-alpha r_nn), float32
-//   ethr       [e_cap]   fire threshold of a candidate in the current step (conflict
-//                        retries); the draw of an electron queued for a new search
-//   rq         [e_cap]   electrons whose nearest hole must be searched again: (slot << 16) | e
-//   xch        [2 NW + 1] (NW > 1) per-wave values exchanged between the waves, and the
-//                        persistent launch's ticket
+//   est        [e_cap]   live electrons: (nearest hole slot << 16) | electron index
+//   ew         [e_cap]   w = exp(-alpha r_nn), float32
+//   rowm       [e_cap / 64]  per row of 64 slots: bit j set when an electron of the
+//                        row may fire in step j of the window (a superset)
+//   nf         [e_cap]   the step of the window in which the electron's draw fires
+//                        (kNever: in none)
+//   lst        [e_cap + 64]  slots gathered from their rows: each wave's from its own
+//                        rows' first entry on, a light step's in the last 64
+//   xch        [2 NW + 5] (NW > 1) per-wave values exchanged between the waves, the
+//                        persistent launch's ticket, and what wave 0 publishes
 //
 // A cluster too large for that (GM: the global-memory form) keeps hole and
 // cstart in its workgroup's slice of a global scratch buffer (slice blockIdx.x,
 // so its launches are persistent: one slice per resident workgroup, reused
-// cluster after cluster); xch opens the LDS block, followed by est, ew, ethr and
-// rq when 16 e_cap bytes fit there (e_lds), otherwise those follow cstart in the
-// slice.  The code is the same; the workgroup barriers order global memory as
-// they order LDS (every wave of a workgroup runs on one CU, behind one L1), and
-// the queue fences of several waves widen to workgroup scope, which waits for
-// the wave's global stores.  Only the slots holes take within a cell can differ
-// from the LDS form (global atomics need not serve the lanes of one instruction
-// in lane order); no result depends on them: every search keys on
+// cluster after cluster); xch opens the LDS block, followed by the electron arrays
+// when they fit there (e_lds), otherwise those follow cstart in the slice.  The
+// code is the same; the workgroup barriers order global memory as they order LDS
+// (every wave of a workgroup runs on one CU, behind one L1), and the fences of one
+// wave widen to workgroup scope.  Only the slots holes take within a cell can
+// differ from the LDS form (global atomics need not serve the lanes of one
+// instruction in lane order); no result depends on them: every search keys on
 // (distance, original hole index).
 //
-// With NW > 1 the 64-slot rows of est/ew are split into NW contiguous ranges, one
-// per wave.  Every per-electron decision is the one-wave kernel's (same draws,
-// same thresholds, same lowest-index conflict rule, same stable compaction
-// order), so the counts are identical for every NW; the waves meet at workgroup
-// barriers where one wave's results reach the others: after the fire pass (any
-// candidate?), after each conflict round's winners (wins, any loser?), at each
-// retry round's claims, and in a compaction (per-wave keep counts; the rows are
-// rewritten into the spare est/ew pair, rq and ethr, whose roles then swap).
-// Each wave searches the queue of its own rows in its own part of rq.
+// First-fire windows.  An electron's draw of step n is the Philox word of counter
+// (n >> 2, e, run, sim|FIRE), and its threshold depends on the step and on its w,
+// which changes only when the electron is searched again, in a step in which its
+// draw fires.  So the step in which it next fires is known in advance: at the start
+// of each 64-step window every live electron's first firing step is found (the
+// scan), and then only the steps in which some electron fires are simulated, with
+// those electrons alone; the others change nothing but the live-step tally.  An
+// electron that fires and stays (its new nearest hole is too far for the draw, or
+// it lost its hole) is scanned again over the rest of the window with its new w.
+// Every draw is tested against exactly the threshold the step-by-step loop would
+// use, once.
+//   scan      one electron a lane, two Philox blocks (eight steps) an iteration,
+//             until every lane of the row has fired.  The draws are compared with
+//             one bound per electron and window (the threshold of x with the
+//             window's largest band term and largest b dt: the threshold is
+//             non-decreasing in x); only a block in which some draw is below its
+//             bound takes the exact thresholds of its four steps.  For isothermal
+//             one-channel runs the bound is the exact threshold.  Rows with few
+//             live electrons take the steps across the lanes instead: 16 lanes
+//             cover an electron's whole window.
+//   light     a step with at most 64 candidates, wave 0 alone, one candidate a lane,
+//             without a workgroup barrier.  (Sharing steps of more than 12 or of more
+//             than one among the waves measured slower: 1000 x 1500 decays 2.12 ms at
+//             64, 2.28 at 12, 2.65 at 1; 250 x 8000 in scratch memory 14.9, 16.2, 18.2.)
+//   ahead     while wave 0 takes the events of a sub-window (8 steps), the other waves
+//             search for the electrons that fire in the next one with events and whose
+//             hole is gone already, so that few searches are left to the steps
+//             themselves (32 x 2000 glow 2.63 -> 2.27 ms, 64 x 1000 tunnelling ramps 2.40
+//             -> 1.92).  One wave alone has nothing to overlap (the decay measured 2 %
+//             slower with it) and leaves every search to its step.
+//   heavy     a step with more candidates: every wave takes the candidates of its
+//             own rows, gathered 64 to a chunk, and they meet at barriers (winners,
+//             each retry round).
 //
 // Electron coordinates are not stored: they are a pure function of the
-// Philox counter (0, e, run, sim|GEOM_E) and are regenerated when an
-// electron's nearest hole has to be searched again.
+// Philox counter (0, e, run, sim|GEOM_E) and are regenerated (each lane its own
+// electron's) when nearest holes have to be searched again.
 //
 // Nearest holes come from a uniform G^3 cell grid over the hole cube: a search
 // scans the 3x3x3 cells around the electron and accepts the minimum of
@@ -51,38 +77,31 @@
 // that block can be (guaranteed face distance, with a margin far above float32
 // rounding); otherwise the whole wave scans every hole for that electron.  The
 // answer is therefore always the first-index argmin of the full scan
-// (engine.py:118-119, 173-175); the grid only removes work.  All electrons that
-// need a search in a step are queued and searched lane-parallel, so a step pays
-// the latency of one search, not one per recombination; each lane fetches the
-// holes of a cell range eight 16-byte records at a time, so one LDS latency
-// covers a chunk.
+// (engine.py:118-119, 173-175); the grid only removes work.
 //
 // Per step n (start-of-step temperature T_n = T0 + T_rate n dt, simulate.py:53-54):
 //   scalars   A = s e^{-E_cb/kT}, B_i = b e^{-E_loc_i/kT} in float64 (own exp),
-//             x_A = A dt, b_i dt in float32; the threshold of x_A once per step.
+//             x_A = A dt, b_i dt in float32; lane j holds those of the window's
+//             step j.
 //   fire      per live electron: u = Philox(n>>2, e, run, sim|FIRE)[n&3],
 //             x = fma(b dt, w, x_A); fire iff u < (uint32)((1 - e^{-x}) 2^32).
-//             When fma(b dt, w, x_A) == x_A (tunnelling below one ulp of the
-//             band term) the per-step threshold is reused: same function of x,
-//             no per-electron transcendental.  Two rows per iteration keep two
-//             independent Philox chains in flight.
+//   repair    an electron whose hole was removed keeps its old w until a step in
+//             which its draw fires against that old w: only then is it searched
+//             again (before its fire test; a conflict loser at once).  Exact: the
+//             new nearest hole is no closer, so w and x = k dt can only fall, and
+//             the threshold of x is non-decreasing in x (checked for every float x
+//             by the oracle), so a draw that fails against the old w fails against
+//             the new one.
 //   conflict  ds_min_u32 of the electron index into the hole's claim field; the
 //             lowest index keeps the hole (src/est_params/functions.py:228-239).
 //   remove    winners' slots become dead, their holes get the x sentinel.
-//   repair    an electron whose hole was removed keeps its old w until a step in
-//             which its draw would fire against that old w: only then is it
-//             searched again (before its fire test; a conflict loser at once).
-//             Exact: the new nearest hole is no closer, so w and x = k dt can only
-//             fall, and the threshold of x is non-decreasing in x (checked for
-//             every float x by the oracle), so a draw that fails against the old
-//             w fails against the new one.
 //   retry     a conflict loser retries on its new nearest hole within the step,
 //             accepted with probability T_new / T_old (one more Philox word), for
 //             up to MCL_MAX_ROUNDS rounds; this removes the O(k dt) delay a
 //             "loser waits a step" rule would put into the decay curves.
-//   compact   stable ballot/mbcnt compaction, only when it drops a 64-slot row.
-// Counts go out per bin (bin of step n = n * n_bins / n_steps), zero-padded
-// after the last electron recombines, like the reference's padded rows.
+//   compact   between windows, stable, when an eighth of the rows can be dropped.
+// Counts go out per bin (bin of step n = n * n_bins / n_steps) into a row that is
+// zeroed first, like the reference's padded rows.
 #pragma once
 
 #include "mc_common.h"
@@ -91,46 +110,35 @@
 
 namespace mcl {
 
-constexpr int kCachePairs = 4;    // row pairs whose Philox blocks stay in registers
-template <int V>
-struct CacheSlot {
-    static constexpr int value = V;
-};
+constexpr int kWindow = 64;            // steps of a window (a multiple of 4; rowm's bits)
+constexpr uint32_t kNever = 255u;      // nf: no firing step in the window
+constexpr int kLogSub = 3, kSub = 1 << kLogSub;   // steps of a sub-window (searched ahead)
+// Rows with at most this many live electrons are scanned four electrons at a time,
+// 16 lanes each, instead of one electron a lane.
+constexpr int kGroupMax = 16;
 
-// Ordering between the steps of one wave that write and then read the search
-// queue: the workgroup barrier with one wave (where it is also the compiler's
-// fence), a fence with several (each wave owns its queue; a workgroup barrier
-// there would not be reached by every wave): wavefront scope when the queue is
+// Ordering between one wave's writes and its lanes' reads of them: wavefront scope
 // in LDS, whose instructions one wave executes in issue order; workgroup scope
-// in the global-memory form, so the wave's global stores have completed before
-// its lanes read them.
-template <int NW, bool GM>
-__device__ __forceinline__ void queue_sync()
+// in the global-memory form, so the wave's global stores come before its loads.
+template <bool GM>
+__device__ __forceinline__ void wave_sync()
 {
-    if constexpr (NW == 1) {
-        __syncthreads();
-    } else if constexpr (GM) {
+    if constexpr (GM) {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     } else {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_lds_fence();
     }
 }
 
 // Simulate cluster c from its geometry to its last step with NW wavefronts, all
 // state in lds_raw (GM: holes and cell starts, and the electron arrays unless
 // a.e_lds, in the workgroup's scratch slice).  Every branch that holds a
-// workgroup barrier depends only on values all waves share (n, n_live, n_slots,
-// and results of the exchanges).  FW: the build with the fixed-threshold path
-// (isothermal one-channel runs keep fire thresholds in their w slots); without
-// it every run computes its thresholds from w, and the code of that path is not
-// in the kernel.  QW: the build with the quiet window (after quiet steps, the rest
-// of a Philox block tested at once).  Every build gives the same counts for every
-// run.
-template <int NW, bool GM, bool FW, bool QW>
+// workgroup barrier depends only on values all waves share (the window, n_live,
+// n_slots, what wave 0 publishes, and results of the exchanges).  WIDE: the build
+// that searches wider blocks before every hole (far_search_wave).
+template <int NW, bool GM, bool WIDE>
 __device__ __forceinline__ void run_cluster(const LaunchArgs& a, const int c,
                                             unsigned char* lds_raw)
 {
@@ -146,7 +154,7 @@ __device__ __forceinline__ void run_cluster(const LaunchArgs& a, const int c,
     const int h_cap = a.h_cap, e_cap = a.e_cap, g_cap = a.g_cap;
 
     unsigned char* hbase;      // hole, cstart
-    unsigned char* ebase;      // est, ew, ethr, rq
+    unsigned char* ebase;      // est, ew, rowm, lst, nf
     uint32_t* xbase;           // xch
     if constexpr (GM) {
         unsigned char* const slice = a.gscratch + (size_t)blockIdx.x * (size_t)a.gstride;
@@ -157,7 +165,7 @@ __device__ __forceinline__ void run_cluster(const LaunchArgs& a, const int c,
     } else {
         hbase = lds_raw;
         ebase = lds_raw + 16 * h_cap + 4 * g_cap;
-        xbase = (uint32_t*)(ebase + 16 * e_cap);
+        xbase = (uint32_t*)(ebase + fixed_dt_electron_bytes(e_cap));
     }
     float4* hole = (float4*)hbase;
     float* hole_f = (float*)hbase;                   // word view: x at 4 s, meta at 4 s + 3
@@ -165,118 +173,239 @@ __device__ __forceinline__ void run_cluster(const LaunchArgs& a, const int c,
     uint32_t* cstart = (uint32_t*)(hole + h_cap);
     uint32_t* est = (uint32_t*)ebase;
     float* ew = (float*)(est + e_cap);
-    uint32_t* ethr = (uint32_t*)(ew + e_cap);
-    uint32_t* rq = ethr + e_cap;
+    unsigned long long* rowm = (unsigned long long*)(ew + e_cap);
+    uint16_t* lst = (uint16_t*)(rowm + e_cap / kWave);
+    uint8_t* nf = (uint8_t*)(lst + e_cap + kWave);
     uint32_t* const xch = xbase;
 
     const uint32_t k0 = a.key0, k1 = a.key1;
     const uint32_t prun = (uint32_t)R.run_id;
     const uint32_t psim = (uint32_t)sim << 4;
     const ElectronGen egen{prun, psim | MCL_TAG_GEOM_E, k0, k1, R.side_nm};
+    const uint64_t ret_thr = R.ret_thr;
+    const uint32_t c3f = psim | MCL_TAG_FIRE, c3c = psim | MCL_TAG_CHAN;
+    const int nb = a.n_bins > 0 ? a.n_bins : n_steps;   // n_bins == 0: one bin per step
+    uint32_t* cnt = a.counts + (size_t)c * (size_t)a.row_len;
+
+    // The counts row starts as zeros (wave 0, which alone writes it later: one
+    // wave's stores to an address keep their order).
+    if (wv == 0)
+        for (int b = lane; b < a.row_len; b += kWave) cnt[b] = 0u;
+
+    uint64_t dist_evals = 0;
+    const Grid grid = setup_cluster_t<NW, WIDE>(R, egen, hole, cstart, est, ew, prun, psim, k0, k1, tid,
+                                          dist_evals);
+    const float alpha_f = (float)R.alpha_nm;
 
     const bool two_ch = R.two_channel != 0;
     const bool always2 = R.always_chan2 != 0;
+    const bool ramp = R.T_rate != 0.0;
+    const bool exact_bound = !ramp && !two_ch;   // the window's bound is every step's threshold
     // single-trap parameter sets share one Boltzmann factor between the channels
     const bool b1_is_a = R.b == R.s && R.E_loc_1 == R.E_cb;
     const bool b2_is_b1 = R.E_loc_2 == R.E_loc_1;
-    // Step scalars of step m: start-of-step temperature, Boltzmann factors in
-    // float64, their float32 products with dt, the threshold of the band term.
-    struct StepScalars {
-        float xA, b1dt, b2dt;
-        FireThr tA;
-    };
-    auto scalars_at = [&](int m) {
+    const int step_limit = a.dump.enabled ? min(a.dump.max_steps, n_steps) : n_steps;
+
+    // The window's steps nb0 .. nb0 + len - 1: lane j holds step nb0 + j's scalars
+    // (start-of-step temperature, Boltzmann factors in float64, their float32
+    // products with dt), lanes past len those of the last step; x_max and b_max are
+    // their largest values (b of the channels a draw can take).
+    int nb0 = 0, len = 0;
+    float l_xA = 0.0f, l_b1 = 0.0f, l_b2 = 0.0f, x_max = 0.0f, b_max = 0.0f;
+    auto window_scalars = [&]() {
+        const int m = nb0 + min(lane, len - 1);
         const double t = (double)m * R.dt;
         const double T = R.T0_K + R.T_rate * t;
         const double kT = R.k_b * T;
         const double A = R.s * exp_own(-(R.E_cb / kT));
         const double B1 = b1_is_a ? A : R.b * exp_own(-(R.E_loc_1 / kT));
         const double B2 = b2_is_b1 ? B1 : R.b * exp_own(-(R.E_loc_2 / kT));
-        StepScalars sc;
-        sc.xA = (float)(A * R.dt);
-        sc.b1dt = (float)(B1 * R.dt);
-        sc.b2dt = (float)(B2 * R.dt);
-        sc.tA = fire_threshold(sc.xA);
-        return sc;
+        l_xA = (float)(A * R.dt);
+        l_b1 = (float)(B1 * R.dt);
+        l_b2 = (float)(B2 * R.dt);
+        // (non-negative floats order as their bits; a NaN, above every number, makes
+        // the bound "always", so the exact thresholds decide)
+        const uint32_t xb = __float_as_uint(l_xA);
+        const uint32_t b1 = __float_as_uint(l_b1), b2 = __float_as_uint(l_b2);
+        x_max = __uint_as_float(wave_max_u32(xb));
+        b_max = __uint_as_float(wave_max_u32(two_ch ? max(b1, b2) : always2 ? b2 : b1));
     };
-    const StepScalars sc0 = scalars_at(0);
-    // An isothermal run with one localisation channel keeps each electron's fire
-    // threshold, constant while its w is, in the w slot (state dumps keep w).
-    const bool fixedw = FW && R.T_rate == 0.0 && !two_ch && a.dump.enabled == 0;
-    const WSlot wslot{fixedw, always2 ? sc0.b2dt : sc0.b1dt, sc0.xA};
-
-    uint64_t dist_evals = 0;
-    const Grid grid = setup_cluster_t<NW>(R, egen, hole, cstart, est, ew, prun, psim, k0, k1, tid,
-                                          dist_evals, wslot);
-    const float alpha_f = (float)R.alpha_nm;
-
-    // ---- step loop (simulate.py:51-92) -------------------------------------------
-    const int nb = a.n_bins > 0 ? a.n_bins : n_steps;   // n_bins == 0: one bin per step
-    uint32_t* cnt = a.counts + (size_t)c * (size_t)a.row_len;
-    const uint64_t ret_thr = R.ret_thr;
-    const uint32_t c3f = psim | MCL_TAG_FIRE, c3c = psim | MCL_TAG_CHAN;
-    const int step_limit = a.dump.enabled ? min(a.dump.max_steps, n_steps) : n_steps;
-
-    int n_live = n_e0, n_slots = n_e0;
-    uint64_t lsteps = 0;
-    int steps_run = 0;
-    uint32_t bin_acc = 0;
-    int bin = 0;
-    int64_t bin_rem = 0;
-    float xA = 0.0f, b1dt = 0.0f, b2dt = 0.0f;
-    FireThr tA{0u, false};
-
-    auto hole_dead = [&](uint32_t nn) {
-        return nn != kNoHole && hole_f[4 * (nn != kNoHole ? nn : 0u)] == kDeadHoleX;
+    auto threshold = [&](float w, bool ch2, float xA, float b1, float b2) -> FireThr {
+        return fire_threshold(__builtin_fmaf(ch2 ? b2 : b1, w, xA));
     };
+    auto fires = [](uint32_t u, const FireThr& t) -> bool { return t.always || u < t.thr; };
+    // Does the channel draw of word d pick channel 2?
+    auto channel_word = [&](const u32x4& r, int d) -> bool {
+        return (uint64_t)pick_word(r, d) < ret_thr;
+    };
+
+    // First firing step (window-relative, kNever: none) from step `from` on of the
+    // electrons of the lanes in mask (index o, w), four at a time, 16 lanes each:
+    // lane q of a row tests block q's four steps.  Writes f in those lanes; returns
+    // the mask of the steps found.  (from may differ between the lanes.)
+    auto group_scan = [&](uint64_t mask, uint32_t o, float w, int from, uint32_t& f) -> uint64_t {
+        uint64_t steps = 0;
+        const int g = lane >> 4, q = lane & 15;
+        while (mask != 0) {
+            int b[4];
+            b[0] = __builtin_ctzll(mask);
+            mask &= mask - 1;
+#pragma unroll
+            for (int i = 1; i < 4; ++i) {          // (a missing one repeats the first)
+                b[i] = mask != 0 ? (int)__builtin_ctzll(mask) : b[0];
+                mask = mask != 0 ? mask & (mask - 1) : 0;
+            }
+            const uint32_t o0 = lane_value(o, b[0]), o1 = lane_value(o, b[1]),
+                           o2 = lane_value(o, b[2]), o3 = lane_value(o, b[3]);
+            const float w0 = lane_value(w, b[0]), w1 = lane_value(w, b[1]),
+                        w2 = lane_value(w, b[2]), w3 = lane_value(w, b[3]);
+            const uint32_t og = g == 0 ? o0 : g == 1 ? o1 : g == 2 ? o2 : o3;
+            const float wg = g == 0 ? w0 : g == 1 ? w1 : g == 2 ? w2 : w3;
+            const uint32_t f0 = lane_value((uint32_t)from, b[0]), f1 = lane_value((uint32_t)from, b[1]),
+                           f2 = lane_value((uint32_t)from, b[2]), f3 = lane_value((uint32_t)from, b[3]);
+            const int fg = (int)(g == 0 ? f0 : g == 1 ? f1 : g == 2 ? f2 : f3);
+            const uint32_t blk = (uint32_t)(nb0 >> 2) + (uint32_t)q;
+            const u32x4 u = philox10(blk, og, prun, c3f, k0, k1);
+            uint32_t first = kNever;
+            if (exact_bound) {
+                const FireThr t = threshold(wg, always2, x_max, b_max, b_max);
+#pragma unroll
+                for (int d = 3; d >= 0; --d) {
+                    const int rel = 4 * q + d;
+                    if (rel >= fg && rel < len && fires(pick_word(u, d), t)) first = (uint32_t)rel;
+                }
+            } else {
+                u32x4 cw{0u, 0u, 0u, 0u};
+                if (two_ch) cw = philox10(blk, og, prun, c3c, k0, k1);
+#pragma unroll
+                for (int d = 3; d >= 0; --d) {
+                    const int rel = 4 * q + d;
+                    const float xA = __shfl(l_xA, rel);
+                    const float b1 = __shfl(l_b1, rel), b2 = __shfl(l_b2, rel);
+                    const bool ch = two_ch ? channel_word(cw, d) : always2;
+                    if (rel >= fg && rel < len && fires(pick_word(u, d), threshold(wg, ch, xA, b1, b2)))
+                        first = (uint32_t)rel;
+                }
+            }
+            first = row_min_u32(first);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t fi = lane_value(first, 16 * i);
+                if (lane == b[i]) f = fi;
+                if (fi != kNever) steps |= 1ull << fi;
+            }
+        }
+        return steps;
+    };
+
+    // The same for one electron a lane (live: the lane has one), the blocks of the
+    // window in order, until every lane has fired.
+    auto lane_scan = [&](bool live, uint32_t o, float w, int from, uint32_t& f) -> uint64_t {
+        FireThr tb;
+        if (exact_bound) {
+            tb = threshold(w, always2, x_max, b_max, b_max);
+        } else {
+            const float xb = __builtin_fmaf(b_max, w, x_max);
+            tb = fire_threshold(xb);
+            tb.always = tb.always || !(xb < __builtin_inff());
+        }
+        bool todo = live && (tb.always || tb.thr != 0u);
+        uint32_t first = kNever;
+        // the four steps of block q (window-relative) with its draws u
+        auto block = [&](int q, const u32x4& u) {
+            const uint32_t um = min(min(u.x, u.y), min(u.z, u.w));
+            const bool hit = todo && (tb.always || um < tb.thr);
+            if (ballot(hit) == 0) return;
+            u32x4 cw{0u, 0u, 0u, 0u};
+            if (two_ch) cw = philox10((uint32_t)(nb0 >> 2) + (uint32_t)q, o, prun, c3c, k0, k1);
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {
+                const int rel = 4 * q + d;
+                if (rel < from || rel >= len) continue;
+                FireThr t = tb;
+                if (!exact_bound) {
+                    const bool ch = two_ch ? channel_word(cw, d) : always2;
+                    t = threshold(w, ch, lane_value(l_xA, rel), lane_value(l_b1, rel),
+                                  lane_value(l_b2, rel));
+                }
+                if (hit && first == kNever && fires(pick_word(u, d), t)) first = (uint32_t)rel;
+            }
+            todo = todo && first == kNever;
+        };
+        const int q_end = (len + 3) >> 2;
+        for (int q = from >> 2; q < q_end && ballot(todo) != 0; q += 2) {
+            const uint32_t blk = (uint32_t)(nb0 >> 2) + (uint32_t)q;
+            const u32x4 ua = philox10(blk, o, prun, c3f, k0, k1);
+            const u32x4 ub = philox10(blk + 1u, o, prun, c3f, k0, k1);
+            block(q, ua);
+            if (q + 1 < q_end) block(q + 1, ub);
+        }
+        if (live) f = first;
+        const uint64_t bit = live && first != kNever ? 1ull << first : 0ull;
+        return ((uint64_t)wave_or_u32((uint32_t)(bit >> 32)) << 32) | wave_or_u32((uint32_t)bit);
+    };
+    auto first_fire = [&](bool live, uint32_t o, float w, int from, uint32_t& f) -> uint64_t {
+        const uint64_t m = ballot(live);
+        if (__popcll(m) <= kGroupMax) return group_scan(m, o, w, from, f);
+        return lane_scan(live, o, w, from, f);
+    };
+    // The slots of rows [r_lo, r_hi) that fire in the 2^lg steps from rel on (a multiple
+    // of 2^lg), to out (at most cap of them); returns how many.  A lane reads eight
+    // slots' nf at once, so one trip covers eight rows, and the row masks skip eight
+    // rows without one.
+    auto gather = [&](int rel, int lg, int r_lo, int r_hi, uint16_t* out, int cap) -> int {
+        const uint32_t bits = (1u << (1 << lg)) - 1u;          // lg <= 3
+        const uint32_t keep = ((0xFFu << lg) & 0xFFu) * 0x01010101u;
+        const uint32_t pat = (uint32_t)rel * 0x01010101u;
+        int k = 0;
+        for (int r0 = r_lo; r0 < r_hi; r0 += kWave) {
+            const uint64_t rm = r0 + lane < r_hi ? (uint64_t)rowm[r0 + lane] : 0ull;
+            const uint64_t ev = ballot(((uint32_t)(rm >> rel) & bits) != 0u);
+            for (int r8 = 0; r8 < kWave && (ev >> r8) != 0; r8 += 8) {
+                if (((ev >> r8) & 0xFFull) == 0) continue;
+                const int p0 = (r0 + r8) * kWave + 8 * lane;
+                const uint2 v = p0 < r_hi * kWave ? *(const uint2*)(nf + p0)
+                                                  : make_uint2(~0u, ~0u);      // (kNever bytes)
+                const uint32_t xa = (v.x ^ pat) & keep, xb = (v.y ^ pat) & keep;
+#pragma unroll
+                for (int t = 0; t < 8; ++t) {
+                    const bool is = (((t < 4 ? xa : xb) >> (8 * (t & 3))) & 0xFFu) == 0u;
+                    const uint64_t m = ballot(is);
+                    if (m == 0) continue;
+                    const int q = k + lanes_below(m);
+                    if (is && q < cap) out[q] = (uint16_t)(p0 + t);
+                    k += __popcll(m);
+                }
+            }
+        }
+        wave_sync<GM>();
+        return k;
+    };
+
     // Claim hole nn for electron o: the claim field keeps the lowest index.
     auto claim = [&](uint32_t nn, uint32_t o) {
         atomicMin(&hole_u[4 * nn + 3], (o << 16) | (hole_u[4 * nn + 3] & 0xFFFFu));
     };
-    // Fire threshold of the electron whose w slot holds v, in channel ch (2 when
-    // set): the one kept in the slot, or that of x = k dt = fma(b dt, w, x_A).
-    auto slot_thr = [&](float v, bool ch) -> FireThr {
-        if (fixedw) return slot_threshold(v);
-        const float x = __builtin_fmaf(ch ? b2dt : b1dt, v, xA);
-        return x != xA ? fire_threshold(x) : tA;
-    };
-    // Test of one live electron (slot p) with draw u and threshold t; candidates
-    // claim their hole and remember their threshold for a conflict retry.
-    auto fire_tail = [&](uint32_t st, uint32_t o, int p, uint32_t u, FireThr t, int rr,
-                         uint64_t& cand) {
-        const uint32_t nn = st >> 16;
-        if (nn == kNoHole) return;
-        if (t.always || u < t.thr) {
-            claim(nn, o);
-            ethr[p] = t.always ? 0xFFFFFFFFu : t.thr;
-            cand |= 1ull << rr;
+    // Nearest live holes of the lanes in mask (coordinates in the lanes), written to
+    // est and ew of their slots p; nn and w follow.
+    auto search = [&](uint64_t mask, bool need, float x, float y, float z, uint32_t o, int p,
+                      uint32_t& nn, float& w) {
+        uint64_t key = ~0ull;
+        search_lanes<WIDE>(grid, mask, need, x, y, z, a.wave_search_max, lane, key, dist_evals);
+        if (need) {
+            nn_from_key(key, alpha_f, nn, w);
+            est[p] = (nn << 16) | o;
+            ew[p] = w;
         }
     };
-    // Pass-A test of one live electron (slot p, draw u, threshold t of its current
-    // w): nothing unless the draw fires; then one 16-byte read of its hole gives
-    // both the removed-hole marker and the claim field.  A removed hole queues the
-    // electron for a new search (its draw kept in ethr; the test against the old w
-    // bounds the one against the new); a live one is claimed.  Returns queued.
-    auto test_fire = [&](uint32_t st, uint32_t o, int p, uint32_t u, FireThr t, int rr,
-                         uint64_t& cand) -> bool {
-        const uint32_t nn = st >> 16;
-        if (nn == kNoHole) return false;
-        if (!(t.always || u < t.thr)) return false;
-        const float4 h = hole[nn];
-        if (h.x == kDeadHoleX) {
-            ethr[p] = u;
-            return true;
-        }
-        atomicMin(&hole_u[4 * nn + 3], (o << 16) | (__float_as_uint(h.w) & 0xFFFFu));
-        ethr[p] = t.always ? 0xFFFFFFFFu : t.thr;
-        cand |= 1ull << rr;
-        return false;
-    };
-    // Search again for the queued electrons q[0..nq): one electron at a time
-    // with the whole wave while the queue is short, lane-parallel otherwise.
-    auto search_queue = [&](const uint32_t* q, int nq) {
-        search_queue_nn(grid, egen, est, ew, q, nq, a.wave_search_max, alpha_f, lane, dist_evals,
-                        wslot);
+    // A conflict loser's retry: accepted with probability T_new / T_old.
+    auto accepted = [&](const FireThr& tn, const FireThr& to, uint32_t blk, int word, uint32_t o,
+                        uint32_t round) -> bool {
+        const uint64_t Tn = tn.always ? 0x100000000ull : (uint64_t)tn.thr;
+        const uint64_t To = to.always ? 0x100000000ull : (uint64_t)to.thr;
+        if (Tn >= To) return true;
+        const u32x4 rr = philox10(blk, o, prun, psim | (MCL_TAG_RETRY0 + round), k0, k1);
+        return (uint64_t)pick_word(rr, word) * To < (Tn << 32);
     };
     // Per-wave values between the waves (NW > 1): lane 0 of each wave publishes
     // v, one workgroup barrier, then every wave reads all NW values.  Consecutive
@@ -302,563 +431,453 @@ __device__ __forceinline__ void run_cluster(const LaunchArgs& a, const int c,
         }
     };
 
-    // Look-ahead for few live electrons: lane j tests step n + j for every live
-    // electron with exactly the draw and threshold that step would use (a stale
-    // electron against its old w, as in pass A).  Returns how many steps from n on
-    // no electron can fire (at most 64, up to step_limit); found tells whether
-    // some step of the window may fire.  Such quiet steps change nothing but
-    // the live-step and bin tallies.
-    auto quiet_steps = [&](int n0, bool& found) -> int {
-        const int len = min(kWave, step_limit - n0);
-        const int m = n0 + lane;
-        StepScalars sc{xA, b1dt, b2dt, tA};
-        if (R.T_rate != 0.0) sc = scalars_at(m);
-        const uint32_t mblk = (uint32_t)m >> 2;
-        const int mword = m & 3;
-        bool fire = false;
-        for (int p = 0; p < n_slots; ++p) {
-            const uint32_t st = est[p];                  // one address: a broadcast read
-            if (st == kDeadSlot || (st >> 16) == kNoHole) continue;
-            const uint32_t o = st & 0xFFFFu;
-            const float w = ew[p];
-            const uint32_t u = pick_word(philox10(mblk, o, prun, c3f, k0, k1), mword);
-            bool ch = always2;
-            if (two_ch)
-                ch = (uint64_t)pick_word(philox10(mblk, o, prun, c3c, k0, k1), mword) < ret_thr;
-            FireThr t;
-            if (fixedw) {
-                t = slot_threshold(w);
-            } else {
-                const float x = __builtin_fmaf(ch ? sc.b2dt : sc.b1dt, w, sc.xA);
-                t = x != sc.xA ? fire_threshold(x) : sc.tA;
-            }
-            fire = fire || t.always || u < t.thr;
+    int n_live = n_e0, n_slots = n_e0;
+    int rows = 0;
+    // wave 0's tallies
+    uint64_t lsteps = 0;
+    int n_acc = 0;               // steps below it are in lsteps
+    int bin = 0;
+    uint32_t bin_acc = 0;
+    const double inv_steps = 1.0 / (double)n_steps;
+    // Step n (the next one with candidates) ended with `wins` recombinations.
+    auto finish_step = [&](int n, uint32_t wins) {
+        lsteps += (uint64_t)n_live * (uint64_t)(n + 1 - n_acc);
+        n_acc = n + 1;
+        n_live -= (int)wins;
+        if (wins == 0u) return;
+        int b = n;
+        if (nb != n_steps) {
+            // floor(n nb / n_steps): the quotient in float64, then one step either way
+            const int64_t num = (int64_t)n * (int64_t)nb;
+            b = (int)((double)num * inv_steps);
+            const int64_t rem = num - (int64_t)b * (int64_t)n_steps;
+            b += rem < 0 ? -1 : rem >= (int64_t)n_steps ? 1 : 0;
+            b = uniform(b);
         }
-        const uint64_t fm = ballot(fire && lane < len);
-        found = fm != 0;
-        return found ? (int)__builtin_ctzll(fm) : len;
-    };
-    // Bin tally at the end of a step with `wins` recombinations.
-    auto finish_step = [&](uint32_t wins) {
+        if (b != bin) {
+            if (lane == 0 && bin_acc != 0u) cnt[bin] = bin_acc;
+            bin = b;
+            bin_acc = 0u;
+        }
         bin_acc += wins;
-        bin_rem += nb;
-        if (bin_rem >= n_steps) {
-            bin_rem -= n_steps;
-            if (tid == 0) cnt[bin] = bin_acc;
-            bin_acc = 0;
-            ++bin;
-        }
     };
 
-    xA = sc0.xA;
-    b1dt = sc0.b1dt;
-    b2dt = sc0.b2dt;
-    tA = sc0.tA;
-    // Philox blocks of the first 2 kCachePairs rows, kept in registers: steps
-    // n .. n+3 share the counter (n >> 2, e, run, sim|tag), so a block computed in
-    // one of them serves the other three.  cache_pairs marks the row pairs whose
-    // blocks are those of block cache_blk for the electrons now in their slots.
-    u32x4 cfa[kCachePairs], cfb[kCachePairs];   // fire blocks of rows 2q, 2q + 1
-    uint32_t cch[kCachePairs];                   // channel bits: row 2q word k at bit k,
-                                                 // row 2q + 1 at bit 4 + k
-    uint32_t cache_pairs = 0u;
-    int cache_blk = -1;
-    float l_xA = 0.0f, l_b1dt = 0.0f, l_b2dt = 0.0f;   // step scalars of step sc_base + lane
-    uint32_t l_thr = 0u, l_always = 0u;
-    int sc_base = -kWave;
-    // The step scalars of step m >= 1 of a ramp, from lane m - sc_base (the 64 steps
-    // from sc_base are evaluated in parallel, refilled from m when m leaves them).
-    auto ramp_scalars = [&](int m, int last) -> StepScalars {
-        if (m < sc_base || last - sc_base >= kWave) {
-            const StepScalars sc = scalars_at(m + lane);
-            l_xA = sc.xA;
-            l_b1dt = sc.b1dt;
-            l_b2dt = sc.b2dt;
-            l_thr = sc.tA.thr;
-            l_always = sc.tA.always ? 1u : 0u;
-            sc_base = m;
-        }
-        const int j = m - sc_base;
-        StepScalars sc;
-        sc.xA = lane_value(l_xA, j);
-        sc.b1dt = lane_value(l_b1dt, j);
-        sc.b2dt = lane_value(l_b2dt, j);
-        sc.tA.thr = lane_value(l_thr, j);
-        sc.tA.always = lane_value(l_always, j) != 0u;
-        return sc;
-    };
-    // Quiet window: the steps n0 .. n0 + W - 1 (n0 >= 1, within one Philox block, so
-    // one block per electron holds all their draws) tested at once, each live
-    // electron's draw of each step against that step's threshold exactly as pass A
-    // tests it (a stale electron against its old w).  Returns how many steps from
-    // n0 no electron of the cluster fires in (W: none); those steps change nothing
-    // but the tallies, and the next step that runs finds its cached rows' blocks in
-    // the register cache.
-    auto quiet_window = [&](int n0, int W) -> int {
-        const uint32_t wblk = (uint32_t)n0 >> 2;
-        const int wd = n0 & 3;
-        const int wrows = (n_slots + kWave - 1) / kWave;
-        const int per = (wrows + NW - 1) / NW;      // rows of a wave, at most (all waves)
-        // only rows whose blocks the register cache keeps (the next step reads them
-        // there); with more rows a wave, the steps run one by one (the same choice
-        // in every wave: a window holds an exchange)
-        if (per > 2 * kCachePairs) return 0;
-        int w_lo = 0, wnr = wrows, w_end = n_slots;
-        if constexpr (NW > 1) {
-            w_lo = min(wrows, wv * per);
-            wnr = min(wrows, w_lo + per) - w_lo;
-            w_end = min(n_slots, (w_lo + wnr) * kWave);
-        }
-        if (R.T_rate != 0.0) (void)ramp_scalars(n0, n0 + W - 1);   // the window's steps in the lanes
-        // step scalars of step n0 + k
-        auto scal = [&](int k) -> StepScalars {
-            if (R.T_rate == 0.0) return StepScalars{xA, b1dt, b2dt, tA};
-            return ramp_scalars(n0 + k, n0 + k);
-        };
-        if ((int)wblk != cache_blk) {
-            cache_blk = (int)wblk;
-            cache_pairs = 0u;
-        }
-        // the first step in which an electron of this wave fires (W: none); a pair
-        // tests only the steps before the first one an earlier pair found
-        int lim = W;
-        auto window_pair = [&](int r, auto slot_tag) {
-            constexpr int q = decltype(slot_tag)::value;
-            const int p0 = (w_lo + r) * kWave + lane, p1 = p0 + kWave;
-            const uint32_t st0 = p0 < w_end ? est[p0] : kDeadSlot;
-            const uint32_t st1 = p1 < w_end ? est[p1] : kDeadSlot;
-            const float v0 = p0 < w_end ? ew[p0] : 0.0f, v1 = p1 < w_end ? ew[p1] : 0.0f;
-            const uint32_t o0 = st0 & 0xFFFFu, o1 = st1 & 0xFFFFu;
-            u32x4 fa, fb;
-            uint32_t cb = 0u;
-            bool hit = false;
-            if constexpr (q >= 0) hit = ((cache_pairs >> q) & 1u) != 0u;
-            if (hit) {
-                if constexpr (q >= 0) {
-                    fa = cfa[q];
-                    fb = cfb[q];
-                    cb = cch[q];
-                }
-            } else {
-                fa = philox10(wblk, o0, prun, c3f, k0, k1);
-                fb = philox10(wblk, o1, prun, c3f, k0, k1);
-                if (two_ch) {
-                    const u32x4 ca = philox10(wblk, o0, prun, c3c, k0, k1);
-                    const u32x4 cc = philox10(wblk, o1, prun, c3c, k0, k1);
-                    cb = (uint32_t)((uint64_t)ca.x < ret_thr) | (uint32_t)((uint64_t)ca.y < ret_thr) << 1 |
-                         (uint32_t)((uint64_t)ca.z < ret_thr) << 2 | (uint32_t)((uint64_t)ca.w < ret_thr) << 3 |
-                         (uint32_t)((uint64_t)cc.x < ret_thr) << 4 | (uint32_t)((uint64_t)cc.y < ret_thr) << 5 |
-                         (uint32_t)((uint64_t)cc.z < ret_thr) << 6 | (uint32_t)((uint64_t)cc.w < ret_thr) << 7;
-                }
-                if constexpr (q >= 0) {
-                    cfa[q] = fa;
-                    cfb[q] = fb;
-                    cch[q] = cb;
-                    cache_pairs |= 1u << q;
-                }
-            }
-            for (int k = 0; k < lim; ++k) {
-                const StepScalars sc = scal(k);
-                const int d = wd + k;
-                const bool ch0 = two_ch ? ((cb >> d) & 1u) != 0u : always2;
-                const bool ch1 = two_ch ? ((cb >> (4 + d)) & 1u) != 0u : always2;
-                FireThr t0, t1;
-                if (fixedw) {
-                    t0 = slot_threshold(v0);
-                    t1 = slot_threshold(v1);
-                } else {
-                    const float x0 = __builtin_fmaf(ch0 ? sc.b2dt : sc.b1dt, v0, sc.xA);
-                    const float x1 = __builtin_fmaf(ch1 ? sc.b2dt : sc.b1dt, v1, sc.xA);
-                    t0 = x0 != sc.xA ? fire_threshold(x0) : sc.tA;
-                    t1 = x1 != sc.xA ? fire_threshold(x1) : sc.tA;
-                }
-                const bool f0 = (st0 >> 16) != kNoHole && (t0.always || pick_word(fa, d) < t0.thr);
-                const bool f1 = (st1 >> 16) != kNoHole && (t1.always || pick_word(fb, d) < t1.thr);
-                if (ballot(f0 || f1) != 0) {
-                    lim = k;
-                    break;
-                }
-            }
-        };
-        if (NW == 1 || wnr > 0) window_pair(0, CacheSlot<0>{});
-        if (wnr > 2) window_pair(2, CacheSlot<1>{});
-        if (wnr > 4) window_pair(4, CacheSlot<2>{});
-        if (wnr > 6) window_pair(6, CacheSlot<3>{});
-        if constexpr (NW > 1) {
-            const uint32_t* x = exchange((uint32_t)lim);
-            uint32_t m = (uint32_t)W;
-#pragma unroll
-            for (int w = 0; w < NW; ++w) m = x[w] < m ? x[w] : m;
-            lim = (int)uniform(m);
-        }
-        return lim;
-    };
-    int quiet_run = 0;           // steps since the last one with a candidate in some wave
-    int quiet_need = 2;          // quiet steps before a window; doubled after a window
-                                 // whose first step fires, back to 2 after a whole one
-    int n = 0;
-    while (n < step_limit && n_live > 0) {
-        if (n_live <= a.lookahead_max) {
-            bool found = false;
-            const int f = quiet_steps(n, found);
-            for (int k = 0; k < f; ++k) {
-                lsteps += (uint64_t)n_live;
-                finish_step(0u);
-            }
-            n += f;
-            steps_run = n;
-            if (!found) continue;
-        } else if (QW && quiet_run >= quiet_need && (n & 3) <= 2) {
-            // a quiet stretch: the rest of the block at once
-            const int W = min(4 - (n & 3), step_limit - n);
-            const int f = quiet_window(n, W);
-            for (int k = 0; k < f; ++k) {
-                lsteps += (uint64_t)n_live;
-                finish_step(0u);
-            }
-            n += f;
-            steps_run = n;
-            quiet_run += f;
-            if (f == 0) quiet_need = min(2 * quiet_need, 64);
-            if (f == W) {
-                quiet_need = 2;
-                continue;
-            }
-        }
-        lsteps += (uint64_t)n_live;
-        steps_run = n + 1;
-        if (n > 0 && R.T_rate != 0.0) {
-            // a ramp: lane j holds the scalars of step sc_base + j (64 steps in one
-            // parallel evaluation instead of 64 serial ones)
-            const StepScalars sc = ramp_scalars(n, n);
-            xA = sc.xA;
-            b1dt = sc.b1dt;
-            b2dt = sc.b2dt;
-            tA = sc.tA;
-        }
+    // A step's conflict rounds with at most one candidate a lane (act), one wave:
+    // round it = 0 searches the candidates whose hole is gone and tests their draw
+    // against the new threshold; later rounds search the losers, which retry.
+    auto light_step = [&](int rel, bool act, int p) -> uint64_t {
+        const int n = nb0 + rel;
         const uint32_t blk = (uint32_t)n >> 2;
         const int word = n & 3;
-        const int rows = (n_slots + kWave - 1) / kWave;
-        // this wave's rows: [r_lo, r_lo + nr), slots below slot_end (all rows with NW = 1)
-        int r_lo = 0, nr = rows, slot_end = n_slots;
+        const float xA = lane_value(l_xA, rel), b1 = lane_value(l_b1, rel), b2 = lane_value(l_b2, rel);
+        const uint32_t st = act ? est[p] : 0u;
+        float w = act ? ew[p] : 0.0f;
+        const uint32_t o = st & 0xFFFFu;
+        uint32_t nn = st >> 16;
+        bool need = act && hole_f[4 * nn] == kDeadHoleX;
+        bool cand = act && !need;
+        bool ch = always2;
+        if (two_ch) ch = channel_word(philox10(blk, o, prun, c3c, k0, k1), word);
+        FireThr t{0u, false};
+        bool have_t = false, have_xyz = false;
+        float x = 0.0f, y = 0.0f, z = 0.0f;
+        uint32_t wins = 0;
+        bool won = false;
+        for (int it = 0;; ++it) {
+            const uint64_t nm = ballot(need);
+            if (nm != 0) {
+                if (!have_xyz) {
+                    egen.xyz(o, x, y, z);
+                    have_xyz = true;
+                }
+                if (it > 0 && !have_t) {
+                    t = threshold(w, ch, xA, b1, b2);
+                    have_t = true;
+                }
+                uint32_t u = 0u;
+                if (it == 0) u = pick_word(philox10(blk, o, prun, c3f, k0, k1), word);
+                search(nm, need, x, y, z, o, p, nn, w);
+                wave_sync<GM>();
+                // (the thresholds of the lanes not searched are unchanged)
+                const FireThr tn = threshold(w, ch, xA, b1, b2);
+                bool ok = nn != kNoHole;
+                if (it == 0) ok = ok && fires(u, tn);
+                else ok = ok && accepted(tn, t, blk, word, o, (uint32_t)(it - 1));
+                if (need) cand = ok;
+                t = tn;
+                have_t = true;
+            }
+            const uint64_t cm = ballot(cand);
+            if (cm == 0) break;
+            bool win = cand;
+            if ((cm & (cm - 1)) != 0) {                  // (a single candidate is not contested)
+                if (cand) claim(nn, o);
+                wave_sync<GM>();
+                // the claim field holds the lowest candidate index for that hole
+                uint32_t meta = 0u;
+                if (cand) meta = hole_u[4 * nn + 3];
+                win = cand && (meta >> 16) == o;
+                if (win) hole_u[4 * nn + 3] = 0xFFFF0000u | (meta & 0xFFFFu);
+            }
+            if (win) {
+                hole_f[4 * nn] = kDeadHoleX;
+                est[p] = kDeadSlot;
+                nf[p] = (uint8_t)kNever;
+                won = true;
+            }
+            wins += (uint32_t)__popcll(ballot(win));
+            wave_sync<GM>();
+            need = cand && !win;
+            cand = false;
+            if (it + 1 == MCL_MAX_ROUNDS || ballot(need) == 0) break;
+        }
+        finish_step(n, wins);
+        // the candidates that stay: their next firing step in the window
+        const bool stay = act && !won;
+        uint64_t more = 0;
+        if (ballot(stay) != 0) {
+            uint32_t f = kNever;
+            if (rel + 1 < len) more = group_scan(ballot(stay && nn != kNoHole), o, w, rel + 1, f);
+            if (stay) {
+                nf[p] = (uint8_t)f;
+                if (f != kNever) atomicOr(&rowm[p >> 6], 1ull << f);
+            }
+            wave_sync<GM>();
+        }
+        return more;
+    };
+
+    // A step with many candidates, every wave: the candidates of the wave's own rows
+    // [r_lo, r_lo + nr), gathered into chunks of 64 (flags per chunk in 64-bit
+    // masks).  Returns the cluster's wins.
+    auto heavy_step = [&](int rel) -> uint32_t {
+        const int n = nb0 + rel;
+        const uint32_t blk = (uint32_t)n >> 2;
+        const int word = n & 3;
+        const float xA = lane_value(l_xA, rel), b1 = lane_value(l_b1, rel), b2 = lane_value(l_b2, rel);
+        int r_lo = 0, nr = rows;
         if constexpr (NW > 1) {
             const int per = (rows + NW - 1) / NW;
             r_lo = min(rows, wv * per);
             nr = min(rows, r_lo + per) - r_lo;
-            slot_end = min(n_slots, (r_lo + nr) * kWave);
         }
-        uint32_t* const rq_w = rq + r_lo * kWave;     // this wave's part of the queue
-        const float bmax = fmaxf(b1dt, b2dt);
-
-        // Pass A, two rows per iteration: an electron whose nearest hole was removed
-        // and whose draw would fire against its old w is queued for a new search
-        // (its test waits for it); one whose draw fails even against the old w stays
-        // as it is; every other live electron takes its fire test now.  Deferring
-        // the search to here changes nothing: no hole disappears in between.
-        uint64_t cand = 0, stale = 0, stale_ch = 0;
-        int nq = 0;
-        if ((int)blk != cache_blk) {
-            cache_blk = (int)blk;
-            cache_pairs = 0u;
-        }
-        auto pass_a_pair = [&](int r, auto slot_tag) {      // r: the wave's row index
-            constexpr int q = decltype(slot_tag)::value;   // register cache slot, -1: none
-            const int p0 = (r_lo + r) * kWave + lane, p1 = p0 + kWave;
-            const uint32_t st0 = p0 < slot_end ? est[p0] : kDeadSlot;
-            const uint32_t st1 = p1 < slot_end ? est[p1] : kDeadSlot;
-            const float w0 = p0 < slot_end ? ew[p0] : 0.0f, w1 = p1 < slot_end ? ew[p1] : 0.0f;
-            const uint32_t o0 = st0 & 0xFFFFu, o1 = st1 & 0xFFFFu;
-            // Below x = 2^-32 (in either channel) the threshold is 0: no draw can
-            // fire, and a stale electron keeps waiting.  Rows whose lanes all sit
-            // there (early in a heating ramp) skip their draws.  (A slot that keeps
-            // the threshold holds 0 exactly then.)
-            const bool live0 = fixedw ? __float_as_uint(w0) != 0u
-                                      : __builtin_fmaf(bmax, w0, xA) >= 0x1p-32f;
-            const bool live1 = fixedw ? __float_as_uint(w1) != 0u
-                                      : __builtin_fmaf(bmax, w1, xA) >= 0x1p-32f;
-            if (ballot(live0 || live1) == 0) return;
-            uint32_t u0 = 0u, u1 = 0u;
-            bool ch0 = always2, ch1 = always2;
-            bool hit = false;
-            if constexpr (q >= 0) hit = ((cache_pairs >> q) & 1u) != 0u;
-            if (hit) {
-                if constexpr (q >= 0) {
-                    u0 = pick_word(cfa[q], word);
-                    u1 = pick_word(cfb[q], word);
-                    if (two_ch) {
-                        ch0 = ((cch[q] >> word) & 1u) != 0u;
-                        ch1 = ((cch[q] >> (4 + word)) & 1u) != 0u;
-                    }
-                }
-            } else {
-                const u32x4 fa = philox10(blk, o0, prun, c3f, k0, k1);
-                const u32x4 fb = philox10(blk, o1, prun, c3f, k0, k1);
-                u0 = pick_word(fa, word);
-                u1 = pick_word(fb, word);
-                uint32_t cb = 0u;
-                if (two_ch) {
-                    const u32x4 ca = philox10(blk, o0, prun, c3c, k0, k1);
-                    const u32x4 cc = philox10(blk, o1, prun, c3c, k0, k1);
-                    cb = (uint32_t)((uint64_t)ca.x < ret_thr) | (uint32_t)((uint64_t)ca.y < ret_thr) << 1 |
-                         (uint32_t)((uint64_t)ca.z < ret_thr) << 2 | (uint32_t)((uint64_t)ca.w < ret_thr) << 3 |
-                         (uint32_t)((uint64_t)cc.x < ret_thr) << 4 | (uint32_t)((uint64_t)cc.y < ret_thr) << 5 |
-                         (uint32_t)((uint64_t)cc.z < ret_thr) << 6 | (uint32_t)((uint64_t)cc.w < ret_thr) << 7;
-                    ch0 = ((cb >> word) & 1u) != 0u;
-                    ch1 = ((cb >> (4 + word)) & 1u) != 0u;
-                }
-                if constexpr (q >= 0) {
-                    cfa[q] = fa;
-                    cfb[q] = fb;
-                    cch[q] = cb;
-                    cache_pairs |= 1u << q;
-                }
-            }
-            const bool s0 = test_fire(st0, o0, p0, u0, slot_thr(w0, ch0), r, cand);
-            const bool s1 = test_fire(st1, o1, p1, u1, slot_thr(w1, ch1), r + 1, cand);
-            const uint64_t m0 = ballot(s0);
-            if (s0) rq_w[nq + lanes_below(m0)] = ((uint32_t)p0 << 16) | o0;
-            nq += __popcll(m0);
-            const uint64_t m1 = ballot(s1);
-            if (s1) rq_w[nq + lanes_below(m1)] = ((uint32_t)p1 << 16) | o1;
-            nq += __popcll(m1);
-            stale |= ((uint64_t)s0 << r) | ((uint64_t)s1 << (r + 1));
-            stale_ch |= ((uint64_t)ch0 << r) | ((uint64_t)ch1 << (r + 1));
-        };
-        if (NW == 1 || nr > 0) pass_a_pair(0, CacheSlot<0>{});
-        if (nr > 2) pass_a_pair(2, CacheSlot<1>{});
-        if (nr > 4) pass_a_pair(4, CacheSlot<2>{});
-        if (nr > 6) pass_a_pair(6, CacheSlot<3>{});
-        for (int r = 2 * kCachePairs; r < nr; r += 2) pass_a_pair(r, CacheSlot<-1>{});
-        if (nq > 0) {
-            queue_sync<NW, GM>();
-            search_queue(rq_w, nq);
-            queue_sync<NW, GM>();
-            uint64_t m = rows_any(stale, nr);
+        uint16_t* const my = lst + r_lo * kWave;
+        const int k = gather(rel, 0, r_lo, r_lo + nr, my, nr * kWave);
+        nr = (k + kWave - 1) / kWave;    // chunks from here on
+        uint64_t cand = 0;               // per chunk: this lane's candidate claims a hole
+        uint32_t wins = 0, step_wins = 0;
+        uint64_t todo = nr >= 64 ? ~0ull : (1ull << nr) - 1ull;   // chunks with a search or test
+        uint64_t lose = 0;
+        for (int round = 0;; ++round) {
+            // round 0: the candidates whose hole is gone; later: the losers, retried
+            cand = 0;
+            uint64_t m = todo;
             while (m != 0) {
                 const int r = __builtin_ctzll(m);
                 m &= m - 1;
-                const int p = (r_lo + r) * kWave + lane;
-                if ((stale >> r) & 1ull) {
-                    // the draw and channel of pass A, the new w
-                    const uint32_t st = est[p];
-                    const bool ch = (stale_ch >> r) & 1ull;
-                    fire_tail(st, st & 0xFFFFu, p, ethr[p], slot_thr(ew[p], ch), r, cand);
+                const int q = r * kWave + lane;
+                const bool is = round == 0 ? q < k : ((lose >> r) & 1ull) != 0;
+                const int p = is ? (int)my[q] : 0;
+                const uint32_t st = is ? est[p] : 0u;
+                float w = is ? ew[p] : 0.0f;
+                const uint32_t o = st & 0xFFFFu;
+                uint32_t nn = st >> 16;
+                bool ch = always2;
+                if (two_ch) ch = channel_word(philox10(blk, o, prun, c3c, k0, k1), word);
+                const bool need = round == 0 ? is && hole_f[4 * nn] == kDeadHoleX : is;
+                bool ok = is;
+                const uint64_t nm = ballot(need);
+                if (nm != 0) {
+                    float x, y, z;
+                    egen.xyz(o, x, y, z);
+                    const FireThr to = threshold(w, ch, xA, b1, b2);
+                    search(nm, need, x, y, z, o, p, nn, w);
+                    const FireThr tn = threshold(w, ch, xA, b1, b2);
+                    bool good;
+                    if (round == 0)
+                        good = fires(pick_word(philox10(blk, o, prun, c3f, k0, k1), word), tn);
+                    else
+                        good = accepted(tn, to, blk, word, o, (uint32_t)(round - 1));
+                    if (need) ok = nn != kNoHole && good;
+                }
+                if (ok) {
+                    claim(nn, o);
+                    cand |= 1ull << r;
                 }
             }
-        }
-        uint64_t rowmask = rows_any(cand, nr);
-        uint32_t wins = 0;          // this wave's winners in this step
-        uint32_t step_wins = 0;     // the cluster's
-        const bool any_cand = any_wave(rowmask != 0);
-        quiet_run = any_cand ? 0 : quiet_run + 1;
-        if (any_cand) {
-            for (int round = 0;; ++round) {
-                if (round > 0) {
-                    // claims of this round's candidates (losers accepted for a retry)
-                    uint64_t m = rowmask;
-                    while (m != 0) {
-                        const int r = __builtin_ctzll(m);
-                        m &= m - 1;
-                        if ((cand >> r) & 1ull) {
-                            const uint32_t st = est[(r_lo + r) * kWave + lane];
-                            claim(st >> 16, st & 0xFFFFu);
-                        }
-                    }
-                    if constexpr (NW > 1) {
-                        if (!any_wave(rowmask != 0)) break;   // also the claims' barrier
-                    }
-                }
-                if constexpr (NW == 1) __syncthreads();
-                // winners: the claim field holds the lowest candidate index for that hole
-                uint64_t lose = 0;
-                uint64_t m = rowmask;
-                while (m != 0) {
-                    const int r = __builtin_ctzll(m);
-                    m &= m - 1;
-                    const int p = (r_lo + r) * kWave + lane;
-                    const bool is_cand = (cand >> r) & 1ull;
-                    bool win = false;
-                    uint32_t nn = 0, meta = 0;
-                    if (is_cand) {
-                        const uint32_t st = est[p];
-                        nn = st >> 16;
-                        meta = hole_u[4 * nn + 3];
-                        win = (meta >> 16) == (st & 0xFFFFu);
-                        if (!win) lose |= 1ull << r;
-                    }
+            const uint64_t crows = rows_any(cand, nr);
+            if constexpr (NW == 1) {
+                if (crows == 0) break;
+                wave_sync<GM>();
+            } else {
+                if (!any_wave(crows != 0)) break;        // also the claims' barrier
+            }
+            // winners: the claim field holds the lowest candidate index for that hole
+            lose = 0;
+            m = crows;
+            while (m != 0) {
+                const int r = __builtin_ctzll(m);
+                m &= m - 1;
+                bool win = false;
+                if ((cand >> r) & 1ull) {
+                    const int p = (int)my[r * kWave + lane];
+                    const uint32_t st = est[p];
+                    const uint32_t nn = st >> 16;
+                    const uint32_t meta = hole_u[4 * nn + 3];
+                    win = (meta >> 16) == (st & 0xFFFFu);
                     if (win) {
                         hole_u[4 * nn + 3] = 0xFFFF0000u | (meta & 0xFFFFu);
                         hole_f[4 * nn] = kDeadHoleX;
                         est[p] = kDeadSlot;
-                    }
-                    wins += (uint32_t)__popcll(ballot(win));
-                }
-                uint64_t lrows;
-                if constexpr (NW == 1) {
-                    __syncthreads();
-                    if (round + 1 == MCL_MAX_ROUNDS) break;
-                    lrows = rows_any(lose, rows);
-                    if (lrows == 0) break;
-                } else {
-                    // the removed holes are visible to every wave after this barrier
-                    lrows = rows_any(lose, nr);
-                    const uint32_t* x = exchange(wins | (lrows != 0 ? 0x80000000u : 0u));
-                    uint32_t t = 0, l = 0;
-#pragma unroll
-                    for (int w = 0; w < NW; ++w) {
-                        t += x[w] & 0x7FFFFFFFu;
-                        l |= x[w] >> 31;
-                    }
-                    step_wins = uniform(t);
-                    if (round + 1 == MCL_MAX_ROUNDS) break;
-                    if (uniform(l) == 0u) break;
-                }
-
-                // a loser's hole is gone: search again now, then it retries in the same
-                // step, accepted with probability T_new / T_old (thinning of the draw
-                // it already won).  Other electrons that lost their hole are searched
-                // again at the start of the next step.
-                int nl = 0;
-                m = lrows;
-                while (m != 0) {
-                    const int r = __builtin_ctzll(m);
-                    m &= m - 1;
-                    const int p = (r_lo + r) * kWave + lane;
-                    const bool l = (lose >> r) & 1ull;
-                    const uint64_t mm = ballot(l);
-                    if (l) rq_w[nl + lanes_below(mm)] = ((uint32_t)p << 16) | (est[p] & 0xFFFFu);
-                    nl += __popcll(mm);
-                }
-                queue_sync<NW, GM>();
-                search_queue(rq_w, nl);
-                queue_sync<NW, GM>();
-                cand = 0;
-                const uint32_t c3r = psim | (MCL_TAG_RETRY0 + (uint32_t)round);
-                m = lrows;
-                while (m != 0) {
-                    const int r = __builtin_ctzll(m);
-                    m &= m - 1;
-                    const int p = (r_lo + r) * kWave + lane;
-                    if ((lose >> r) & 1ull) {
-                        const uint32_t st = est[p];
-                        const uint32_t o = st & 0xFFFFu, nn = st >> 16;
-                        if (nn != kNoHole) {
-                            bool chan2 = always2;
-                            if (two_ch) {
-                                const u32x4 rc = philox10(blk, o, prun, c3c, k0, k1);
-                                chan2 = (uint64_t)pick_word(rc, word) < ret_thr;
-                            }
-                            const FireThr t = slot_thr(ew[p], chan2);
-                            const uint64_t Tn = t.always ? 0x100000000ull : (uint64_t)t.thr;
-                            const uint32_t eo = ethr[p];
-                            const uint64_t To = eo == 0xFFFFFFFFu ? 0x100000000ull : (uint64_t)eo;
-                            bool acc = Tn >= To;
-                            if (!acc) {
-                                const u32x4 rr = philox10(blk, o, prun, c3r, k0, k1);
-                                acc = (uint64_t)pick_word(rr, word) * To < (Tn << 32);
-                            }
-                            if (acc) {
-                                ethr[p] = t.always ? 0xFFFFFFFFu : t.thr;
-                                cand |= 1ull << r;
-                            }
-                        }
+                    } else {
+                        lose |= 1ull << r;
                     }
                 }
-                rowmask = rows_any(cand, nr);
-                if constexpr (NW == 1) {
-                    if (rowmask == 0) break;
-                }
+                wins += (uint32_t)__popcll(ballot(win));
             }
-            if constexpr (NW == 1) step_wins = wins;
-            n_live -= (int)step_wins;
-
-            // lazy stable compaction when a 64-slot row can be dropped (an electron
-            // waiting for a new search moves with its stale nearest hole)
-            if ((n_live + kWave - 1) / kWave < rows) {
-                if constexpr (NW == 1) {
-                    int base = 0;
-                    for (int r = 0; r < rows; ++r) {
-                        const int p = r * kWave + lane;
-                        const uint32_t st = p < n_slots ? est[p] : kDeadSlot;
-                        const float w = p < n_slots ? ew[p] : 0.0f;
-                        const bool keep = st != kDeadSlot;
-                        const uint64_t km = ballot(keep);
-                        if (keep) {
-                            const int q = base + lanes_below(km);
-                            est[q] = st;
-                            ew[q] = w;
-                        }
-                        base += __popcll(km);
-                    }
-                    n_slots = base;
-                } else {
-                    // per-wave keep counts give each wave's first new slot; the rows
-                    // are rewritten into the spare pair (rq, ethr), which becomes est/ew
-                    uint32_t kept = 0;
-                    for (int r = 0; r < nr; ++r) {
-                        const int p = (r_lo + r) * kWave + lane;
-                        const uint32_t st = p < slot_end ? est[p] : kDeadSlot;
-                        kept += (uint32_t)__popcll(ballot(st != kDeadSlot));
-                    }
-                    const uint32_t* x = exchange(kept);
-                    uint32_t before = 0, total = 0;
+            todo = rows_any(lose, nr);
+            bool any_lose;
+            if constexpr (NW == 1) {
+                wave_sync<GM>();
+                step_wins = wins;
+                any_lose = todo != 0;
+            } else {
+                // the removed holes are visible to every wave after this barrier
+                const uint32_t* x = exchange(wins | (todo != 0 ? 0x80000000u : 0u));
+                uint32_t t = 0, l = 0;
 #pragma unroll
-                    for (int w = 0; w < NW; ++w) {
-                        before += w < wv ? x[w] : 0u;
-                        total += x[w];
-                    }
-                    int base = (int)uniform(before);
-                    uint32_t* const n_est = rq;
-                    float* const n_ew = (float*)ethr;
-                    for (int r = 0; r < nr; ++r) {
-                        const int p = (r_lo + r) * kWave + lane;
-                        const uint32_t st = p < slot_end ? est[p] : kDeadSlot;
-                        const float w = p < slot_end ? ew[p] : 0.0f;
-                        const bool keep = st != kDeadSlot;
-                        const uint64_t km = ballot(keep);
-                        if (keep) {
-                            const int q = base + lanes_below(km);
-                            n_est[q] = st;
-                            n_ew[q] = w;
-                        }
-                        base += __popcll(km);
-                    }
-                    rq = est;
-                    ethr = (uint32_t*)ew;
-                    est = n_est;
-                    ew = n_ew;
-                    n_slots = (int)uniform(total);
+                for (int w = 0; w < NW; ++w) {
+                    t += x[w] & 0x7FFFFFFFu;
+                    l |= x[w] >> 31;
                 }
-                cache_pairs = 0u;                   // electrons moved to other slots
-                __syncthreads();
+                step_wins = uniform(t);
+                any_lose = uniform(l) != 0u;
+            }
+            if (round + 1 == MCL_MAX_ROUNDS || !any_lose) break;
+        }
+        // the candidates that stay: their next firing step in the window
+        for (int r = 0; r < nr; ++r) {
+            const int q = r * kWave + lane;
+            const bool is = q < k;
+            const int p = is ? (int)my[q] : 0;
+            const uint32_t st = is ? est[p] : kDeadSlot;
+            const float w = is ? ew[p] : 0.0f;
+            uint32_t f = kNever;
+            if (rel + 1 < len)
+                (void)first_fire(st != kDeadSlot && (st >> 16) != kNoHole, st & 0xFFFFu, w, rel + 1, f);
+            if (is) {
+                nf[p] = (uint8_t)f;
+                if (f != kNever) atomicOr(&rowm[p >> 6], 1ull << f);
             }
         }
-        finish_step(step_wins);
-        ++n;
+        if constexpr (NW == 1) wave_sync<GM>();
+        else __syncthreads();
+        return step_wins;
+    };
+
+    // The electrons of rows [r_lo, r_hi) that fire in sub-window j and whose nearest hole
+    // is gone already: searched now, together, instead of one step after the other.
+    // Exact: the hole found is no farther than the one a search in the firing step
+    // would find, and is that one if it still lives then (else it is searched again
+    // there); an electron whose draw fails against the new threshold is scanned again.
+    auto pre_search = [&](int j, int r_lo, int r_hi) {
+        uint16_t* const my = lst + r_lo * kWave;
+        const int k = gather(j * kSub, kLogSub, r_lo, r_hi, my, (r_hi - r_lo) * kWave);
+        for (int c0 = 0; c0 < k; c0 += kWave) {
+            const bool is = c0 + lane < k;
+            const int p = is ? (int)my[c0 + lane] : 0;
+            const uint32_t st = is ? est[p] : 0u;
+            const uint32_t o = st & 0xFFFFu;
+            uint32_t nn = st >> 16;
+            const bool need = is && hole_f[4 * nn] == kDeadHoleX;
+            const uint64_t nm = ballot(need);
+            if (nm == 0) continue;
+            float x, y, z, w = 0.0f;
+            egen.xyz(o, x, y, z);
+            search(nm, need, x, y, z, o, p, nn, w);
+            const int rel = need ? (int)nf[p] : 0;
+            const int n = nb0 + rel;
+            const uint32_t u = pick_word(philox10((uint32_t)n >> 2, o, prun, c3f, k0, k1), n & 3);
+            bool ch = always2;
+            if (two_ch) ch = channel_word(philox10((uint32_t)n >> 2, o, prun, c3c, k0, k1), n & 3);
+            const FireThr t = threshold(w, ch, __shfl(l_xA, rel), __shfl(l_b1, rel), __shfl(l_b2, rel));
+            const bool again = need && !(nn != kNoHole && fires(u, t));
+            if (ballot(again) != 0) {
+                uint32_t f = kNever;
+                (void)group_scan(ballot(again && nn != kNoHole), o, w, rel + 1, f);
+                if (again) {
+                    nf[p] = (uint8_t)f;
+                    if (f != kNever) atomicOr(&rowm[p >> 6], 1ull << f);
+                }
+            }
+        }
+        wave_sync<GM>();
+    };
+
+    // ---- windows (the step loop, simulate.py:51-92) ------------------------------
+    // (NW > 1) what wave 0 publishes: {heavy step or kNever, n_live, steps (two words)}
+    uint32_t* const pub = xch + 2 * NW + 1;
+    while (nb0 < step_limit && n_live > 0) {
+        const int w_len = min(kWindow, step_limit - nb0);
+        if (nb0 == 0 || ramp || w_len != len) {
+            len = w_len;
+            window_scalars();
+        }
+        rows = (n_slots + kWave - 1) / kWave;
+        // stable compaction in place, wave 0 (an electron waiting for a new search moves
+        // with its stale nearest hole)
+        if ((n_live + kWave - 1) / kWave <= rows - max(1, rows >> 3)) {
+            if (wv == 0) {
+                int base = 0;
+                for (int r = 0; r < rows; ++r) {
+                    const int p = r * kWave + lane;
+                    const uint32_t st = p < n_slots ? est[p] : kDeadSlot;
+                    const float w = p < n_slots ? ew[p] : 0.0f;
+                    const bool keep = st != kDeadSlot;
+                    const uint64_t km = ballot(keep);
+                    if (keep) {
+                        const int q = base + lanes_below(km);
+                        est[q] = st;
+                        ew[q] = w;
+                    }
+                    base += __popcll(km);
+                    wave_sync<GM>();
+                }
+            }
+            n_slots = n_live;
+            rows = (n_slots + kWave - 1) / kWave;
+            __syncthreads();
+        }
+        // scan: rows wv, wv + NW, ...
+        for (int r = wv; r < rows; r += NW) {
+            const int p = r * kWave + lane;
+            const uint32_t st = p < n_slots ? est[p] : kDeadSlot;
+            const float w = p < n_slots ? ew[p] : 0.0f;
+            uint32_t f = kNever;
+            const uint64_t m =
+                first_fire(st != kDeadSlot && (st >> 16) != kNoHole, st & 0xFFFFu, w, 0, f);
+            nf[p] = (uint8_t)f;
+            if (lane == 0) rowm[r] = m;
+        }
+        if constexpr (NW == 1) wave_sync<GM>();
+        else __syncthreads();
+
+        // Sub-windows of kSub steps.  While wave 0 takes the events of one, the others
+        // search ahead for the next one with events (they touch only electrons that
+        // fire there, wave 0 only those that fire now).
+        uint64_t steps = 0;              // steps of the window that may have candidates
+        auto all_rows = [&](int above) {
+            uint64_t s = 0;
+            for (int r = lane; r < rows; r += kWave) s |= (uint64_t)rowm[r];
+            steps = ((uint64_t)wave_or_u32((uint32_t)(s >> 32)) << 32) | wave_or_u32((uint32_t)s);
+            steps &= above >= kWindow ? 0ull : ~0ull << above;
+        };
+        all_rows(0);
+        uint32_t searched = 0;           // sub-windows searched ahead
+        for (int j = 0; j < kWindow / kSub && n_live > 0; ++j) {
+            const uint64_t sub = ((1ull << kSub) - 1ull) << (j * kSub);
+            if ((steps & sub) == 0) continue;
+            // (from steps, which every wave has alike here: searched decides on a barrier)
+            int next = -1;               // the next sub-window with events, to search ahead
+            if constexpr (NW > 1) {
+                const uint64_t rest = j + 1 < kWindow / kSub ? steps & (~0ull << ((j + 1) * kSub)) : 0ull;
+                if (rest != 0) next = (int)__builtin_ctzll(rest) / kSub;
+                if (next >= 0 && ((searched >> next) & 1u) != 0u) next = -1;
+            }
+            if (NW > 1 && ((searched >> j) & 1u) == 0u) {
+                const int per = (rows + NW - 1) / NW;
+                const int lo = min(rows, wv * per);
+                pre_search(j, lo, min(rows, lo + per));
+                if constexpr (NW > 1) __syncthreads();
+                if (wv == 0) all_rows(j * kSub);
+            }
+            bool ahead = false;
+            for (;;) {
+                uint32_t heavy = kNever;
+                if (wv == 0) {
+                    while ((steps & sub) != 0) {
+                        const int rel = __builtin_ctzll(steps);
+                        const int k = gather(rel, 0, 0, rows, lst + e_cap, kWave);
+                        if (k > kWave) {
+                            heavy = (uint32_t)rel;
+                            break;
+                        }
+                        steps &= steps - 1;
+                        if (k == 0) continue;
+                        steps |= light_step(rel, lane < k, lane < k ? (int)lst[e_cap + lane] : 0);
+                        if (n_live == 0) {
+                            steps = 0;
+                            break;
+                        }
+                    }
+                } else if (!ahead && next >= 0) {
+                    const int per = (rows + NW - 2) / (NW > 1 ? NW - 1 : 1);
+                    const int lo = min(rows, (wv - 1) * per);
+                    pre_search(next, lo, min(rows, lo + per));
+                }
+                ahead = true;
+                if constexpr (NW > 1) {
+                    if (tid == 0) {
+                        pub[0] = heavy;
+                        pub[1] = (uint32_t)n_live;
+                    }
+                    __syncthreads();
+                    heavy = uniform(pub[0]);
+                    n_live = (int)uniform(pub[1]);
+                }
+                if (heavy == kNever) break;
+                const uint32_t w = heavy_step((int)heavy);
+                if (wv == 0) {
+                    finish_step(nb0 + (int)heavy, w);
+                    all_rows((int)heavy + 1);
+                    if (n_live == 0) steps = 0;
+                }
+            }
+            if constexpr (NW > 1) {
+                if (next >= 0) searched |= 1u << next;
+                // the steps left, with what the searches ahead moved
+                if (wv == 0) {
+                    all_rows((j + 1) * kSub);
+                    if (lane == 0) {
+                        pub[2] = (uint32_t)steps;
+                        pub[3] = (uint32_t)(steps >> 32);
+                    }
+                }
+                __syncthreads();
+                steps = ((uint64_t)uniform(pub[3]) << 32) | uniform(pub[2]);
+            }
+        }
+        nb0 += len;
     }
-    if (bin < nb) {
-        if (tid == 0) cnt[bin] = bin_acc;
-        ++bin;
+    int steps_run = n_acc;               // up to the step that emptied the cluster
+    if (n_live > 0) {
+        lsteps += (uint64_t)n_live * (uint64_t)(step_limit - n_acc);
+        steps_run = step_limit;
     }
-    for (int b = bin + tid; b < a.row_len; b += NW * kWave) cnt[b] = 0u;
+    if (tid == 0 && bin_acc != 0u) cnt[bin] = bin_acc;
     if (a.live_steps != nullptr && tid == 0) a.live_steps[c] = lsteps;
 
     // (state dumps are one-wave launches only)
     if (NW == 1 && a.dump.enabled) {
-        // searches deferred to the next step happen now, so the dump shows every
+        // searches deferred to a later step happen now, so the dump shows every
         // survivor's current nearest hole
         __syncthreads();
-        int nq = 0;
         for (int r = 0; r * kWave < n_slots; ++r) {
             const int p = r * kWave + lane;
             const uint32_t st = p < n_slots ? est[p] : kDeadSlot;
-            const bool s = hole_dead(st >> 16);
-            const uint64_t m = ballot(s);
-            if (s) rq[nq + lanes_below(m)] = ((uint32_t)p << 16) | (st & 0xFFFFu);
-            nq += __popcll(m);
+            const uint32_t nn = st >> 16;
+            const bool s = nn != kNoHole && hole_f[4 * (nn != kNoHole ? nn : 0u)] == kDeadHoleX;
+            float x = 0.0f, y = 0.0f, z = 0.0f;
+            if (s) egen.xyz(st & 0xFFFFu, x, y, z);
+            const uint64_t key = nn_resolve<WIDE>(grid, s, x, y, z, lane, dist_evals);
+            if (s) {
+                uint32_t slot;
+                float w;
+                nn_from_key(key, alpha_f, slot, w);
+                est[p] = (slot << 16) | (st & 0xFFFFu);
+                ew[p] = w;
+            }
         }
-        __syncthreads();
-        search_queue(rq, nq);
         __syncthreads();
     }
 
@@ -927,13 +946,13 @@ __device__ __forceinline__ void run_cluster(const LaunchArgs& a, const int c,
 // from order[] (null: 0 .. n_order-1) through a global atomic ticket until the
 // list is exhausted.  Every workgroup leaves the loop when the ticket passes
 // n_order.  The global-memory form always runs persistent.
-template <bool GM, bool FW, bool QW>
+template <bool GM, bool WIDE>
 __global__ __launch_bounds__(64, GM ? 2 : 1) void fixed_dt_kernel(LaunchArgs a)
 {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     if (a.queue == nullptr) {
         const int i = blockIdx.x;
-        if (i < a.n_order) run_cluster<1, GM, FW, QW>(a, a.order != nullptr ? a.order[i] : i, lds_raw);
+        if (i < a.n_order) run_cluster<1, GM, WIDE>(a, a.order != nullptr ? a.order[i] : i, lds_raw);
         return;
     }
     for (;;) {
@@ -941,7 +960,7 @@ __global__ __launch_bounds__(64, GM ? 2 : 1) void fixed_dt_kernel(LaunchArgs a)
         if (threadIdx.x == 0) i = (int)atomicAdd(a.queue, 1u);
         i = __shfl(i, 0);
         if (i >= a.n_order) break;
-        run_cluster<1, GM, FW, QW>(a, a.order != nullptr ? a.order[i] : i, lds_raw);
+        run_cluster<1, GM, WIDE>(a, a.order != nullptr ? a.order[i] : i, lds_raw);
         __syncthreads();
     }
 }
@@ -950,102 +969,73 @@ __global__ __launch_bounds__(64, GM ? 2 : 1) void fixed_dt_kernel(LaunchArgs a)
 // most 256 VGPRs a wave, as the one-wave kernel).  The persistent ticket goes
 // through LDS (the word after the exchange slots), read by every wave between
 // two barriers, so all waves take the same cluster and leave the loop together.
-template <int NW, bool GM, bool FW, bool QW>
+template <int NW, bool GM, bool WIDE>
 __global__ __launch_bounds__(NW * 64, 2) void fixed_dt_mw_kernel(LaunchArgs a)
 {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     if (a.queue == nullptr) {
         const int i = blockIdx.x;
-        if (i < a.n_order) run_cluster<NW, GM, FW, QW>(a, a.order != nullptr ? a.order[i] : i, lds_raw);
+        if (i < a.n_order) run_cluster<NW, GM, WIDE>(a, a.order != nullptr ? a.order[i] : i, lds_raw);
         return;
     }
     uint32_t* const ticket =
         (GM ? (uint32_t*)lds_raw
-            : (uint32_t*)(lds_raw + 16 * a.h_cap + 4 * a.g_cap + 16 * a.e_cap)) + 2 * NW;
+            : (uint32_t*)(lds_raw + 16 * a.h_cap + 4 * a.g_cap +
+                          fixed_dt_electron_bytes(a.e_cap))) + 2 * NW;
     for (;;) {
         if (threadIdx.x == 0) *ticket = atomicAdd(a.queue, 1u);
         __syncthreads();
         const int i = (int)uniform(*ticket);
         __syncthreads();
         if (i >= a.n_order) break;
-        run_cluster<NW, GM, FW, QW>(a, a.order != nullptr ? a.order[i] : i, lds_raw);
+        run_cluster<NW, GM, WIDE>(a, a.order != nullptr ? a.order[i] : i, lds_raw);
         __syncthreads();
     }
 }
 
-template <bool GM, bool FW, bool QW>
-const void* fixed_dt_fn_t(int waves)
+template <bool GM, bool WIDE>
+const void* fixed_dt_fn(int waves)
 {
-    return waves == 8 ? (const void*)fixed_dt_mw_kernel<8, GM, FW, QW>
-         : waves == 4 ? (const void*)fixed_dt_mw_kernel<4, GM, FW, QW>
-         : waves == 2 ? (const void*)fixed_dt_mw_kernel<2, GM, FW, QW>
-                      : (const void*)fixed_dt_kernel<GM, FW, QW>;
+    return waves == 8 ? (const void*)fixed_dt_mw_kernel<8, GM, WIDE>
+         : waves == 4 ? (const void*)fixed_dt_mw_kernel<4, GM, WIDE>
+         : waves == 2 ? (const void*)fixed_dt_mw_kernel<2, GM, WIDE>
+                      : (const void*)fixed_dt_kernel<GM, WIDE>;
 }
 
-// The build of the NW-wave kernel with the quiet window or not (QW) and with the
-// fixed-threshold path or not (fw).
-template <bool GM, bool QW>
-const void* fixed_dt_fn(int waves, bool fw)
-{
-    return fw ? fixed_dt_fn_t<GM, true, QW>(waves) : fixed_dt_fn_t<GM, false, QW>(waves);
-}
-
-template <bool GM, bool FW, bool QW>
-void launch_fixed_dt_w(const LaunchArgs& a, dim3 g, unsigned lds, int waves, hipStream_t stream)
-{
-    if (waves == 8)
-        hipLaunchKernelGGL((fixed_dt_mw_kernel<8, GM, FW, QW>), g, dim3(8 * kWave), lds, stream, a);
-    else if (waves == 4)
-        hipLaunchKernelGGL((fixed_dt_mw_kernel<4, GM, FW, QW>), g, dim3(4 * kWave), lds, stream, a);
-    else if (waves == 2)
-        hipLaunchKernelGGL((fixed_dt_mw_kernel<2, GM, FW, QW>), g, dim3(2 * kWave), lds, stream, a);
-    else
-        hipLaunchKernelGGL((fixed_dt_kernel<GM, FW, QW>), g, dim3(kWave), lds, stream, a);
-}
-
-// The builds with the quiet window (QW) or without are instantiated in separate
-// sources (mc_fixed_dt*.hip without it, mc_fixed_dt*_window.hip with it), which
-// the launch functions choose between by a.quiet_window.
-template <bool GM, bool QW>
+template <bool GM, bool WIDE>
 hipError_t launch_fixed_dt_t(const LaunchArgs& a, int grid, unsigned lds, int waves,
                              hipStream_t stream)
 {
     const dim3 g((unsigned)grid);
-    if (a.fixed_thr != 0)
-        launch_fixed_dt_w<GM, true, QW>(a, g, lds, waves, stream);
+    if (waves == 8)
+        hipLaunchKernelGGL((fixed_dt_mw_kernel<8, GM, WIDE>), g, dim3(8 * kWave), lds, stream, a);
+    else if (waves == 4)
+        hipLaunchKernelGGL((fixed_dt_mw_kernel<4, GM, WIDE>), g, dim3(4 * kWave), lds, stream, a);
+    else if (waves == 2)
+        hipLaunchKernelGGL((fixed_dt_mw_kernel<2, GM, WIDE>), g, dim3(2 * kWave), lds, stream, a);
     else
-        launch_fixed_dt_w<GM, false, QW>(a, g, lds, waves, stream);
+        hipLaunchKernelGGL((fixed_dt_kernel<GM, WIDE>), g, dim3(kWave), lds, stream, a);
     return hipGetLastError();
 }
 
-// Resident workgroups per CU of the NW-wave kernel with this much dynamic LDS:
-// the smaller count of its two fixed-threshold builds.
-template <bool GM, bool QW>
+// Resident workgroups per CU of the NW-wave kernel with this much dynamic LDS.
+template <bool GM, bool WIDE>
 hipError_t fixed_dt_occupancy_t(size_t lds, int waves, int* blocks_per_cu)
 {
-    int b0 = 0, b1 = 0;
-    hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&b0, fixed_dt_fn<GM, QW>(waves, false),
-                                                                waves * kWave, lds);
-    if (e == hipSuccess)
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&b1, fixed_dt_fn<GM, QW>(waves, true),
-                                                         waves * kWave, lds);
-    *blocks_per_cu = b0 < b1 ? b0 : b1;
-    return e;
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, fixed_dt_fn<GM, WIDE>(waves),
+                                                        waves * kWave, lds);
 }
 
-// Dynamic-LDS limits of the builds of one form (GM) and window choice (QW).
-template <bool GM, bool QW>
+// Dynamic-LDS limits of the kernels of one form.
+template <bool GM, bool WIDE>
 hipError_t prepare_fixed_dt_t(int bytes_one_wave, int max_lds)
 {
     hipError_t e = hipSuccess;
     for (int w : {1, 2, 4, 8}) {
-        for (bool fw : {false, true}) {
-            int b = bytes_one_wave + fixed_dt_waves_lds(w);
-            b = b < max_lds ? b : max_lds;
-            if (e == hipSuccess)
-                e = hipFuncSetAttribute(fixed_dt_fn<GM, QW>(w, fw),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, b);
-        }
+        int b = bytes_one_wave + fixed_dt_waves_lds(w);
+        b = b < max_lds ? b : max_lds;
+        if (e == hipSuccess)
+            e = hipFuncSetAttribute(fixed_dt_fn<GM, WIDE>(w), hipFuncAttributeMaxDynamicSharedMemorySize, b);
     }
     return e;
 }

@@ -1,9 +1,7 @@
 // mc_fixed_dt.hip — the fixed-dt kernels whose clusters live wholly in LDS (the
-// cluster body, its layout and the kernel templates are in mc_fixed_dt.h), the
-// builds without the quiet window; mc_fixed_dt_window.hip holds those with it.
+// cluster body, its layout and the kernel templates are in mc_fixed_dt.h);
+// mc_fixed_dt_wide.hip holds those of clusters with large grids.
 #include "mc_fixed_dt.h"
-
-#include <algorithm>
 
 namespace mcl {
 
@@ -17,15 +15,14 @@ __global__ void reset_tickets_kernel(uint32_t* tickets, int n)
 
 hipError_t prepare_fixed_dt(int lds_bytes, int max_lds)
 {
-    hipError_t e = prepare_fixed_dt_t<false, false>(lds_bytes, max_lds);
-    if (e == hipSuccess) e = prepare_fixed_dt_window(lds_bytes, max_lds);
-    return e;
+    const hipError_t e = prepare_fixed_dt_t<false, false>(lds_bytes, max_lds);
+    return e == hipSuccess ? prepare_fixed_dt_wide(lds_bytes, max_lds) : e;
 }
 
 hipError_t launch_fixed_dt(const LaunchArgs& a, int grid, int lds_bytes, int waves,
                            hipStream_t stream)
 {
-    if (a.quiet_window != 0) return launch_fixed_dt_window(a, grid, lds_bytes, waves, stream);
+    if (a.wide != 0) return launch_fixed_dt_wide(a, grid, lds_bytes, waves, stream);
     return launch_fixed_dt_t<false, false>(a, grid, (unsigned)(lds_bytes + fixed_dt_waves_lds(waves)),
                                            waves, stream);
 }
@@ -37,14 +34,11 @@ hipError_t launch_reset_tickets(uint32_t* tickets, int n, hipStream_t stream)
     return hipGetLastError();
 }
 
-hipError_t fixed_dt_occupancy(int lds_bytes, int waves, int* blocks_per_cu)
+hipError_t fixed_dt_occupancy(int lds_bytes, int waves, bool wide, int* blocks_per_cu)
 {
-    int b0 = 0, b1 = 0;
-    hipError_t e = fixed_dt_occupancy_t<false, false>((size_t)(lds_bytes + fixed_dt_waves_lds(waves)),
-                                                      waves, &b0);
-    if (e == hipSuccess) e = fixed_dt_window_occupancy(lds_bytes, waves, &b1);
-    *blocks_per_cu = b0 < b1 ? b0 : b1;
-    return e;
+    if (wide) return fixed_dt_wide_occupancy(lds_bytes, waves, blocks_per_cu);
+    return fixed_dt_occupancy_t<false, false>((size_t)(lds_bytes + fixed_dt_waves_lds(waves)), waves,
+                                       blocks_per_cu);
 }
 
 }  // namespace mcl

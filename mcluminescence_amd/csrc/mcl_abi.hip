@@ -142,8 +142,7 @@ struct Plan {
     int32_t h_cap = 0, e_cap = 0, g_cap = 0, lds = 0;
     int32_t max_e = 0, max_h = 0;
     int32_t waves = 1;            // wavefronts per cluster of the one-workgroup-per-cluster launch
-    int32_t fixed_thr = 0;        // some run keeps its fire thresholds (keeps_thresholds)
-    int32_t window = 0;           // some run takes the quiet window (uses_window)
+    int32_t wide = 0;             // the kernels of clusters with large grids
     uint32_t flags = 0;
     // clusters beyond one workgroup's LDS (global-memory form): the plain launch is
     // persistent, ggrid workgroups with a scratch slice of gstride bytes each
@@ -162,8 +161,7 @@ struct Plan {
         int32_t h_cap = 0, e_cap = 0, g_cap = 0, lds = 0, grid = 0;
         int32_t max_e = 0, max_h = 0;
         int32_t waves = 1;
-        int32_t fixed_thr = 0;          // some cluster's run keeps its fire thresholds
-        int32_t window = 0;             // some cluster's run takes the quiet window
+        int32_t wide = 0;
         bool global = false;            // global-memory form: scratch at goff, gstride a slice
         int32_t e_lds = 0;
         int64_t gstride = 0;
@@ -182,6 +180,13 @@ struct Plan {
 };
 
 constexpr double kPi = 0x1.921fb54442d18p+1;
+
+// Does a launch whose largest hole grid has this many cells take the kernels of
+// large grids?
+int32_t wide_grids(int max_cells)
+{
+    return max_cells >= mcl::kWideGrid * mcl::kWideGrid * mcl::kWideGrid ? 1 : 0;
+}
 
 void geometry(const mcl_run_params& p, mcl_geometry& g)
 {
@@ -244,23 +249,6 @@ int validate_run(Ctx* c, const mcl_run_params& p, int r, int32_t n_bins, mcl_geo
         return fail(c, MCL_ERANGE, "run %d: %d electrons / %d holes exceed 16-bit indices", r,
                     g.n_e0, g.n_h);
     return MCL_OK;
-}
-
-// Runs whose clusters keep their fire thresholds in the w slots (isothermal, one
-// localisation channel): a launch with any of them takes the kernels built with
-// that path.
-bool keeps_thresholds(const Ctx* c, const mcl::RunDesc& d)
-{
-    return c->fixed_thresholds != 0.0 && d.T_rate == 0.0 && !d.two_channel;
-}
-
-// Runs on a temperature ramp: a launch with one of them takes the kernels with the
-// quiet window (long stretches in which no electron fires, before and after the
-// glow peak; an isothermal decay fires in nearly every step until its last few
-// electrons, which the look-ahead covers).
-bool uses_window(const Ctx* c, const mcl::RunDesc& d)
-{
-    return c->quiet_window != 0.0 && d.T_rate != 0.0;
 }
 
 mcl::RunDesc make_desc(const mcl_run_params& p, const mcl_geometry& g, int run_id,
@@ -336,7 +324,7 @@ void plan_free(Plan* p, bool idle)
 // that cover their rows (the knob included), above 32768 none do (MCL_ERANGE).
 // per_cu: that kernel's workgroups per CU (global: of the global-memory kernels).
 int choose_waves(Ctx* c, int lds, int e_cap, int64_t count, int max_waves, int* waves,
-                 int* per_cu, bool global)
+                 int* per_cu, bool global, bool wide)
 {
     const int rows = e_cap / 64;                            // 64-slot rows
     int need = 1;
@@ -354,7 +342,7 @@ int choose_waves(Ctx* c, int lds, int e_cap, int64_t count, int max_waves, int* 
         if (lds + mcl::fixed_dt_waves_lds(w) > c->max_lds) continue;
         int pc = 0;
         const hipError_t e = global ? mcl::fixed_dt_global_occupancy(lds, w, &pc)
-                                    : mcl::fixed_dt_occupancy(lds, w, &pc);
+                                    : mcl::fixed_dt_occupancy(lds, w, wide, &pc);
         if (e != hipSuccess) return fail(c, MCL_EDEVICE, "occupancy query: %s", hipGetErrorString(e));
         const int64_t res = (int64_t)w * std::min<int64_t>(count, (int64_t)std::max(pc, 1) * c->n_cu);
         if (res > best_res) {
@@ -372,10 +360,9 @@ int choose_waves(Ctx* c, int lds, int e_cap, int64_t count, int max_waves, int* 
 }
 
 // Where the clusters of given capacities live: wholly in LDS when
-// fixed_dt_lds_bytes and the largest exchange block fit a workgroup (and the
-// global_memory knob is off); otherwise
-// the global-memory form, with the electron arrays in LDS when they fit beside
-// the largest exchange block.
+// cluster_lds_bytes and the largest exchange block fit a workgroup (and the
+// global_memory knob is off); otherwise the global-memory form, with the electron
+// arrays (e_bytes) in LDS when they fit beside the largest exchange block.
 // lds: the launch's dynamic LDS before the per-wave extra.
 struct Layout {
     bool global = false;
@@ -384,15 +371,15 @@ struct Layout {
     int64_t gstride = 0;
 };
 
-Layout layout_for(const Ctx* c, int h_cap, int e_cap, int g_cap)
+Layout layout_for(const Ctx* c, int h_cap, int g_cap, int e_bytes)
 {
     Layout L;
-    L.lds = mcl::fixed_dt_lds_bytes(h_cap, e_cap, g_cap);
+    L.lds = mcl::cluster_lds_bytes(h_cap, g_cap, e_bytes);
     if (L.lds + mcl::fixed_dt_waves_lds(8) <= c->max_lds && c->global_memory == 0.0) return L;
     L.global = true;
-    L.e_lds = mcl::fixed_dt_global_lds(e_cap, true) + mcl::fixed_dt_waves_lds(8) <= c->max_lds;
-    L.lds = mcl::fixed_dt_global_lds(e_cap, L.e_lds != 0);
-    L.gstride = mcl::fixed_dt_global_stride(h_cap, e_cap, g_cap, L.e_lds != 0);
+    L.e_lds = mcl::cluster_global_lds(e_bytes, true) + mcl::fixed_dt_waves_lds(8) <= c->max_lds;
+    L.lds = mcl::cluster_global_lds(e_bytes, L.e_lds != 0);
+    L.gstride = mcl::cluster_global_stride(h_cap, g_cap, e_bytes, L.e_lds != 0);
     return L;
 }
 
@@ -439,21 +426,21 @@ int build_classes(Ctx* c, Plan* p, const mcl_run_params* runs, int32_t n_runs,
             cl.max_e = std::max(cl.max_e, d.n_e0);
             cl.max_h = std::max(cl.max_h, d.n_h);
             max_cells = std::max(max_cells, d.grid * d.grid * d.grid);
-            if (keeps_thresholds(c, d)) cl.fixed_thr = 1;
-            if (uses_window(c, d)) cl.window = 1;
         }
         cl.h_cap = ((cl.max_h + 3) / 4) * 4 + 4;
         cl.e_cap = std::max(64, ((cl.max_e + 63) / 64) * 64);
         cl.g_cap = ((max_cells + 1 + 3) / 4) * 4;
-        const Layout L = layout_for(c, cl.h_cap, cl.e_cap, cl.g_cap);
+        const Layout L = layout_for(c, cl.h_cap, cl.g_cap, mcl::fixed_dt_electron_bytes(cl.e_cap));
         cl.lds = L.lds;
         cl.global = L.global;
         cl.e_lds = L.e_lds;
         cl.gstride = L.gstride;
+        cl.wide = wide_grids(max_cells);
         // (the kernels' dynamic-LDS limit was raised to the plan's largest class)
         int per_cu = 0;
         const int st = choose_waves(c, cl.lds, cl.e_cap, cl.count,
-                                    p->classes.size() > 1 ? 4 : 8, &cl.waves, &per_cu, cl.global);
+                                    p->classes.size() > 1 ? 4 : 8, &cl.waves, &per_cu, cl.global,
+                                    cl.wide != 0);
         if (st) return st;
         const double frac = c->persist_frac;
         int grid = (int)std::max(1.0, std::floor((double)std::max(per_cu, 1) * c->n_cu * frac));
@@ -517,7 +504,7 @@ int make_plan(Ctx* c, const mcl_run_params* runs, int32_t n_runs, const int32_t*
     const int h_cap = ((max_h + 3) / 4) * 4 + 4;
     const int e_cap = std::max(64, ((max_e + 63) / 64) * 64);
     const int g_cap = ((max_cells + 1 + 3) / 4) * 4;
-    const Layout L = layout_for(c, h_cap, e_cap, g_cap);
+    const Layout L = layout_for(c, h_cap, g_cap, mcl::fixed_dt_electron_bytes(e_cap));
     const int lds = L.lds;
     std::vector<int32_t> crun((size_t)total), csim((size_t)total);
     int64_t k = 0;
@@ -541,13 +528,10 @@ int make_plan(Ctx* c, const mcl_run_params* runs, int32_t n_runs, const int32_t*
     p->max_e = max_e;
     p->max_h = max_h;
     p->flags = flags;
-    for (int r = 0; r < n_runs; ++r)
-        if (runs[r].sims > 0 && keeps_thresholds(c, desc[(size_t)r])) p->fixed_thr = 1;
-    for (int r = 0; r < n_runs; ++r)
-        if (runs[r].sims > 0 && uses_window(c, desc[(size_t)r])) p->window = 1;
     p->global = L.global;
     p->e_lds = L.e_lds;
     p->gstride = L.gstride;
+    p->wide = wide_grids(max_cells);
     hipError_t e = mcl::pool_alloc(c, (void**)&p->d_runs, sizeof(mcl::RunDesc) * (size_t)n_runs);
     if (e == hipSuccess) e = mcl::pool_alloc(c, (void**)&p->d_crun, sizeof(int32_t) * (size_t)total);
     if (e == hipSuccess) e = mcl::pool_alloc(c, (void**)&p->d_csim, sizeof(int32_t) * (size_t)total);
@@ -567,7 +551,8 @@ int make_plan(Ctx* c, const mcl_run_params* runs, int32_t n_runs, const int32_t*
     if (e == hipSuccess) e = hipEventCreate(&p->ev1);
     // (LDS limits: the plan's largest need, at most a workgroup's; classes need less)
     if (e == hipSuccess)
-        e = mcl::prepare_fixed_dt(mcl::fixed_dt_lds_bytes(h_cap, e_cap, g_cap), c->max_lds);
+        e = mcl::prepare_fixed_dt(
+            mcl::cluster_lds_bytes(h_cap, g_cap, mcl::fixed_dt_electron_bytes(e_cap)), c->max_lds);
     if (e == hipSuccess && L.global) e = mcl::prepare_fixed_dt_global(c->max_lds);
     if (e != hipSuccess) {
         plan_free(p, false);
@@ -576,7 +561,8 @@ int make_plan(Ctx* c, const mcl_run_params* runs, int32_t n_runs, const int32_t*
     }
     int per_cu = 0;
     {
-        const int st = choose_waves(c, lds, e_cap, total, 8, &p->waves, &per_cu, L.global);
+        const int st = choose_waves(c, lds, e_cap, total, 8, &p->waves, &per_cu, L.global,
+                                    p->wide != 0);
         if (st) {
             plan_free(p, true);
             return st;
@@ -629,10 +615,8 @@ mcl::LaunchArgs launch_args(const Plan* p, uint32_t* counts, uint64_t* live)
     a.e_cap = p->e_cap;
     a.g_cap = p->g_cap;
     a.wave_search_max = (int32_t)p->ctx->wave_search_max;
-    a.lookahead_max = (int32_t)p->ctx->lookahead_max;
-    a.quiet_window = p->window;
+    a.wide = p->wide;
     a.dump.enabled = 0;
-    a.fixed_thr = p->fixed_thr;
     return a;
 }
 
@@ -651,8 +635,7 @@ hipError_t enqueue_persistent(Plan* p, uint32_t* counts, uint64_t* live, hipStre
         a.order = p->d_order + cl.first;
         a.n_order = cl.count;
         a.queue = p->d_tickets + k;
-        a.fixed_thr = cl.fixed_thr;
-        a.quiet_window = cl.window;
+        a.wide = cl.wide;
         a.h_cap = cl.h_cap;
         a.e_cap = cl.e_cap;
         a.g_cap = cl.g_cap;
@@ -1218,7 +1201,7 @@ int mcl_run_event(void* ctx, const mcl_run_params* runs, int32_t n_runs, const d
     const int g_cap = ((max_cells + 1 + 3) / 4) * 4;
     // clusters beyond LDS: holes (and electrons, when they do not fit either) in a
     // scratch slice per resident workgroup, persistent over a ticket
-    const Layout L = layout_for(c, h_cap, e_cap, g_cap);
+    const Layout L = layout_for(c, h_cap, g_cap, mcl::event_electron_bytes(e_cap));
     const int lds = L.lds;
     int ggrid = 0;
     if (L.global) {
@@ -1467,7 +1450,8 @@ int mcl_run_fixed_dt_noalloc(void* ctx, const mcl_run_params* runs, int32_t n_ru
     const int h_cap = ((max_h + 3) / 4) * 4 + 4;
     const int e_cap = std::max(64, ((max_e + 63) / 64) * 64);
     const int g_cap = ((max_cells + 1 + 3) / 4) * 4;
-    const int lds = mcl::fixed_dt_lds_bytes(h_cap, e_cap, g_cap);
+    const int lds =
+        mcl::cluster_lds_bytes(h_cap, g_cap, mcl::fixed_dt_electron_bytes(e_cap));
     if (lds > c->max_lds)
         return fail(c, MCL_ERANGE,
                     "cluster of %d electrons / %d holes needs %d B of LDS; a workgroup has %d B "
@@ -1476,7 +1460,6 @@ int mcl_run_fixed_dt_noalloc(void* ctx, const mcl_run_params* runs, int32_t n_ru
     // descriptors and cluster map through a fixed host staging block, one chunk
     // at a time (each copied and waited for before the block is refilled)
     alignas(64) unsigned char stage[16384];
-    int32_t fixed_thr = 0, window = 0;
     auto upload = [&](size_t dst_off, size_t bytes) -> hipError_t {
         hipError_t r = hipMemcpyAsync(base + dst_off, stage, bytes, hipMemcpyHostToDevice, c->stream);
         if (r == hipSuccess) r = hipStreamSynchronize(c->stream);
@@ -1491,8 +1474,6 @@ int mcl_run_fixed_dt_noalloc(void* ctx, const mcl_run_params* runs, int32_t n_ru
                 mcl_geometry g;
                 geometry(runs[r0 + j], g);
                 d[j] = make_desc(runs[r0 + j], g, r0 + j, c->holes_per_cell);
-                if (runs[r0 + j].sims > 0 && keeps_thresholds(c, d[j])) fixed_thr = 1;
-                if (runs[r0 + j].sims > 0 && uses_window(c, d[j])) window = 1;
             }
             e = upload(sizeof(mcl::RunDesc) * (size_t)r0, sizeof(mcl::RunDesc) * (size_t)k);
         }
@@ -1523,7 +1504,7 @@ int mcl_run_fixed_dt_noalloc(void* ctx, const mcl_run_params* runs, int32_t n_ru
     if (e != hipSuccess)
         return fail(c, MCL_EDEVICE, "noalloc setup: %s", hipGetErrorString(e));
     int waves = 1, per_cu = 0;
-    int st = choose_waves(c, lds, e_cap, total, 8, &waves, &per_cu, false);
+    int st = choose_waves(c, lds, e_cap, total, 8, &waves, &per_cu, false, wide_grids(max_cells) != 0);
     if (st) return st;
     mcl::LaunchArgs a{};
     a.runs = (const mcl::RunDesc*)base;
@@ -1544,10 +1525,8 @@ int mcl_run_fixed_dt_noalloc(void* ctx, const mcl_run_params* runs, int32_t n_ru
     a.e_cap = e_cap;
     a.g_cap = g_cap;
     a.wave_search_max = (int32_t)c->wave_search_max;
-    a.lookahead_max = (int32_t)c->lookahead_max;
-    a.quiet_window = window;
+    a.wide = wide_grids(max_cells);
     a.dump.enabled = 0;
-    a.fixed_thr = fixed_thr;
     e = hipEventRecord(c->na_ev0, c->stream);
     if (e == hipSuccess) e = mcl::launch_fixed_dt(a, (int)total, lds, waves, c->stream);
     if (e == hipSuccess) e = hipEventRecord(c->na_ev1, c->stream);

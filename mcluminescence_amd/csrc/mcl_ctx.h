@@ -25,15 +25,16 @@ struct Ctx {
     double holes_per_cell = 2.0;   // hole-grid density target (tunable)
     double persist_frac = 1.0;     // persistent workgroups per class / device capacity
     double wave_search_max = 32.0; // queue length searched by the whole wave
-    double lookahead_max = 8.0;    // live electrons up to which quiet steps are skipped
-    double quiet_window = 1.0;     // 1: after a step with no candidate, the rest of its
-                                   // Philox block is tested at once
+    // Accepted and kept for programs and tables that set them; they chose between ways
+    // of skipping quiet steps, which every fixed-dt launch now does by its first-fire
+    // windows.
+    double lookahead_max = 8.0;
+    double quiet_window = 1.0;
+    double fixed_thresholds = 1.0;
     double waves_per_cluster = 0.0; // wavefronts per fixed-dt cluster: 1, 2, 4, 8 or 0 (chosen per launch)
     double mlp_fused = 1.0;        // surrogate inference as one kernel (1) or per layer (0)
     double global_memory = 0.0;    // fixed-dt clusters in the global-memory form: 0 when
                                    // they exceed LDS, 1 always
-    double fixed_thresholds = 1.0; // 1: launches with an isothermal one-channel run take the
-                                   // kernels with the fixed-threshold path; 0: never
     std::string err;
     // timing events of mcl_run_fixed_dt_noalloc, made once by mcl_create
     hipEvent_t na_ev0 = nullptr, na_ev1 = nullptr;

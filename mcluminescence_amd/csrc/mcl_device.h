@@ -78,30 +78,32 @@ __device__ __forceinline__ float em1_core(float r)
     return __builtin_fmaf(r2, p, r);
 }
 
+// (The special cases are selects, not early returns: a divergent return is a branch
+// and a save of the execution mask each, which cost more than the few operations.)
 __device__ __forceinline__ float expm1_own(float x)
 {
-    if (x != x) return x;
-    if (x < -17.5f) return -1.0f;
-    if (x > 88.0f) return __builtin_inff();
     const float kf = __builtin_rintf(x * kFInvLn2);
     float r = __builtin_fmaf(-kf, kFLn2Hi, x);
     r = __builtin_fmaf(-kf, kFLn2Lo, r);
     const float em1 = em1_core(r);
-    if (kf == 0.0f) return em1;
     const float t = pow2i_f((int)kf);
-    return __builtin_fmaf(t, em1, t - 1.0f);
+    float v = __builtin_fmaf(t, em1, t - 1.0f);
+    v = kf == 0.0f ? em1 : v;
+    v = x < -17.5f ? -1.0f : v;
+    v = x > 88.0f ? __builtin_inff() : v;
+    return x != x ? x : v;
 }
 
 __device__ __forceinline__ float exp_own(float x)
 {
-    if (x != x) return x;
-    if (x < -87.0f) return 0.0f;
-    if (x > 88.0f) return __builtin_inff();
     const float kf = __builtin_rintf(x * kFInvLn2);
     float r = __builtin_fmaf(-kf, kFLn2Hi, x);
     r = __builtin_fmaf(-kf, kFLn2Lo, r);
     const float e = 1.0f + em1_core(r);
-    return e * pow2i_f((int)kf);
+    float v = e * pow2i_f((int)kf);
+    v = x < -87.0f ? 0.0f : v;
+    v = x > 88.0f ? __builtin_inff() : v;
+    return x != x ? x : v;
 }
 
 constexpr double kDInvLn2 = 0x1.71547652b82fep+0;
@@ -115,9 +117,6 @@ __device__ __forceinline__ double pow2i_d(int k)  // 2^k, -1022 <= k <= 1023
 
 __device__ __forceinline__ double exp_own(double x)
 {
-    if (x != x) return x;
-    if (x < -708.0) return 0.0;
-    if (x > 709.0) return __builtin_inf();
     const double kd = __builtin_rint(x * kDInvLn2);
     double r = __builtin_fma(-kd, kDLn2Hi, x);
     r = __builtin_fma(-kd, kDLn2Lo, r);
@@ -135,7 +134,10 @@ __device__ __forceinline__ double exp_own(double x)
     p = __builtin_fma(p, r, 0x1p-1);
     p = __builtin_fma(p, r, 0x1p+0);
     const double e = __builtin_fma(p, r, 1.0);
-    return e * pow2i_d((int)kd);
+    double v = e * pow2i_d((int)kd);
+    v = x < -708.0 ? 0.0 : v;
+    v = x > 709.0 ? __builtin_inf() : v;
+    return x != x ? x : v;
 }
 
 // Fire threshold for x = k dt: p = 1 - e^{-x}; an electron with draw u fires
@@ -246,6 +248,31 @@ __device__ __forceinline__ uint32_t wave_min_u32(uint32_t v)
     return a < b ? a : b;
 }
 
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) { return ~wave_min_u32(~v); }
+
+// Bitwise or over the 64 lanes (all active), in every lane, by the same steps.
+__device__ __forceinline__ uint32_t wave_or_u32(uint32_t v)
+{
+    v |= dpp_u32<kDppQuad1032>(v);
+    v |= dpp_u32<kDppQuad2301>(v);
+    v |= dpp_u32<kDppRowHalfMirror>(v);
+    v |= dpp_u32<kDppRowMirror>(v);
+    return (lane_value(v, 0) | lane_value(v, 16)) | (lane_value(v, 32) | lane_value(v, 48));
+}
+
+// Minimum over each 16-lane row (all lanes active), in every lane of the row.
+__device__ __forceinline__ uint32_t row_min_u32(uint32_t v)
+{
+    uint32_t u = dpp_u32<kDppQuad1032>(v);
+    v = u < v ? u : v;
+    u = dpp_u32<kDppQuad2301>(v);
+    v = u < v ? u : v;
+    u = dpp_u32<kDppRowHalfMirror>(v);
+    v = u < v ? u : v;
+    u = dpp_u32<kDppRowMirror>(v);
+    return u < v ? u : v;
+}
+
 // Minimum of a 64-bit key over the 64 lanes (all active): the high words first;
 // the low word of the single lane holding that minimum, or the minimum low word
 // among the tied lanes.
@@ -274,17 +301,6 @@ __device__ __forceinline__ uint64_t row_min_u64(uint64_t v)
     v = u < v ? u : v;
     u = ((uint64_t)dpp_u32<kDppRowMirror>((uint32_t)(v >> 32)) << 32) | dpp_u32<kDppRowMirror>((uint32_t)v);
     return u < v ? u : v;
-}
-
-__device__ __forceinline__ uint64_t wave_or_u64(uint64_t v)
-{
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        const uint32_t lo = (uint32_t)__shfl_xor((int)(uint32_t)v, off);
-        const uint32_t hi = (uint32_t)__shfl_xor((int)(uint32_t)(v >> 32), off);
-        v |= ((uint64_t)hi << 32) | lo;
-    }
-    return v;
 }
 
 }  // namespace mcl

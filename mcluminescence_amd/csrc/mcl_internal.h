@@ -64,9 +64,7 @@ struct LaunchArgs {
     int32_t e_cap;          // LDS electron capacity (multiple of 64, >= n_e0)
     int32_t g_cap;          // LDS cell-start capacity (>= G^3 + 1, multiple of 4)
     int32_t wave_search_max;  // queues up to this long are searched one electron per wave (<= 64)
-    int32_t lookahead_max;    // with at most this many live electrons, quiet steps are skipped
-    int32_t quiet_window;     // 1: the kernels built with the quiet window (after quiet
-                              // steps, the rest of a Philox block tested at once)
+    int32_t wide;             // 1: the kernels of clusters with large grids (wide_grid)
     StateDump dump;
     // global-memory form (clusters beyond one workgroup's LDS): workgroup b keeps its
     // cluster's holes and cell starts (and, unless e_lds, its electron arrays) in
@@ -74,10 +72,6 @@ struct LaunchArgs {
     unsigned char* gscratch;
     int64_t gstride;
     int32_t e_lds;            // electron arrays in LDS after the exchange slots
-    // 1: some run of the launch is isothermal with one localisation channel, and
-    // the kernels built with the fixed-threshold path run it; 0: the kernels
-    // without that path (same counts, shorter code for ramped or two-channel runs)
-    int32_t fixed_thr;
 };
 
 // Event-mode launch: one cluster per workgroup, one event per step.
@@ -129,20 +123,29 @@ int lab_lds_bytes(int h_cap, int e_cap);
 
 constexpr int kWaveHost = 64;   // wavefront width of gfx950
 
-// LDS bytes the fixed-dt kernel needs for the given capacities.
-inline int fixed_dt_lds_bytes(int h_cap, int e_cap, int g_cap)
+// Bytes of a cluster's electron arrays (e_cap a multiple of 64): the fixed-dt
+// kernel's est, ew, nf and lst (11 B an electron, and 64 entries of lst more) and rowm
+// (8 B a row of 64), and the event kernel's four words an electron.
+__host__ __device__ constexpr int fixed_dt_electron_bytes(int e_cap)
 {
-    return 16 * h_cap + 4 * g_cap + 16 * e_cap;
+    return 11 * e_cap + e_cap / 8 + 128;
+}
+constexpr int event_electron_bytes(int e_cap) { return 16 * e_cap; }
+
+// LDS bytes of a cluster wholly in LDS, with e_bytes of electron arrays.
+inline int cluster_lds_bytes(int h_cap, int g_cap, int e_bytes)
+{
+    return 16 * h_cap + 4 * g_cap + e_bytes;
 }
 
 // Global-memory form: scratch bytes per workgroup (a multiple of 256), and the
 // LDS of the cluster arrays kept there (the per-wave extra is added at launch).
-inline int64_t fixed_dt_global_stride(int h_cap, int e_cap, int g_cap, bool e_lds)
+inline int64_t cluster_global_stride(int h_cap, int g_cap, int e_bytes, bool e_lds)
 {
-    const int64_t b = 16 * (int64_t)h_cap + 4 * (int64_t)g_cap + (e_lds ? 0 : 16 * (int64_t)e_cap);
+    const int64_t b = 16 * (int64_t)h_cap + 4 * (int64_t)g_cap + (e_lds ? 0 : (int64_t)e_bytes);
     return (b + 255) / 256 * 256;
 }
-inline int fixed_dt_global_lds(int e_cap, bool e_lds) { return e_lds ? 16 * e_cap : 0; }
+inline int cluster_global_lds(int e_bytes, bool e_lds) { return e_lds ? e_bytes : 0; }
 
 // Cells per axis of a cluster's hole grid: about holes_per_cell holes a cell.
 inline int grid_dim(int n_h, double holes_per_cell)
@@ -153,37 +156,39 @@ inline int grid_dim(int n_h, double holes_per_cell)
     return G;
 }
 
-// LDS beyond fixed_dt_lds_bytes for a workgroup of `waves` wavefronts: the
-// per-wave exchange slots (2 x waves words) and the persistent ticket.
-constexpr int fixed_dt_waves_lds(int waves)
+// Grids of at least this many cells per axis (1,458 holes at two a cell) take the
+// kernels that search wider blocks before they scan every hole: the scan costs
+// n_h / 64 dependent round trips (216 in scratch memory for 13,800 holes), a wider
+// block a few.  Below, the scan is the shorter of the two (863 holes: 14 trips) and the
+// blocks' code costs registers (the 4096 x 400 decay 1.17 against 1.21 ms with it).
+constexpr int kWideGrid = 9;
+
+// LDS beyond cluster_lds_bytes for a workgroup of `waves` wavefronts: the
+// per-wave exchange slots (2 x waves words), the persistent ticket and the four
+// words wave 0 publishes.
+__host__ __device__ constexpr int fixed_dt_waves_lds(int waves)
 {
-    return waves > 1 ? ((4 * (2 * waves + 1) + 15) / 16) * 16 : 0;
+    return waves > 1 ? ((4 * (2 * waves + 5) + 15) / 16) * 16 : 0;
 }
 
-// waves = wavefronts per cluster (1, 2, 4 or 8); lds_bytes = fixed_dt_lds_bytes of the
+// waves = wavefronts per cluster (1, 2, 4 or 8); lds_bytes = cluster_lds_bytes of the
 // launch (the per-wave extra is added here)
 hipError_t launch_fixed_dt(const LaunchArgs& a, int grid, int lds_bytes, int waves,
                            hipStream_t stream);
 hipError_t launch_reset_tickets(uint32_t* tickets, int n, hipStream_t stream);
 hipError_t prepare_fixed_dt(int lds_bytes, int max_lds);
-hipError_t fixed_dt_occupancy(int lds_bytes, int waves, int* blocks_per_cu);
+hipError_t fixed_dt_occupancy(int lds_bytes, int waves, bool wide, int* blocks_per_cu);
+// The builds for large grids (mc_fixed_dt_wide.hip); the functions above call them.
+hipError_t prepare_fixed_dt_wide(int lds_bytes, int max_lds);
+hipError_t launch_fixed_dt_wide(const LaunchArgs& a, int grid, int lds_bytes, int waves,
+                                hipStream_t stream);
+hipError_t fixed_dt_wide_occupancy(int lds_bytes, int waves, int* blocks_per_cu);
 // The global-memory form: persistent launches only (a.queue set, grid at most the
-// slices of a.gscratch); lds_bytes = fixed_dt_global_lds.
+// slices of a.gscratch); lds_bytes = cluster_global_lds.
 hipError_t launch_fixed_dt_global(const LaunchArgs& a, int grid, int lds_bytes, int waves,
                                   hipStream_t stream);
 hipError_t prepare_fixed_dt_global(int max_lds);
 hipError_t fixed_dt_global_occupancy(int lds_bytes, int waves, int* blocks_per_cu);
-// The builds with the quiet window (mc_fixed_dt_window.hip,
-// mc_fixed_dt_global_window.hip); the functions above call them when
-// a.quiet_window is set and take both builds into the limits and occupancy.
-hipError_t prepare_fixed_dt_window(int lds_bytes, int max_lds);
-hipError_t launch_fixed_dt_window(const LaunchArgs& a, int grid, int lds_bytes, int waves,
-                                  hipStream_t stream);
-hipError_t fixed_dt_window_occupancy(int lds_bytes, int waves, int* blocks_per_cu);
-hipError_t prepare_fixed_dt_global_window(int max_lds);
-hipError_t launch_fixed_dt_global_window(const LaunchArgs& a, int grid, int lds_bytes, int waves,
-                                         hipStream_t stream);
-hipError_t fixed_dt_global_window_occupancy(int lds_bytes, int waves, int* blocks_per_cu);
 hipError_t launch_event(const EventArgs& a, int lds_bytes, hipStream_t stream);
 // The event kernel's global-memory form: grid workgroups over a.queue's ticket.
 hipError_t launch_event_global(const EventArgs& a, int grid, int lds_bytes, hipStream_t stream);
