@@ -19,7 +19,7 @@ ROOT = PKG.parent
 OUT = PKG / "libmcl.so"
 
 SOURCES = ["mc_fixed_dt.hip", "mc_fixed_dt_wide.hip", "mc_fixed_dt_global.hip", "mc_event.hip",
-           "mc_lab.hip", "glow.hip", "curves.hip", "mcl_abi.hip", "mlp.hip", "mlp_fused.hip", "mlp_abi.hip", "de.hip"]
+           "mc_lab.hip", "glow.hip", "curves.hip", "mcl_abi.hip", "mlp.hip", "mlp_fused.hip", "mlp_train.hip", "mlp_abi.hip", "de.hip"]
 
 # -ffp-contract=off: every fused multiply-add in a decision path is an explicit
 # __builtin_fma, so the CPU replay harness can reproduce each rounding.

@@ -58,18 +58,6 @@ __device__ __forceinline__ uint32_t below(uint32_t w, uint32_t n)
     return (uint32_t)(((uint64_t)w * n) >> 32);
 }
 
-// Workgroup barrier that orders LDS only: the wave's global loads stay in flight
-// across it (a full barrier waits for every outstanding load, since the vector
-// memory counter counts loads and stores alike).  Every exchange between the
-// waves of these kernels goes through LDS; the global data they read (population,
-// keys, weights) does not change during a generation.
-__device__ __forceinline__ void lds_barrier()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 __global__ __launch_bounds__(256) void de_init_kernel(DeArgs a)
 {
     const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);

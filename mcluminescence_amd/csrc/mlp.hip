@@ -267,14 +267,6 @@ __global__ __launch_bounds__(kThreads) void finish_loss_kernel(const float* part
     if (threadIdx.x == 0) *loss = red[0] * scale;
 }
 
-__device__ __forceinline__ void adamw(float& w, float& m, float& v, float gr, const OptArgs& a)
-{
-    w = w * (1.0f - a.lr * a.wd);
-    m = a.beta1 * m + (1.0f - a.beta1) * gr;
-    v = a.beta2 * v + (1.0f - a.beta2) * (gr * gr);
-    w = w - a.step_size * (m / (sqrtf(v) / a.sqrt_bc2 + a.eps));
-}
-
 // One workgroup per 32x32 weight tile (W and W^T written through an LDS
 // transpose), then one per four biases (one wave each).
 __global__ __launch_bounds__(kThreads) void optimizer_kernel(OptArgs a)
@@ -316,7 +308,7 @@ __global__ __launch_bounds__(kThreads) void optimizer_kernel(OptArgs a)
             float* wp = &w.x; float* mp = &m.x; float* vp = &v.x;
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                if (k + i < L.k_in) adamw(wp[i], mp[i], vp[i], gv[i], a);
+                if (k + i < L.k_in) adamw(wp[i], mp[i], vp[i], gv[i], a.hp);
             *reinterpret_cast<float4*>(L.w + o) = w;
             *reinterpret_cast<float4*>(L.m + o) = m;
             *reinterpret_cast<float4*>(L.v + o) = v;
@@ -325,6 +317,7 @@ __global__ __launch_bounds__(kThreads) void optimizer_kernel(OptArgs a)
         bf16x4 wb;
         wb[0] = (bf16)w.x; wb[1] = (bf16)w.y; wb[2] = (bf16)w.z; wb[3] = (bf16)w.w;
         *reinterpret_cast<bf16x4*>(L.wb + o) = wb;
+        if (L.wf) *reinterpret_cast<bf16x4*>(L.wf + fragment_offset(n, k, L.kp)) = wb;
 #pragma unroll
         for (int i = 0; i < 4; ++i) tile[r][c4 + i] = wb[i];
         __syncthreads();
@@ -333,7 +326,9 @@ __global__ __launch_bounds__(kThreads) void optimizer_kernel(OptArgs a)
         bf16x4 tv;
 #pragma unroll
         for (int i = 0; i < 4; ++i) tv[i] = tile[n4 + i][kr];
-        *reinterpret_cast<bf16x4*>(L.wt + (int64_t)(tk0 + kr) * L.out + tn0 + n4) = tv;
+        if (L.wtf)
+            *reinterpret_cast<bf16x4*>(L.wtf + fragment_offset(tk0 + kr, tn0 + n4, L.out)) = tv;
+        if (L.wt) *reinterpret_cast<bf16x4*>(L.wt + (int64_t)(tk0 + kr) * L.out + tn0 + n4) = tv;
         return;
     }
     if (a.mode == kOptRefresh) return;
@@ -352,7 +347,7 @@ __global__ __launch_bounds__(kThreads) void optimizer_kernel(OptArgs a)
         a.flat[L.flat_b + n] = s;
         return;
     }
-    adamw(L.bw[n], L.bm[n], L.bv[n], s, a);
+    adamw(L.bw[n], L.bm[n], L.bv[n], s, a.hp);
 }
 
 template <int BM, int BN, int EPI>

@@ -45,13 +45,16 @@ struct Mlp {
     float* loss_tmp = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     bool timed = false;
-    // the fused inference kernel's network: weights in fragment order (repacked
-    // after any change of the weights), biases, LDS bytes; usable iff fused_ok
+    // the fused inference kernel's network: weights in fragment order, biases, LDS
+    // bytes; usable iff fused_ok
     M::DeNet fnet{};
-    bf16* wf = nullptr;
-    bool wf_stale = true;
+    bf16* wf = nullptr;                   // kept current by every change of the weights
     bool fused_ok = false;
     int fused_lds = 0;
+    // training in two kernels (train_fused_ok): W^T of layers >= 1 in fragment order; the
+    // transposed buffers At, dZt, X0t and dYt then hold fragments
+    bool train_fused = false;
+    std::vector<bf16*> wtf;
 
     ~Mlp()
     {
@@ -130,6 +133,8 @@ M::OptArgs opt_args(Mlp* m, int mode, int batch, int* groups)
         const Layer& s = m->L[i];
         M::OptLayer& o = a.L[i];
         o.w = s.w; o.m = s.m; o.v = s.v; o.wb = s.wb; o.wt = s.wt;
+        o.wf = m->fused_ok ? const_cast<bf16*>(m->fnet.L[i].w) : nullptr;
+        o.wtf = m->train_fused ? m->wtf[i] : nullptr;
         o.part = s.part; o.splits = 0;
         o.bw = s.bw; o.bm = s.bm; o.bv = s.bv;
         o.dzt = i + 1 < m->L.size() ? m->dZt[i] : m->dYt;
@@ -189,15 +194,6 @@ int forward(Mlp* m, const float* x, int32_t B, float* y)
 {
     hipStream_t st = m->ctx->stream;
     if (m->fused_ok && m->ctx->mlp_fused != 0.0) {
-        if (m->wf_stale) {
-            int64_t off = 0;
-            for (size_t l = 0; l < m->L.size(); ++l) {
-                const Layer& s = m->L[l];
-                HIP_TRY(m->ctx, M::de_pack(s.wb, s.out, s.kp, m->wf + off, st));
-                off += (int64_t)s.out * s.kp;
-            }
-            m->wf_stale = false;
-        }
         HIP_TRY(m->ctx, M::infer_fused(x, B, m->d.n_in, m->fnet, y, m->d.n_out, m->fused_lds, st));
         return MCL_OK;
     }
@@ -362,6 +358,20 @@ int forward_backward(Mlp* m, const float* x, const float* t, const int32_t* idx,
     return MCL_OK;
 }
 
+M::AdamWArgs adamw_args(const mcl_adamw& hp)
+{
+    const double t = (double)hp.step;
+    M::AdamWArgs a{};
+    a.lr = (float)hp.lr;
+    a.beta1 = (float)hp.beta1;
+    a.beta2 = (float)hp.beta2;
+    a.eps = (float)hp.eps;
+    a.wd = (float)hp.weight_decay;
+    a.step_size = (float)(hp.lr / (1.0 - std::pow(hp.beta1, t)));
+    a.sqrt_bc2 = (float)std::sqrt(1.0 - std::pow(hp.beta2, t));
+    return a;
+}
+
 int run_optimizer(Mlp* m, int mode, int B, const std::vector<int>& splits, float* flat,
                   const mcl_adamw* hp)
 {
@@ -369,17 +379,74 @@ int run_optimizer(Mlp* m, int mode, int B, const std::vector<int>& splits, float
     M::OptArgs a = opt_args(m, mode, B, &groups);
     for (size_t i = 0; i < m->L.size(); ++i) a.L[i].splits = i < splits.size() ? splits[i] : 0;
     a.flat = flat;
-    if (hp) {
-        const double t = (double)hp->step;
-        a.lr = (float)hp->lr;
-        a.beta1 = (float)hp->beta1;
-        a.beta2 = (float)hp->beta2;
-        a.eps = (float)hp->eps;
-        a.wd = (float)hp->weight_decay;
-        a.step_size = (float)(hp->lr / (1.0 - std::pow(hp->beta1, t)));
-        a.sqrt_bc2 = (float)std::sqrt(1.0 - std::pow(hp->beta2, t));
-    }
+    if (hp) a.hp = adamw_args(*hp);
     HIP_TRY(m->ctx, M::optimizer(a, groups, m->ctx->stream));
+    return MCL_OK;
+}
+
+// The gradient of batch B (mode kOptExportGrad: to flat, or only the loss without it)
+// or a training step (kOptAdamW): two kernels where the network's shape allows, else
+// layer by layer.
+int gradient(Mlp* m, const float* x, const float* t, const int32_t* idx, int32_t B, int mode,
+             float* flat, float* loss, const mcl_adamw* hp)
+{
+    if (!m->train_fused) {
+        std::vector<int> splits;
+        TRY(forward_backward(m, x, t, idx, B, loss, splits));
+        if (mode == M::kOptAdamW || flat) TRY(run_optimizer(m, mode, B, splits, flat, hp));
+        return MCL_OK;
+    }
+    hipStream_t st = m->ctx->stream;
+    const int nl = (int)m->L.size(), nh = nl - 1, n_out = m->d.n_out;
+    M::TrainArgs a{};
+    a.x = x;
+    a.t = t;
+    a.idx = idx;
+    a.n_in = m->d.n_in;
+    a.B = B;
+    a.grad_scale = (float)(2.0 / ((double)B * n_out));
+    a.net = m->fnet;
+    a.xf = m->X0t;
+    for (int l = 0; l < nl; ++l) {
+        a.wtf[l] = m->wtf[l];
+        a.af[l] = l < nh ? m->At[l] : nullptr;
+        a.dzf[l] = l < nh ? m->dZt[l] : m->dYt;
+    }
+    a.loss_part = m->loss_part;
+    HIP_TRY(m->ctx, M::train_chain(a, n_out, st));
+    const int n_part = B / M::kTrainRows;
+    const float scale = (float)(1.0 / ((double)B * n_out));
+    if (mode == M::kOptExportGrad && !flat) {
+        if (loss) HIP_TRY(m->ctx, M::finish_loss(m->loss_part, n_part, scale, loss, st));
+        return MCL_OK;
+    }
+    M::UpdateArgs u{};
+    u.n_layers = nl;
+    u.mode = mode;
+    u.S = B / 16;
+    for (int l = 0; l < nl; ++l) {
+        const Layer& s = m->L[l];
+        M::UpdateLayer& o = u.L[l];
+        o.dzf = a.dzf[l];
+        o.xf = l == 0 ? a.xf : a.af[l - 1];
+        o.w = s.w; o.m = s.m; o.v = s.v;
+        o.wb = s.wb; o.wf = const_cast<bf16*>(m->fnet.L[l].w); o.wtf = m->wtf[l];
+        o.bw = s.bw; o.bm = s.bm; o.bv = s.bv;
+        o.out = s.out; o.kp = s.kp; o.k_in = s.in;
+        o.blk0 = u.n_blocks;
+        o.flat_w = s.flat_w; o.flat_b = s.flat_b;
+        u.n_blocks += (s.out / 64) * (s.kp / 64) + s.out / 32;
+    }
+    ++u.n_blocks;                          // the loss
+    u.parts = 1;
+    while (u.parts < kMaxSplits && B % (128 * u.parts) == 0) u.parts *= 2;
+    u.flat = flat;
+    if (hp) u.hp = adamw_args(*hp);
+    u.loss_part = m->loss_part;
+    u.n_part = n_part;
+    u.loss_scale = scale;
+    u.loss = loss;
+    HIP_TRY(m->ctx, M::train_update(u, st));
     return MCL_OK;
 }
 
@@ -425,12 +492,32 @@ int mcl_mlp_create(void* ctxp, const mcl_mlp_desc* desc, void** out)
     const int64_t B = d.max_batch;
     int st = MCL_OK;
     auto run = [&]() -> int {
+        // which fused kernels take the network (their views need the biases below)
+        int64_t widest = 0;
+        for (size_t l = 0; l < m->L.size(); ++l) {
+            const Layer& s = m->L[l];
+            m->fnet.L[l] = M::DeLayer{nullptr, nullptr, s.out, s.kp};
+            widest = std::max<int64_t>(widest, s.kp);
+            if (l + 1 < m->L.size()) widest = std::max<int64_t>(widest, s.out);
+        }
+        m->fnet.n_layers = (int)m->L.size();
+        m->fnet.lda = (int)widest + 8;
+        m->fused_lds = M::infer_fused_lds(m->fnet);
+        m->fused_ok = M::infer_fused_ok(m->fnet) && m->fused_lds <= c->max_lds &&
+                      M::infer_fused_prepare(m->fused_lds) == hipSuccess;
+        m->train_fused = m->fused_ok && M::train_fused_ok(m->fnet, c->max_lds) &&
+                         M::train_fused_prepare() == hipSuccess;
+        (void)hipGetLastError();
         for (Layer& s : m->L) {
             const int64_t nw = (int64_t)s.out * s.kp;
             TRY(dalloc(m, &s.w, nw)); TRY(dalloc(m, &s.m, nw)); TRY(dalloc(m, &s.v, nw));
             TRY(dalloc(m, &s.bw, s.out)); TRY(dalloc(m, &s.bm, s.out)); TRY(dalloc(m, &s.bv, s.out));
-            TRY(dalloc(m, &s.wb, nw)); TRY(dalloc(m, &s.wt, nw));
-            TRY(dalloc(m, &s.part, kMaxSplits * nw));
+            TRY(dalloc(m, &s.wb, nw));
+            if (!m->train_fused) {
+                TRY(dalloc(m, &s.wt, nw));
+                TRY(dalloc(m, &s.part, kMaxSplits * nw));
+                HIP_TRY(c, hipMemset(s.wt, 0, nw * sizeof(bf16)));
+            }
             HIP_TRY(c, hipMemset(s.w, 0, nw * sizeof(float)));
             HIP_TRY(c, hipMemset(s.m, 0, nw * sizeof(float)));
             HIP_TRY(c, hipMemset(s.v, 0, nw * sizeof(float)));
@@ -438,15 +525,18 @@ int mcl_mlp_create(void* ctxp, const mcl_mlp_desc* desc, void** out)
             HIP_TRY(c, hipMemset(s.bm, 0, s.out * sizeof(float)));
             HIP_TRY(c, hipMemset(s.bv, 0, s.out * sizeof(float)));
             HIP_TRY(c, hipMemset(s.wb, 0, nw * sizeof(bf16)));
-            HIP_TRY(c, hipMemset(s.wt, 0, nw * sizeof(bf16)));
         }
+        for (size_t l = 0; l < m->L.size(); ++l) m->fnet.L[l].b = m->L[l].bw;
         const int H = d.n_hidden;
         TRY(dalloc(m, &m->X0, B * 64));
         TRY(dalloc(m, &m->X0t, B * 64));
         for (int l = 0; l < d.n_hidden_layers; ++l) {
-            bf16 *z, *a, *at, *dz, *dzt;
-            TRY(dalloc(m, &z, B * H)); TRY(dalloc(m, &a, B * H)); TRY(dalloc(m, &at, B * H));
-            TRY(dalloc(m, &dz, B * H)); TRY(dalloc(m, &dzt, B * H));
+            bf16 *z = nullptr, *a = nullptr, *at, *dz = nullptr, *dzt;
+            TRY(dalloc(m, &at, B * H)); TRY(dalloc(m, &dzt, B * H));
+            // (the two-kernel step keeps z and row-major errors on the chip; inference
+            // layer by layer takes two activation buffers)
+            if (!m->train_fused) { TRY(dalloc(m, &z, B * H)); TRY(dalloc(m, &dz, B * H)); }
+            if (!m->train_fused || l < 2) TRY(dalloc(m, &a, B * H));
             m->Z.push_back(z); m->A.push_back(a); m->At.push_back(at);
             m->dZ.push_back(dz); m->dZt.push_back(dzt);
         }
@@ -455,33 +545,27 @@ int mcl_mlp_create(void* ctxp, const mcl_mlp_desc* desc, void** out)
             TRY(dalloc(m, &a2, B * H));
             m->A.push_back(a2);
         }
-        TRY(dalloc(m, &m->dY, B * d.n_out));
+        if (!m->train_fused) TRY(dalloc(m, &m->dY, B * d.n_out));
         TRY(dalloc(m, &m->dYt, B * d.n_out));
+        // (n_out >= 128: at least the chain's B / 32 partials too)
         TRY(dalloc(m, &m->loss_part, (B / 64) * (d.n_out / 64)));
         TRY(dalloc(m, &m->loss_tmp, 1));
         HIP_TRY(c, hipEventCreate(&m->ev0));
         HIP_TRY(c, hipEventCreate(&m->ev1));
-        // the fused inference kernel's view of the network
-        int64_t nwf = 0, widest = 0;
-        for (size_t l = 0; l < m->L.size(); ++l) {
-            const Layer& s = m->L[l];
-            m->fnet.L[l] = M::DeLayer{nullptr, s.bw, s.out, s.kp};
-            nwf += (int64_t)s.out * s.kp;
-            widest = std::max<int64_t>(widest, s.kp);
-            if (l + 1 < m->L.size()) widest = std::max<int64_t>(widest, s.out);
-        }
-        m->fnet.n_layers = (int)m->L.size();
-        m->fnet.lda = (int)widest + 8;
-        m->fused_lds = M::infer_fused_lds(m->fnet);
-        if (M::infer_fused_ok(m->fnet) && m->fused_lds <= c->max_lds &&
-            M::infer_fused_prepare(m->fused_lds) == hipSuccess) {
+        // the fused kernels' copies of the weights
+        if (m->fused_ok) {
+            int64_t nwf = 0;
+            for (const Layer& s : m->L) nwf += (int64_t)s.out * s.kp;
             TRY(dalloc(m, &m->wf, nwf));
             int64_t off = 0;
             for (size_t l = 0; l < m->L.size(); ++l) {
+                const Layer& s = m->L[l];
                 m->fnet.L[l].w = m->wf + off;
-                off += (int64_t)m->L[l].out * m->L[l].kp;
+                off += (int64_t)s.out * s.kp;
+                bf16* wtf = nullptr;
+                if (m->train_fused && l > 0) TRY(dalloc(m, &wtf, (int64_t)s.out * s.kp));
+                m->wtf.push_back(wtf);
             }
-            m->fused_ok = true;
         }
         (void)hipGetLastError();
         return MCL_OK;
@@ -550,7 +634,6 @@ int mcl_mlp_set_params(void* mlp, const float* params)
         HIP_TRY(c, hipMemset(s.bv, 0, s.out * sizeof(float)));
     }
     TRY(run_optimizer(m, M::kOptRefresh, 64, {}, nullptr, nullptr));
-    m->wf_stale = true;
     HIP_TRY(c, hipStreamSynchronize(c->stream));
     return MCL_OK;
 }
@@ -572,9 +655,7 @@ int mcl_mlp_grad(void* mlp, const float* x, const float* t, const int32_t* idx, 
     if (!m || !x || !t) return MCL_EINVAL;
     TRY(check_batch(m, B));
     begin(m);
-    std::vector<int> splits;
-    TRY(forward_backward(m, x, t, idx, B, loss, splits));
-    if (grad) TRY(run_optimizer(m, M::kOptExportGrad, B, splits, grad, nullptr));
+    TRY(gradient(m, x, t, idx, B, M::kOptExportGrad, grad, loss, nullptr));
     return end(m);
 }
 
@@ -588,10 +669,7 @@ int mcl_mlp_train_step(void* mlp, const float* x, const float* t, const int32_t*
         !(hp->beta2 >= 0 && hp->beta2 < 1) || !(hp->eps > 0) || !(hp->weight_decay >= 0))
         return fail(m->ctx, MCL_EINVAL, "invalid AdamW hyper-parameters");
     begin(m);
-    std::vector<int> splits;
-    TRY(forward_backward(m, x, t, idx, B, loss, splits));
-    TRY(run_optimizer(m, M::kOptAdamW, B, splits, nullptr, hp));
-    m->wf_stale = true;
+    TRY(gradient(m, x, t, idx, B, M::kOptAdamW, nullptr, loss, hp));
     return end(m);
 }
 

@@ -14,6 +14,18 @@ namespace mlp {
 // their results bit-identical.
 __device__ __forceinline__ float sigmoid(float z) { return __builtin_amdgcn_rcpf(1.0f + __expf(-z)); }
 
+// Workgroup barrier that orders LDS only: the wave's global loads stay in flight
+// across it (a full barrier waits for every outstanding load, since the vector
+// memory counter counts loads and stores alike).  Every exchange between the
+// waves that needs this one goes through LDS; the global data they read (weights,
+// populations, inputs) does not change during the kernel.
+__device__ __forceinline__ void lds_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // What a GEMM's epilogue does with the FP32 accumulator acc[m][n] of
 // C = A B^T (A [M][K], B [N][K], both K-contiguous BF16).
 enum Epi : int {
@@ -71,6 +83,8 @@ struct OptLayer {
     float* w; float* m; float* v;     // FP32 master weight and moments [out][kp]
     __bf16* wb;                       // BF16 copy [out][kp]
     __bf16* wt;                       // BF16 transposed copy [kp][out]
+    __bf16* wf;                       // fragment-order copies of W and W^T (null: none;
+    __bf16* wtf;                      // written by a refresh)
     const float* part;                // weight-gradient partial sums [splits][out][kp]
     int splits;
     float* bw; float* bm; float* bv;  // bias master and moments [out]
@@ -82,21 +96,42 @@ struct OptLayer {
 
 enum OptMode : int { kOptAdamW = 0, kOptExportGrad = 1, kOptRefresh = 2 };
 
+struct AdamWArgs {
+    float lr, beta1, beta2, eps, wd;
+    float step_size;                  // lr / (1 - beta1^t)
+    float sqrt_bc2;                   // sqrt(1 - beta2^t)
+};
+
+__device__ __forceinline__ void adamw(float& w, float& m, float& v, float gr, const AdamWArgs& a)
+{
+    w = w * (1.0f - a.lr * a.wd);
+    m = a.beta1 * m + (1.0f - a.beta1) * gr;
+    v = a.beta2 * v + (1.0f - a.beta2) * (gr * gr);
+    w = w - a.step_size * (m / (sqrtf(v) / a.sqrt_bc2 + a.eps));
+}
+
 struct OptArgs {
     OptLayer L[kMaxLayers];
     int n_layers;
     int mode;
     int batch;
     float* flat;                      // kOptExportGrad destination
-    float lr, beta1, beta2, eps, wd;
-    float step_size;                  // lr / (1 - beta1^t)
-    float sqrt_bc2;                   // sqrt(1 - beta2^t)
+    AdamWArgs hp;
 };
 
 // Workgroups of the optimizer kernel: one per 32x32 weight tile, one per four biases.
 __host__ __device__ inline int opt_tiles(int out, int kp) { return (out / 32) * (kp / 32); }
 __host__ __device__ inline int opt_bias_groups(int out) { return out / 4; }
 hipError_t optimizer(const OptArgs& a, int n_groups, hipStream_t stream);
+
+// Element (row, col) of a row-major [rows][cols] BF16 matrix in fragment order: the
+// operand fragments of v_mfma_f32_32x32x16_bf16 (32 rows, 16 columns, 64 lanes of 8
+// columns), 16-column steps in order within each 32 rows.
+__host__ __device__ inline int64_t fragment_offset(int row, int col, int cols)
+{
+    return (((int64_t)(row >> 5) * (cols >> 4) + (col >> 4)) * 64 + (row & 31) +
+            32 * ((col >> 3) & 1)) * 8 + (col & 7);
+}
 
 // Network-scored differential evolution (de.hip).  x [pop][dim] the population,
 // f [pop] its objectives, X [pop_pad][n_in] the network input (trials in the first
@@ -152,6 +187,58 @@ int infer_fused_lds(const DeNet& net);
 hipError_t infer_fused_prepare(int lds_bytes);
 hipError_t infer_fused(const float* x, int B, int n_in, const DeNet& net, float* y, int n_out,
                        int lds_bytes, hipStream_t stream);
+
+// A training step in two kernels (mlp_train.hip) for networks of kTrainHidden hidden
+// layers of 512 (the first with its inputs padded to 64) and 256 or 512 outputs; other
+// shapes train layer by layer.
+constexpr int kTrainHidden = 4;
+constexpr int kTrainRows = 32;        // batch rows of a chain workgroup (batches: multiples of 64)
+
+// The forward and backward chain of batch B.  net: weights in fragment order; wtf[l]: W_l^T
+// in fragment order (l >= 1).  xf, af[l], dzf[l]: the packed input, activations and
+// errors as [features / 32][B / 16] fragments of 64 lanes of 8 batch rows.
+struct TrainArgs {
+    const float* x;                   // [rows][n_in]
+    const float* t;                   // [rows][n_out]
+    const int32_t* idx;               // batch row -> row of x and t (null: itself)
+    int n_in;
+    int64_t B;
+    float grad_scale;                 // 2 / (B n_out)
+    DeNet net;
+    const __bf16* wtf[kMaxLayers];
+    __bf16* xf;
+    __bf16* af[kMaxLayers];
+    __bf16* dzf[kMaxLayers];          // [n_layers - 1]: of the output
+    float* loss_part;                 // [B / kTrainRows]
+};
+
+struct UpdateLayer {
+    const __bf16* dzf;                // errors [out][B], fragments
+    const __bf16* xf;                 // inputs [kp][B], fragments
+    float *w, *m, *v;                 // [out][kp]
+    __bf16 *wb, *wf, *wtf;            // BF16 copies: row-major, fragments of W and (or null) W^T
+    float *bw, *bm, *bv;
+    int out, kp, k_in;
+    int blk0;                         // first workgroup: its 64 x 64 tiles, then 32 biases each
+    int64_t flat_w, flat_b;
+};
+
+struct UpdateArgs {
+    UpdateLayer L[kMaxLayers];
+    int n_layers, n_blocks, mode;     // kOptAdamW or kOptExportGrad
+    int64_t S;                        // B / 16
+    int parts;                        // 1, 2, 4 or 8 parts of the batch, summed in order
+    float* flat;
+    AdamWArgs hp;
+    const float* loss_part;
+    int n_part;
+    float loss_scale;
+    float* loss;                      // or null
+};
+bool train_fused_ok(const DeNet& net, int max_lds);
+hipError_t train_fused_prepare();
+hipError_t train_chain(const TrainArgs& a, int n_out, hipStream_t stream);
+hipError_t train_update(const UpdateArgs& a, hipStream_t stream);
 
 }  // namespace mlp
 }  // namespace mcl
