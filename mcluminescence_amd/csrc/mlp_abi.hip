@@ -433,11 +433,12 @@ int gradient(Mlp* m, const float* x, const float* t, const int32_t* idx, int32_t
         o.wb = s.wb; o.wf = const_cast<bf16*>(m->fnet.L[l].w); o.wtf = m->wtf[l];
         o.bw = s.bw; o.bm = s.bm; o.bv = s.bv;
         o.out = s.out; o.kp = s.kp; o.k_in = s.in;
-        o.blk0 = u.n_blocks;
+        o.tile0 = u.n_tiles;
+        o.bias0 = u.n_bias;
         o.flat_w = s.flat_w; o.flat_b = s.flat_b;
-        u.n_blocks += (s.out / 64) * (s.kp / 64) + s.out / 32;
+        u.n_tiles += (s.out / 64) * (s.kp / 64);
+        u.n_bias += s.out / 32;
     }
-    ++u.n_blocks;                          // the loss
     u.parts = 1;
     while (u.parts < kMaxSplits && B % (128 * u.parts) == 0) u.parts *= 2;
     u.flat = flat;

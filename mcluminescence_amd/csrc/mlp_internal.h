@@ -219,13 +219,13 @@ struct UpdateLayer {
     __bf16 *wb, *wf, *wtf;            // BF16 copies: row-major, fragments of W and (or null) W^T
     float *bw, *bm, *bv;
     int out, kp, k_in;
-    int blk0;                         // first workgroup: its 64 x 64 tiles, then 32 biases each
+    int tile0, bias0;                 // first 64 x 64 tile, first group of 32 biases
     int64_t flat_w, flat_b;
 };
 
 struct UpdateArgs {
     UpdateLayer L[kMaxLayers];
-    int n_layers, n_blocks, mode;     // kOptAdamW or kOptExportGrad
+    int n_layers, n_tiles, n_bias, mode;   // mode: kOptAdamW or kOptExportGrad
     int64_t S;                        // B / 16
     int parts;                        // 1, 2, 4 or 8 parts of the batch, summed in order
     float* flat;

@@ -327,16 +327,35 @@ __device__ __forceinline__ void update_biases(const UpdateArgs& a, const UpdateL
     constexpr int kLd = kBiasRows + 1;
     const int n = tid & 31;
     const int64_t groups = 2 * a.S;
-    for (int c = tid >> 5; c < 64; c += kThreadsT / 32) {
-        float s = 0.0f;
-        for (int64_t gr = c; gr < groups; gr += 64) {
-            const bf16x8 v = *reinterpret_cast<const bf16x8*>(
-                L.dzf + (((int64_t)T * a.S + (gr >> 1)) * 64 + n + 32 * (gr & 1)) * 8);
+    // a thread takes four of a row's 64 lanes, 16 fragments in flight: one at a time, its 32
+    // dependent trips at batch 4096 were longer than the tiles' products
+    constexpr int kC = 64 / (kThreadsT / 32), kU = 4;
+    const int c0 = tid >> 5;
+    float acc[kC];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) s += (float)v[i];
-        }
-        sums[c * kLd + n] = s;
+    for (int j = 0; j < kC; ++j) acc[j] = 0.0f;
+    for (int64_t g0 = 0; g0 < groups; g0 += 64 * kU) {
+        bf16x8 v[kU][kC];
+#pragma unroll
+        for (int u = 0; u < kU; ++u)
+#pragma unroll
+            for (int j = 0; j < kC; ++j) {
+                const int64_t gr = g0 + 64 * u + c0 + (kThreadsT / 32) * j;
+                const int64_t gl = gr < groups ? gr : 0;
+                v[u][j] = *reinterpret_cast<const bf16x8*>(
+                    L.dzf + (((int64_t)T * a.S + (gl >> 1)) * 64 + n + 32 * (gl & 1)) * 8);
+            }
+#pragma unroll
+        for (int u = 0; u < kU; ++u)
+#pragma unroll
+            for (int j = 0; j < kC; ++j)
+                if (g0 + 64 * u + c0 + (kThreadsT / 32) * j < groups) {
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) acc[j] += (float)v[u][j][i];
+                }
     }
+#pragma unroll
+    for (int j = 0; j < kC; ++j) sums[(c0 + (kThreadsT / 32) * j) * kLd + n] = acc[j];
     __syncthreads();
     for (int o = 32; o > 0; o >>= 1) {
         for (int c = tid >> 5; c < o; c += kThreadsT / 32) sums[c * kLd + n] += sums[(c + o) * kLd + n];
@@ -354,8 +373,20 @@ __global__ __launch_bounds__(kThreadsT, 2) void train_update_kernel(UpdateArgs a
     float* part = reinterpret_cast<float*>(smem_u);                    // [kWaves][kTile][kTile]
     bf16* tr = reinterpret_cast<bf16*>(part + kWaves * kTile * kTile); // [kTile][kTileLd]
     const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int blk = (int)blockIdx.x;
-    if (blk == a.n_blocks - 1) {                // the loss: chain partials in a fixed order
+    // Biases and the loss first: they are short, and the tiles left when every CU is
+    // taken start in their place.  Tiles then go to the XCDs (workgroups are dealt
+    // round-robin over them) in contiguous runs of a layer's row-major tiles, about four rows
+    // of dZ fragments and all columns of A: 5.8 MB through each L2 instead of the 16 that
+    // a column of every layer per XCD reads.
+    int blk = (int)blockIdx.x;
+    if (blk < a.n_bias) {
+        int li = 0;
+        while (li + 1 < a.n_layers && blk >= a.L[li + 1].bias0) ++li;
+        update_biases(a, a.L[li], blk - a.L[li].bias0, part, tid);
+        return;
+    }
+    blk -= a.n_bias;
+    if (blk == 0) {                             // the loss: chain partials in a fixed order
         if (a.loss == nullptr) return;
         float s = 0.0f;
         for (int i = tid; i < a.n_part; i += kThreadsT) s += a.loss_part[i];
@@ -368,15 +399,15 @@ __global__ __launch_bounds__(kThreadsT, 2) void train_update_kernel(UpdateArgs a
         if (tid == 0) *a.loss = part[0] * a.loss_scale;
         return;
     }
-    int li = 0;
-    while (li + 1 < a.n_layers && blk >= a.L[li + 1].blk0) ++li;
-    const UpdateLayer& L = a.L[li];
-    const int t = blk - L.blk0, tk_n = L.kp / kTile;
-    const int tiles = (L.out / kTile) * tk_n;
-    if (t >= tiles) {
-        update_biases(a, L, t - tiles, part, tid);
-        return;
+    {
+        const int i = blk - 1, whole = a.n_tiles / 8 * 8;
+        const int x = ((int)blockIdx.x) % 8, first = (a.n_bias + 1) % 8;   // XCD; of tile 0
+        blk = i < whole ? ((x - first + 8) % 8) * (a.n_tiles / 8) + i / 8 : i;
     }
+    int li = 0;
+    while (li + 1 < a.n_layers && blk >= a.L[li + 1].tile0) ++li;
+    const UpdateLayer& L = a.L[li];
+    const int t = blk - L.tile0, tk_n = L.kp / kTile;
     const int tn = t / tk_n, tk = t % tk_n;
     // the batch in `parts` contiguous ranges of steps; eight waves over the parts, and with
     // fewer than eight over the tile's 32 x 32 quarters too
@@ -488,7 +519,7 @@ hipError_t train_chain(const TrainArgs& a, int n_out, hipStream_t stream)
 
 hipError_t train_update(const UpdateArgs& a, hipStream_t stream)
 {
-    hipLaunchKernelGGL(train_update_kernel, dim3((unsigned)a.n_blocks), dim3(kThreadsT), kUpdateLds,
+    hipLaunchKernelGGL(train_update_kernel, dim3((unsigned)(a.n_bias + 1 + a.n_tiles)), dim3(kThreadsT), kUpdateLds,
                        stream, a);
     return hipGetLastError();
 }
