@@ -601,11 +601,16 @@ int mcl_mlp_get_params(void* mlp, float* params)
     HIP_TRY(m->ctx, hipStreamSynchronize(m->ctx->stream));
     std::vector<float> buf;
     for (const Layer& s : m->L) {
-        buf.resize((size_t)s.out * s.kp);
-        HIP_TRY(m->ctx, hipMemcpy(buf.data(), s.w, buf.size() * sizeof(float), hipMemcpyDeviceToHost));
-        for (int n = 0; n < s.out; ++n)
-            std::copy(buf.begin() + (size_t)n * s.kp, buf.begin() + (size_t)n * s.kp + s.in,
-                      params + s.flat_w + (int64_t)n * s.in);
+        const size_t nw = (size_t)s.out * s.kp;
+        if (s.kp == s.in) {
+            HIP_TRY(m->ctx, hipMemcpy(params + s.flat_w, s.w, nw * sizeof(float), hipMemcpyDeviceToHost));
+        } else {                       // rows of kp, of which the flat layout holds the first in
+            buf.resize(nw);
+            HIP_TRY(m->ctx, hipMemcpy(buf.data(), s.w, nw * sizeof(float), hipMemcpyDeviceToHost));
+            for (int n = 0; n < s.out; ++n)
+                std::copy(buf.begin() + (size_t)n * s.kp, buf.begin() + (size_t)n * s.kp + s.in,
+                          params + s.flat_w + (int64_t)n * s.in);
+        }
         HIP_TRY(m->ctx, hipMemcpy(params + s.flat_b, s.bw, s.out * sizeof(float), hipMemcpyDeviceToHost));
     }
     return MCL_OK;

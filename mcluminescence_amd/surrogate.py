@@ -347,11 +347,14 @@ class Network:
     def train_step(self, x, t, idx, hp: AdamW, loss_out=None) -> None:
         """One AdamW step on rows idx (int32 CUDA tensor) of x / t; the batch loss
         goes to loss_out (a one-element CUDA tensor) without a host sync."""
-        B = idx.shape[0]
         with self._on_stream(x, t, idx, loss_out):
-            self.ctx.check(self.lib.mcl_mlp_train_step(
-                self.handle, x.data_ptr(), t.data_ptr(), idx.data_ptr(), B, C.byref(hp),
-                None if loss_out is None else loss_out.data_ptr()), "mcl_mlp_train_step")
+            self._step(x, t, idx, hp, loss_out)
+
+    def _step(self, x, t, idx, hp: AdamW, loss_out) -> None:
+        """train_step on the stream the context is set to."""
+        self.ctx.check(self.lib.mcl_mlp_train_step(
+            self.handle, x.data_ptr(), t.data_ptr(), idx.data_ptr(), idx.shape[0], C.byref(hp),
+            None if loss_out is None else loss_out.data_ptr()), "mcl_mlp_train_step")
 
     def last_ms(self) -> float:
         v = C.c_double()
@@ -406,17 +409,19 @@ def train(net: Network, x, t, cfg: TrainConfig = TrainConfig(),
     ms = []
     for ep in range(cfg.epochs):
         perm = torch.randperm(N, generator=gen).to(torch.int32).to(x.device)
-        for b in range(steps_per_epoch):
-            step += 1
-            if step <= cfg.warmup_steps:
-                lr = cfg.lr * step / cfg.warmup_steps
-            else:
-                f = (step - cfg.warmup_steps) / max(1, total - cfg.warmup_steps)
-                lr = cfg.lr_min + 0.5 * (cfg.lr - cfg.lr_min) * (1.0 + math.cos(math.pi * f))
-            hp.lr = lr
-            hp.step = step
-            idx = perm[b * cfg.batch:(b + 1) * cfg.batch]
-            net.train_step(x, t, idx, hp, loss_buf[step - 1:step])
+        # one handshake of the two streams an epoch, not one a step (28 us of idle GPU and
+        # 50 us of host time each)
+        with net._on_stream(x, t, perm, loss_buf):
+            for b in range(steps_per_epoch):
+                step += 1
+                if step <= cfg.warmup_steps:
+                    lr = cfg.lr * step / cfg.warmup_steps
+                else:
+                    f = (step - cfg.warmup_steps) / max(1, total - cfg.warmup_steps)
+                    lr = cfg.lr_min + 0.5 * (cfg.lr - cfg.lr_min) * (1.0 + math.cos(math.pi * f))
+                hp.lr = lr
+                hp.step = step
+                net._step(x, t, perm[b * cfg.batch:(b + 1) * cfg.batch], hp, loss_buf[step - 1:step])
         ms.append(net.last_ms())
         if log and (ep % max(1, cfg.epochs // 10) == 0 or ep == cfg.epochs - 1):
             torch.cuda.synchronize()
