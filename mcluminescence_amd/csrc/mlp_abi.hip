@@ -194,7 +194,7 @@ int forward(Mlp* m, const float* x, int32_t B, float* y)
 {
     hipStream_t st = m->ctx->stream;
     if (m->fused_ok && m->ctx->mlp_fused != 0.0) {
-        HIP_TRY(m->ctx, M::infer_fused(x, B, m->d.n_in, m->fnet, y, m->d.n_out, m->fused_lds, st));
+        HIP_TRY(m->ctx, M::infer_fused(x, B, m->d.n_in, m->fnet, y, m->d.n_out, st));
         return MCL_OK;
     }
     HIP_TRY(m->ctx, M::pack_input(x, nullptr, m->d.n_in, B, m->L[0].kp, m->X0, nullptr, st));

@@ -178,7 +178,7 @@ hipError_t de_fused_prepare(int lds_bytes);
 hipError_t de_generation_fused(const DeArgs& a, const DeNet& net, uint32_t gen, int lds_bytes,
                                hipStream_t stream);
 
-// The inference forward in one kernel (mlp_fused.hip): 128 rows per workgroup
+// The inference forward in one kernel (mlp_fused.hip): 32 or 64 rows per workgroup
 // through every layer, activations in LDS, weights in fragment order (de_pack).
 // Hidden layers 512 wide (the first with its inputs padded to 64), the output
 // layer 256 or 512 wide.
@@ -186,7 +186,7 @@ bool infer_fused_ok(const DeNet& net);
 int infer_fused_lds(const DeNet& net);
 hipError_t infer_fused_prepare(int lds_bytes);
 hipError_t infer_fused(const float* x, int B, int n_in, const DeNet& net, float* y, int n_out,
-                       int lds_bytes, hipStream_t stream);
+                       hipStream_t stream);
 
 // A training step in two kernels (mlp_train.hip) for networks of kTrainHidden hidden
 // layers of 512 (the first with its inputs padded to 64) and 256 or 512 outputs; other
