@@ -43,6 +43,9 @@
 
 namespace mcl {
 
+// Steps tested at once when one is found quiet.  A step is 4 operations of the time's
+// chain of additions, so 16 cost about what one step did by itself.
+constexpr int kQuietRun = 16;
 
 __device__ __forceinline__ double exp1_of(uint32_t u)
 {
@@ -160,6 +163,7 @@ __device__ __forceinline__ void run_cluster_event(const EventArgs& a, const int 
     double l_et = 0.0, l_ef = 0.0;
     // The rows go out 64 at a time: lane j keeps row out_base + j until the
     // block is full or the loop ends, then every lane stores its own (coalesced).
+    // (out_base is sb_base in every step: both move on after 64 steps.)
     int out_base = 0;
     uint32_t o_lum = 0u;
     double o_t = 0.0, o_er = 0.0;
@@ -175,6 +179,17 @@ __device__ __forceinline__ void run_cluster_event(const EventArgs& a, const int 
             if (erat) erat[row] = o_er;
         }
         out_base = upto;
+    };
+
+    // Is a step at temperature kT with draw et certainly capped (see below)?  Bounds of the
+    // factors, not the factors: a step that skips K needs no more.
+    auto certainly_capped = [&](double kT, double et) -> bool {
+        const double a_ub = boltzmann_ub(R.s, s_ok, R.E_cb, kT);
+        const double b1_ub = b1_is_a ? a_ub : boltzmann_ub(R.b, b_ok, R.E_loc_1, kT);
+        const double b2_ub = b2_is_b1 ? b1_ub : boltzmann_ub(R.b, b_ok, R.E_loc_2, kT);
+        const double bm = two_ch ? fmax(b1_ub, b2_ub) : (always2 ? b2_ub : b1_ub);
+        const double k_ub = (bm * w_ub + (double)n_live * a_ub) * (1.0 + 0x1p-30);
+        return et > dt_cap * k_ub * (1.0 + 0x1p-30);
     };
 
     while (t <= R.duration) {
@@ -243,13 +258,40 @@ __device__ __forceinline__ void run_cluster_event(const EventArgs& a, const int 
                 w_ub = row_total_d(ws) * (1.0 + 0x1p-30);
                 w_valid = true;
             }
-            // bounds of the factors (not the factors: a step that skips K needs no more)
-            const double a_ub = boltzmann_ub(R.s, s_ok, R.E_cb, kT);
-            const double b1_ub = b1_is_a ? a_ub : boltzmann_ub(R.b, b_ok, R.E_loc_1, kT);
-            const double b2_ub = b2_is_b1 ? b1_ub : boltzmann_ub(R.b, b_ok, R.E_loc_2, kT);
-            const double bm = two_ch ? fmax(b1_ub, b2_ub) : (always2 ? b2_ub : b1_ub);
-            const double k_ub = (bm * w_ub + (double)n_live * a_ub) * (1.0 + 0x1p-30);
-            quiet = e_t > dt_cap * k_ub * (1.0 + 0x1p-30);
+            quiet = certainly_capped(kT, e_t);
+        }
+        if (quiet && fill_never) {
+            // Quiet steps change nothing but the time, so the run of them from this one on
+            // is taken at once: lane js + m holds step i + m as it is after m capped steps
+            // (its time the same m additions) and tests it with its own draw; the steps
+            // before the first that may not be quiet, or would not run, are rows of no event.
+            if (erat && n_live + filled != erat_n) {
+                erat_n = n_live + filled;
+                erat_v = (double)erat_n / R.N_e;
+            }
+            double tl = t;
+#pragma unroll
+            for (int k = 0; k < kQuietRun - 1; ++k) tl = lane - js > k ? tl + dt_cap : tl;
+            const double kTl = R.k_b * ((R.T_start_C + R.T_rate * tl) + 273.15);
+            const bool runs = lane == js || (tl <= R.duration && !(R.duration != 0.0 && tl >= R.duration));
+            const bool ok = certainly_capped(kTl, l_et) && runs && sb_base + lane < max_steps &&
+                            lane < js + kQuietRun;
+            const uint64_t stop = ~ballot(ok) & (~0ull << js);
+            const int f = stop != 0 ? (int)__builtin_ctzll(stop) : kWave;
+            if (f > js) {
+                const double after = tl + dt_cap;
+                if (lane >= js && lane < f) {
+                    o_lum = 0u;
+                    o_t = after;
+                    o_er = erat_v;
+                }
+                t = lane_value_d(after, f - 1);
+                lsteps += (uint64_t)n_live * (uint64_t)(f - js - 1);
+                i += f - js;
+                if (i - out_base == kWave) flush_rows(i);
+                if (R.duration != 0.0 && t >= R.duration) break;
+                continue;
+            }
         }
         const int rows = (n_live + kWave - 1) / kWave;
         double K = 0.0;
