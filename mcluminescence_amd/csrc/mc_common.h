@@ -118,141 +118,7 @@ __device__ __forceinline__ uint64_t block_search_lane(const Grid& g, float x, fl
     return key;
 }
 
-// 3x3x3 cell block around (x, y, z): cell bounds, clamped to the grid.
-struct Block {
-    int x0, x1, y0, y1, z0, z1;
-    __device__ __forceinline__ Block(const Grid& g, float x, float y, float z)
-    {
-        const int G = g.G;
-        const int cx = cell_of(x, g.inv_cell, G), cy = cell_of(y, g.inv_cell, G),
-                  cz = cell_of(z, g.inv_cell, G);
-        x0 = max(cx - 1, 0);
-        x1 = min(cx + 1, G - 1);
-        y0 = max(cy - 1, 0);
-        y1 = min(cy + 1, G - 1);
-        z0 = max(cz - 1, 0);
-        z1 = min(cz + 1, G - 1);
-    }
-    // Is the block minimum d2 provably the nearest live hole of (x, y, z)?
-    __device__ __forceinline__ bool conclusive(const Grid& g, float x, float y, float z,
-                                               float best_d2) const
-    {
-        const int G = g.G;
-        const bool whole = x0 == 0 && y0 == 0 && z0 == 0 && x1 == G - 1 && y1 == G - 1 &&
-                           z1 == G - 1;
-        const float gap = fminf(face_gap(x, x0, x1, G, g.cell),
-                                fminf(face_gap(y, y0, y1, G, g.cell), face_gap(z, z0, z1, G, g.cell)));
-        return whole || block_conclusive(best_d2, gap, g.cell);
-    }
-};
-
-// Wave-cooperative search for one electron (x, y, z wave-uniform).  The 3x3x3
-// block is at most 9 contiguous slot ranges (one per (z, y) row of cells); lane
-// l takes range l / 7 at offsets l % 7, l % 7 + 7, ... so every lane finds its
-// slots from two cell starts, with no cross-lane bookkeeping, then a wave min.
-// Ranges longer than 7 holes cost one more pass each 7.
-__device__ __forceinline__ uint64_t block_search_wave(const Grid& g, float x, float y, float z,
-                                                      int lane, bool& conclusive, uint64_t& evals)
-{
-    constexpr int kPer = 7;                          // lanes per range (9 x 7 = 63 lanes)
-    const int G = g.G;
-    const int cx = cell_of(x, g.inv_cell, G), cy = cell_of(y, g.inv_cell, G),
-              cz = cell_of(z, g.inv_cell, G);
-    const int x0 = max(cx - 1, 0), x1 = min(cx + 1, G - 1);
-    const int y0 = max(cy - 1, 0), y1 = min(cy + 1, G - 1);
-    const int z0 = max(cz - 1, 0), z1 = min(cz + 1, G - 1);
-    const int j = lane / kPer, o = lane - j * kPer;
-    // (z, y) row j of the unclamped block; rows outside the grid are empty
-    const int jz = j / 3, zz = cz - 1 + jz, yy = cy - 1 + (j - 3 * jz);
-    int s = 0, e = 0;
-    if (j < 9 && (unsigned)zz < (unsigned)G && (unsigned)yy < (unsigned)G) {
-        const int base = (zz * G + yy) * G;
-        s = (int)g.cstart[base + x0];
-        e = (int)g.cstart[base + x1 + 1];
-    }
-    if (o == 0) evals += (uint64_t)(e - s);          // summed over lanes at the end
-    uint64_t key = ~0ull;
-    for (int slot = s + o;; slot += kPer) {
-        const bool v = slot < e;
-        if (ballot(v) == 0) break;
-        if (v) {
-            const uint64_t k = key_of(g.hole[slot], x, y, z, slot);
-            key = k < key ? k : key;
-        }
-    }
-    key = wave_min_u64(key);
-    const bool whole = x0 == 0 && y0 == 0 && z0 == 0 && x1 == G - 1 && y1 == G - 1 && z1 == G - 1;
-    const float gap = fminf(face_gap(x, x0, x1, G, g.cell),
-                            fminf(face_gap(y, y0, y1, G, g.cell), face_gap(z, z0, z1, G, g.cell)));
-    conclusive = whole || block_conclusive(__uint_as_float((uint32_t)(key >> 32)), gap, g.cell);
-    return key;
-}
-
-// Wave-cooperative 3x3x3 block searches for up to kSearchBatch (four) electrons at
-// once, one 16-lane row each (x, y, z: the row's electron, the same in all its
-// lanes).  A block is at most 9 contiguous slot ranges (one per (z, y) row of
-// cells); lane q of the row takes offsets q, q + 16, ... of every range, so its 9
-// range loads are independent; ranges longer than 16 holes take further passes.
-// The row minimum is four DPP steps.  Returns the row's block minimum key in every
-// lane of the row (~0 for rows at or beyond nb).
-constexpr int kSearchBatch = 4;
-__device__ __forceinline__ uint64_t block_search_rows(const Grid& g, int nb, float x, float y,
-                                                      float z, int lane, uint64_t& evals)
-{
-    const int G = g.G;
-    const int q = lane & 15;
-    const bool act = (lane >> 4) < nb;
-    int s[9], e[9];
-    int longest = 0, total = 0;
-    const Block k(g, x, y, z);
-    const int cz = cell_of(z, g.inv_cell, G), cy = cell_of(y, g.inv_cell, G);
-    // (z, y) row r of the unclamped block; rows outside the grid, and all rows of a lane
-    // row without an electron, are empty (their reads go to the nearest row inside).
-    // No branches, so that the 18 cell starts and then the 9 holes are in flight
-    // together: inside `if`s each would wait for the one before.
-#pragma unroll
-    for (int r = 0; r < 9; ++r) {
-        const int zz = cz - 1 + r / 3, yy = cy - 1 + r % 3;
-        const int base = (min(max(zz, 0), G - 1) * G + min(max(yy, 0), G - 1)) * G;
-        s[r] = (int)g.cstart[base + k.x0];
-        e[r] = (int)g.cstart[base + k.x1 + 1];
-    }
-#pragma unroll
-    for (int r = 0; r < 9; ++r) {
-        const int zz = cz - 1 + r / 3, yy = cy - 1 + r % 3;
-        const bool in = act && (unsigned)zz < (unsigned)G && (unsigned)yy < (unsigned)G;
-        e[r] = in ? e[r] : s[r];
-        total += e[r] - s[r];
-        longest = max(longest, e[r] - s[r]);
-    }
-    evals += q == 0 ? (uint64_t)total : 0ull;          // summed over lanes at the end
-    uint64_t key = ~0ull;
-    float4 hv[9];
-    // (a range's first slot is within the hole array's capacity, empty ranges included)
-#pragma unroll
-    for (int r = 0; r < 9; ++r) hv[r] = g.hole[s[r] + q < e[r] ? s[r] + q : s[r]];
-#pragma unroll
-    for (int r = 0; r < 9; ++r) {
-        const int slot = s[r] + q;
-        uint64_t k2 = key_of(hv[r], x, y, z, slot);
-        k2 = slot < e[r] ? k2 : ~0ull;
-        key = k2 < key ? k2 : key;
-    }
-    if (ballot(longest > 16) != 0) {
-#pragma unroll 1
-        for (int r = 0; r < 9; ++r) {
-            const int zz = cz - 1 + r / 3, yy = cy - 1 + r % 3;
-            if (!act || (unsigned)zz >= (unsigned)G || (unsigned)yy >= (unsigned)G) continue;
-            const int base = (zz * G + yy) * G;
-            const int e2 = (int)g.cstart[base + k.x1 + 1];
-            for (int slot = (int)g.cstart[base + k.x0] + q + 16; slot < e2; slot += 16) {
-                const uint64_t k2 = key_of(g.hole[slot], x, y, z, slot);
-                key = k2 < key ? k2 : key;
-            }
-        }
-    }
-    return row_min_u64(key);
-}
+constexpr int kSearchBatch = 4;   // electrons searched at once by the whole wave
 
 // The whole wave scans every hole for one electron (x, y, z wave-uniform).
 __device__ __forceinline__ uint64_t full_scan_wave(const Grid& g, float x, float y, float z,
@@ -618,86 +484,6 @@ __device__ __forceinline__ Grid setup_cluster(const RunDesc& R, const ElectronGe
                                               uint64_t& dist_evals)
 {
     return setup_cluster_t<1, WIDE>(R, egen, hole, cstart, est, ew, prun, psim, k0, k1, lane, dist_evals);
-}
-
-// New nearest holes for the queued electrons rq[0..nq) ((slot << 16) | index):
-// wave-cooperative searches, kSearchBatch electrons at a time, while the queue
-// is short (at most wave_search_max), lane-parallel otherwise; writes est and ew
-// of their slots.
-template <bool WIDE>
-__device__ __forceinline__ void search_queue_nn(const Grid& grid, const ElectronGen& egen,
-                                                uint32_t* est, float* ew, const uint32_t* rq,
-                                                int nq, int wave_search_max, float alpha_f,
-                                                int lane, uint64_t& dist_evals)
-{
-    if (nq <= wave_search_max) {
-        for (int i0 = 0; i0 < nq; i0 += kSearchBatch) {
-            const int nb = min(kSearchBatch, nq - i0);
-            if (nb == 1) {
-                // one electron: the whole wave takes its block (9 ranges x 7 lanes)
-                const uint32_t qq = rq[i0];
-                float qx, qy, qz;
-                egen.xyz(qq & 0xFFFFu, qx, qy, qz);
-                bool ok = true;
-                uint64_t key = block_search_wave(grid, qx, qy, qz, lane, ok, dist_evals);
-                if (!ok) key = far_search_wave<WIDE>(grid, qx, qy, qz, lane, dist_evals);
-                if (lane == 0) {
-                    uint32_t slot;
-                    float w;
-                    nn_from_key(key, alpha_f, slot, w);
-                    est[qq >> 16] = (slot << 16) | (qq & 0xFFFFu);
-                    ew[qq >> 16] = w;
-                }
-                continue;
-            }
-            // two to four electrons: one 16-lane row each; every lane of row b
-            // regenerates electron b's coordinates (the same Philox call in all lanes)
-            const int b = lane >> 4;
-            const bool act = b < nb;
-            const uint32_t qq = act ? rq[i0 + b] : 0u;
-            float qx = 0.0f, qy = 0.0f, qz = 0.0f;
-            if (act) egen.xyz(qq & 0xFFFFu, qx, qy, qz);
-            uint64_t key = block_search_rows(grid, nb, qx, qy, qz, lane, dist_evals);
-            bool ok = true;
-            if (act) {
-                const Block k(grid, qx, qy, qz);
-                ok = k.conclusive(grid, qx, qy, qz, __uint_as_float((uint32_t)(key >> 32)));
-            }
-            // rows whose block was inconclusive: the whole wave scans every hole
-            uint64_t fb = ballot((lane & 15) == 0 && act && !ok);
-            while (fb != 0) {
-                const int l = __builtin_ctzll(fb);
-                fb &= fb - 1;
-                const uint64_t k = far_search_wave<WIDE>(grid, lane_value(qx, l), lane_value(qy, l),
-                                                  lane_value(qz, l), lane, dist_evals);
-                if ((lane >> 4) == (l >> 4)) key = k;
-            }
-            if (act && (lane & 15) == 0) {
-                uint32_t slot;
-                float w;
-                nn_from_key(key, alpha_f, slot, w);
-                est[qq >> 16] = (slot << 16) | (qq & 0xFFFFu);
-                ew[qq >> 16] = w;
-            }
-        }
-        return;
-    }
-    for (int q0 = 0; q0 < nq; q0 += kWave) {
-        const int i = q0 + lane;
-        const bool act = i < nq;
-        const uint32_t q = act ? rq[i] : 0u;
-        const uint32_t o = q & 0xFFFFu;
-        float x = 0.0f, y = 0.0f, z = 0.0f;
-        if (act) egen.xyz(o, x, y, z);
-        const uint64_t key = nn_resolve<WIDE>(grid, act, x, y, z, lane, dist_evals);
-        if (act) {
-            uint32_t slot;
-            float w;
-            nn_from_key(key, alpha_f, slot, w);
-            est[q >> 16] = (slot << 16) | o;
-            ew[q >> 16] = w;
-        }
-    }
 }
 
 }  // namespace mcl

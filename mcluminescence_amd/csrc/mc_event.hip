@@ -43,9 +43,8 @@
 
 namespace mcl {
 
-// Steps tested at once when one is found quiet.  A step is 4 operations of the time's
-// chain of additions, so 16 cost about what one step did by itself.
-constexpr int kQuietRun = 16;
+// Recombinations after which the bound of the sum of w is summed anew.
+constexpr int kWRefresh = 64;
 
 __device__ __forceinline__ double exp1_of(uint32_t u)
 {
@@ -167,10 +166,13 @@ __device__ __forceinline__ void run_cluster_event(const EventArgs& a, const int 
     int out_base = 0;
     uint32_t o_lum = 0u;
     double o_t = 0.0, o_er = 0.0;
-    // An upper bound of the sum of w over the live electrons that have a hole,
-    // valid until the next recombination changes the electrons or their w.
+    // An upper bound of the sum of w over the live electrons that have a hole.  A
+    // recombination takes its electron's w off it and replaces those searched again; w_tol
+    // covers the roundings of those sums (each below 2^-52 of the first bound, with up to a
+    // few hundred terms between two full sums; it is summed anew after kWRefresh events).
     bool w_valid = false;
-    double w_ub = 0.0;
+    double w_ub = 0.0, w_tol = 0.0;
+    int w_age = 0;
     auto flush_rows = [&](int upto) {
         const int row = out_base + lane;
         if (row < upto) {
@@ -256,68 +258,75 @@ __device__ __forceinline__ void run_cluster_event(const EventArgs& a, const int 
                     ws += (sa >> 16) != kNoHole ? (double)wa : 0.0;
                 }
                 w_ub = row_total_d(ws) * (1.0 + 0x1p-30);
+                w_tol = w_ub * 0x1p-44;
                 w_valid = true;
             }
-            quiet = certainly_capped(kT, e_t);
-        }
-        if (quiet && fill_never) {
-            // Quiet steps change nothing but the time, so the run of them from this one on
-            // is taken at once: lane js + m holds step i + m as it is after m capped steps
-            // (its time the same m additions) and tests it with its own draw; the steps
-            // before the first that may not be quiet, or would not run, are rows of no event.
-            if (erat && n_live + filled != erat_n) {
-                erat_n = n_live + filled;
-                erat_v = (double)erat_n / R.N_e;
-            }
-            double tl = t;
-#pragma unroll
-            for (int k = 0; k < kQuietRun - 1; ++k) tl = lane - js > k ? tl + dt_cap : tl;
-            const double kTl = R.k_b * ((R.T_start_C + R.T_rate * tl) + 273.15);
-            const bool runs = lane == js || (tl <= R.duration && !(R.duration != 0.0 && tl >= R.duration));
-            const bool ok = certainly_capped(kTl, l_et) && runs && sb_base + lane < max_steps &&
-                            lane < js + kQuietRun;
-            const uint64_t stop = ~ballot(ok) & (~0ull << js);
-            const int f = stop != 0 ? (int)__builtin_ctzll(stop) : kWave;
-            if (f > js) {
-                const double after = tl + dt_cap;
-                if (lane >= js && lane < f) {
-                    o_lum = 0u;
-                    o_t = after;
-                    o_er = erat_v;
+            if (fill_never) {
+                // Quiet steps change nothing but the time, so the run of them from this one
+                // on is taken at once.  Lane js + m tests step i + m, with its own draw, at
+                // the time after m capped steps: t + m dt_cap here, whose difference from the
+                // m additions (a few ulp) the bounds' margins cover; a step that may reach
+                // the duration is left to the loop.
+                const double ta = t + (double)(lane - js) * dt_cap;
+                const bool runs = lane == js || ta < R.duration * (1.0 - 0x1p-40);
+                const bool ok = certainly_capped(R.k_b * ((R.T_start_C + R.T_rate * ta) + 273.15), l_et) &&
+                                runs && sb_base + lane < max_steps;
+                const uint64_t stop = ~ballot(ok) & (~0ull << js);
+                const int f = stop != 0 ? (int)__builtin_ctzll(stop) : kWave;
+                if (f > js) {
+                    if (erat && n_live + filled != erat_n) {
+                        erat_n = n_live + filled;
+                        erat_v = (double)erat_n / R.N_e;
+                    }
+                    // the rows of steps js .. f - 1: no event, the time by its additions
+                    double tl = t;
+                    for (int m = js; m < f; ++m) {
+                        tl += dt_cap;
+                        if (lane == m) o_t = tl;
+                    }
+                    if (lane >= js && lane < f) {
+                        o_lum = 0u;
+                        o_er = erat_v;
+                    }
+                    t = tl;
+                    lsteps += (uint64_t)n_live * (uint64_t)(f - js - 1);
+                    i += f - js;
+                    if (i - out_base == kWave) flush_rows(i);
+                    if (R.duration != 0.0 && t >= R.duration) break;
+                    continue;
                 }
-                t = lane_value_d(after, f - 1);
-                lsteps += (uint64_t)n_live * (uint64_t)(f - js - 1);
-                i += f - js;
-                if (i - out_base == kWave) flush_rows(i);
-                if (R.duration != 0.0 && t >= R.duration) break;
-                continue;
+            } else {
+                quiet = certainly_capped(kT, e_t);
             }
         }
         const int rows = (n_live + kWave - 1) / kWave;
-        double K = 0.0;
+        double K = 0.0, l_rt = 0.0;
         if (!quiet) {
             A = boltzmann(R.s, s_ok, R.E_cb, kT);
             B1 = b1_is_a ? A : boltzmann(R.b, b_ok, R.E_loc_1, kT);
             B2 = b2_is_b1 ? B1 : boltzmann(R.b, b_ok, R.E_loc_2, kT);
             // row totals (the scan's lane-63 values), two rows at a time (independent
-            // chains), added in order
+            // chains), added in order; up to 64 rows' totals stay in the lanes, so that the
+            // selection reads them without an LDS trip each
+            auto keep = [&](int r, double v) {
+                if (rows <= kWave) l_rt = lane == r ? v : l_rt;
+                else if (lane == 0) rtot[r] = v;
+            };
             int r = 0;
             for (; r + 1 < rows; r += 2) {
                 const double ra = row_total_d(rate_of(r * kWave + lane));
                 const double rb = row_total_d(rate_of((r + 1) * kWave + lane));
-                if (lane == 0) {
-                    rtot[r] = ra;
-                    rtot[r + 1] = rb;
-                }
+                keep(r, ra);
+                keep(r + 1, rb);
                 K = K + ra;
                 K = K + rb;
             }
             if (r < rows) {
                 const double rt = row_total_d(rate_of(r * kWave + lane));
-                if (lane == 0) rtot[r] = rt;
+                keep(r, rt);
                 K = K + rt;
             }
-            event_fence<GM>();
+            if (rows > kWave) event_fence<GM>();
         }
         double dt_rec = dt_fill;
         if (n_live > 0) dt_rec = quiet ? __builtin_inf() : (K > 0.0 ? e_t / K : __builtin_inf());
@@ -336,7 +345,7 @@ __device__ __forceinline__ void run_cluster_event(const EventArgs& a, const int 
             int pw = -1;
             double carry = 0.0;
             for (int r = 0; r < rows; ++r) {
-                const double c2 = carry + rtot[r];
+                const double c2 = carry + (rows <= kWave ? lane_value_d(l_rt, r) : rtot[r]);
                 if (c2 > target) {
                     const double v = row_scan_d(rate_of(r * kWave + lane), lane);
                     const uint64_t m = ballot(carry + v > target);
@@ -354,37 +363,67 @@ __device__ __forceinline__ void run_cluster_event(const EventArgs& a, const int 
             }
             pw = uniform(pw);
             const uint32_t sw = est[pw];
+            const double w_gone = (double)ew[pw];
             const uint32_t hw = sw >> 16;
             if (lane == 0) hole_f[4 * hw] = kDeadHoleX;
-            // One pass over the rows: slots pw + 1 .. n_live - 1 move down by one (the
-            // index order kept; a row reads its sources before it writes, and the next
-            // row's sources lie beyond what it wrote), and the electrons whose nearest
-            // hole was hw are queued, at their new slots, for a new search
-            // (engine.py:168-175).
+            // Slots pw + 1 .. n_live - 1 move down by one (the index order kept), and the
+            // electrons whose nearest hole was hw are searched again, at their new slots
+            // (engine.py:168-175).  Two rows at a time: their sources are read before either
+            // is written, and the next rows' sources lie beyond what they wrote.
             const int n_new = n_live - 1;
             int nq = 0;
-            for (int r = 0; r * kWave < n_new; ++r) {
-                const int p = r * kWave + lane;
-                const bool in = p < n_new, moves = in && p >= pw;
-                const uint32_t st = in ? est[moves ? p + 1 : p] : kDeadSlot;
-                const float w = moves ? ew[p + 1] : 0.0f;
-                if (moves) {
-                    est[p] = st;
-                    ew[p] = w;
+            double w_change = -w_gone;
+            for (int r = 0; r * kWave < n_new; r += 2) {
+                const int p0 = r * kWave + lane, p1 = p0 + kWave;
+                const bool in0 = p0 < n_new, in1 = p1 < n_new;
+                const bool mv0 = in0 && p0 >= pw, mv1 = in1 && p1 >= pw;
+                const uint32_t s0 = in0 ? est[mv0 ? p0 + 1 : p0] : kDeadSlot;
+                const uint32_t s1 = in1 ? est[mv1 ? p1 + 1 : p1] : kDeadSlot;
+                const float w0 = mv0 ? ew[p0 + 1] : 0.0f, w1 = mv1 ? ew[p1 + 1] : 0.0f;
+                if (mv0) {
+                    est[p0] = s0;
+                    ew[p0] = w0;
                 }
-                const bool s = (st >> 16) == hw;
-                const uint64_t m = ballot(s);
-                if (s) rq[nq + lanes_below(m)] = ((uint32_t)p << 16) | (st & 0xFFFFu);
-                nq += __popcll(m);
+                if (mv1) {
+                    est[p1] = s1;
+                    ew[p1] = w1;
+                }
+                const bool q0 = (s0 >> 16) == hw, q1 = (s1 >> 16) == hw;
+                const uint64_t m0 = ballot(q0);
+                if (q0) rq[nq + lanes_below(m0)] = ((uint32_t)p0 << 16) | (s0 & 0xFFFFu);
+                nq += __popcll(m0);
+                const uint64_t m1 = ballot(q1);
+                if (q1) rq[nq + lanes_below(m1)] = ((uint32_t)p1 << 16) | (s1 & 0xFFFFu);
+                nq += __popcll(m1);
             }
             n_live = n_new;
             recomb += 1;
-            w_valid = false;
             event_fence<GM>();
-            if (nq > 0) {
-                search_queue_nn<GM>(grid, egen, est, ew, rq, nq, a.wave_search_max, alpha_f, lane,
-                                dist_evals);
+            // the queued electrons, one a lane
+            for (int q0 = 0; q0 < nq; q0 += kWave) {
+                const bool act = q0 + lane < nq;
+                const uint32_t qq = act ? rq[q0 + lane] : 0u;
+                float x, y, z;
+                egen.xyz(qq & 0xFFFFu, x, y, z);
+                uint64_t key = ~0ull;
+                search_lanes<GM>(grid, ballot(act), act, x, y, z, a.wave_search_max, lane, key,
+                                 dist_evals);
+                double dw = 0.0;
+                if (act) {
+                    uint32_t slot;
+                    float w;
+                    nn_from_key(key, alpha_f, slot, w);
+                    dw = (double)w - (double)ew[qq >> 16];
+                    est[qq >> 16] = (slot << 16) | (qq & 0xFFFFu);
+                    ew[qq >> 16] = w;
+                }
+                w_change += row_total_d(dw);
                 event_fence<GM>();
+            }
+            w_ub = w_ub + w_change + w_tol;
+            if (++w_age >= kWRefresh) {
+                w_age = 0;
+                w_valid = false;
             }
             ev = 1;
         }
