@@ -1042,8 +1042,9 @@ int mcl_run_lab(void* ctx, const mcl_run_params* runs, int32_t n_runs, const dou
     const int e_cap = ((max_e + 64 + 63) / 64) * 64;
     const int h_cap = ((max_h + 2 * max_e + 64 + 3) / 4) * 4;
     const int lds = mcl::lab_lds_bytes(h_cap, e_cap);
-    if (lds > c->max_lds)
-        return fail(c, MCL_ERANGE, "lab cluster needs %d B of LDS; a workgroup has %d B", lds,
+    const int need = mcl::lab_capacity_bytes(h_cap, e_cap);
+    if (need > c->max_lds)
+        return fail(c, MCL_ERANGE, "lab cluster needs %d B of LDS; a workgroup has %d B", need,
                     c->max_lds);
     std::vector<int32_t> crun((size_t)total), csim((size_t)total);
     {

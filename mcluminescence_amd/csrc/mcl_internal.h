@@ -120,6 +120,9 @@ struct LabArgs {
     uint32_t options;           // MCL_LAB_* bits
 };
 int lab_lds_bytes(int h_cap, int e_cap);
+// What a lab cluster counts against a workgroup's LDS when it is accepted: 20 bytes a hole slot
+// and an electron slot (its layout takes fewer, lab_lds_bytes).
+int lab_capacity_bytes(int h_cap, int e_cap);
 
 constexpr int kWaveHost = 64;   // wavefront width of gfx950
 
