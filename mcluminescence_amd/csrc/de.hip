@@ -3,18 +3,21 @@
 // with no host round trip.
 //
 // Two forms of a generation, with identical results:
-//   - fused (de_generation_kernel): one kernel.  A workgroup takes 16 members:
-//     their trials, the whole network forward with the activations in LDS and
-//     the weights read from L2 straight into matrix-core registers, the
+//   - fused (de_generation_kernel): one kernel.  A workgroup takes 4, 8 or 16
+//     members: their trials, the whole network forward with the activations in LDS
+//     and the weights read from L2 straight into matrix-core registers, the
 //     objectives and the selection; 16 waves, one 32-wide output tile each, so
 //     for networks whose layers are at most 512 wide.  The matrix-core tiles are
-//     32 rows: the members' 16 and 16 zero rows, whose outputs no epilogue
-//     computes, so that each workgroup's share of the SiLU epilogues and
-//     objectives is half of what 32 members would give, over twice the CUs (every
-//     CU streams the whole weight set either way).  The weights are read from a
-//     copy in fragment order (de_pack_kernel, made when the search is created),
-//     so that one load instruction of a wave reads 1 KB of contiguous memory
-//     instead of 32 bytes of 32 rows.
+//     32 rows: the members' and zero rows, whose outputs no epilogue computes.
+//     What bounds it: every CU streams the whole weight set (1.9 MB at 64 B a cycle,
+//     29.8 k cycles of the kernel's 39 k with 8 members: the hidden layers run at
+//     that rate), so the members are spread over more CUs until those contend for
+//     the L2s; the rest is the start (arguments, keys and partner rows, the best
+//     member's row: three trips to memory one after another, 6 k cycles) and the
+//     objectives (2 k).  The weights are read from a copy in fragment order
+//     (de_pack_kernel, made when the search is created), so that one load
+//     instruction of a wave reads 1 KB of contiguous memory instead of 32 bytes of
+//     32 rows.
 //   - layered: a propose kernel that writes the trials into the network's packed
 //     BF16 input rows, the network's own GEMM kernels (mlp.hip), and a
 //     score-and-accept kernel.
@@ -46,8 +49,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr uint32_t kInitGen = 0xFFFFFFFFu;   // counter word 0 of the initial population
 constexpr int kRows = 32;                    // rows of the fused kernel's matrix-core tiles
-constexpr int kMembers = 16;                 // members per workgroup: tile rows 0-15 (16-31 are
-                                             // zero padding rows, which no epilogue writes)
+constexpr int kMembers = 16;                 // members of a workgroup at other shapes
 constexpr int kFusedThreads = 1024;          // its 16 waves: one 32-wide output tile each
 
 __device__ __forceinline__ float unit_f(uint32_t w) { return ((float)(w >> 8) + 0.5f) * 0x1p-24f; }
@@ -82,100 +84,127 @@ __global__ __launch_bounds__(256) void de_init_kernel(DeArgs a)
 // Population argmin from the members' keys (objective bits << 32 | member; the
 // objectives are >= 0, so their float bits order as the values, and ties go to
 // the lowest member), reduced by each workgroup of NT threads: a strided minimum
-// per thread, then across the wave by shuffles and across the waves in LDS.
-template <int NT>
-__device__ __forceinline__ int population_argmin(const DeArgs& a)
+// per thread (k: its first key, first_key), then across the wave and, through LDS,
+// across the waves.
+__device__ __forceinline__ uint64_t first_key(const DeArgs& a)
 {
-    __shared__ unsigned long long wmin[NT / 64];
-    unsigned long long k = ~0ull;
-    for (int j = (int)threadIdx.x; j < a.pop; j += NT) k = a.keys[j] < k ? a.keys[j] : k;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const unsigned long long v = (unsigned long long)__shfl_xor((long long)k, o, 64);
-        k = v < k ? v : k;
-    }
-    if ((threadIdx.x & 63u) == 0u) wmin[threadIdx.x >> 6] = k;
-    lds_barrier();
-    k = wmin[0];
-    for (int w = 1; w < NT / 64; ++w) k = wmin[w] < k ? wmin[w] : k;
-    return (int)(uint32_t)k;
+    // (threads past the population repeat its last key)
+    return a.keys[(int)threadIdx.x < a.pop ? (int)threadIdx.x : a.pop - 1];
 }
 
-// The trial of member i (< pop) in two halves, so that its draws and partner
-// rows can be fetched before the population argmin is known: trial_fetch takes
-// the draws and the rows of the member and its three partners, trial_finish the
-// best member's row and the mutant, crossover and redraws.  Together they are
-// the one-step computation the layered form's propose kernel does.
-struct Trial {
-    u32x4 c0, c1, d0, d1;       // crossover and redraw words
-    int jr;                     // the coordinate that always crosses over
-    float xi[8], x0[8], x1[8], x2[8];
+template <int NT>
+__device__ __forceinline__ int population_argmin(const DeArgs& a, uint64_t k)
+{
+    __shared__ uint64_t wmin[NT / 64];
+    for (int j = (int)threadIdx.x + NT; j < a.pop; j += NT) k = a.keys[j] < k ? a.keys[j] : k;
+    k = wave_min_u64(k);
+    if ((threadIdx.x & 63u) == 0u) wmin[threadIdx.x >> 6] = k;
+    lds_barrier();
+    const int lane = (int)(threadIdx.x & 63u);
+    return (int)(uint32_t)wave_min_u64(lane < NT / 64 ? wmin[lane] : ~0ull);
+}
+
+// The members that member i (< pop) is crossed with, three distinct offsets in [1, P) from
+// one Philox block's words: they differ from i and from one another.
+struct Partners {
+    uint32_t a, b, c;
 };
 
-__device__ __forceinline__ void trial_fetch(const DeArgs& a, int i, uint32_t gen, Trial& T)
+__device__ __forceinline__ Partners partners(uint32_t rx, uint32_t ry, uint32_t rz, uint32_t P)
 {
-    const uint32_t P = (uint32_t)a.pop;
-    const u32x4 r = philox10(gen, (uint32_t)i, 0u, 0u, a.key0, a.key1);
-    // three distinct offsets in [1, P): partners differ from i and from one another
-    const uint32_t oa = 1u + below(r.x, P - 1u);
-    uint32_t ob = 1u + below(r.y, P - 2u);
+    const uint32_t oa = 1u + below(rx, P - 1u);
+    uint32_t ob = 1u + below(ry, P - 2u);
     ob += ob >= oa ? 1u : 0u;
-    uint32_t oc = 1u + below(r.z, P - 3u);
+    uint32_t oc = 1u + below(rz, P - 3u);
     const uint32_t lo = oa < ob ? oa : ob, hi = oa < ob ? ob : oa;
     oc += oc >= lo ? 1u : 0u;
     oc += oc >= hi ? 1u : 0u;
-    T.jr = (int)below(r.w, (uint32_t)a.dim);
-    const float* xi = a.x + (int64_t)i * a.dim;
-    const float* x0 = a.x + (int64_t)((i + oa) % P) * a.dim;
-    const float* x1 = a.x + (int64_t)((i + ob) % P) * a.dim;
-    const float* x2 = a.x + (int64_t)((i + oc) % P) * a.dim;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const bool in = j < a.dim;
-        T.xi[j] = in ? xi[j] : 0.0f;
-        T.x0[j] = in ? x0[j] : 0.0f;
-        T.x1[j] = in ? x1[j] : 0.0f;
-        T.x2[j] = in ? x2[j] : 0.0f;
-    }
-    T.c0 = philox10(gen, (uint32_t)i, 1u, 0u, a.key0, a.key1);   // crossover
-    T.c1 = philox10(gen, (uint32_t)i, 2u, 0u, a.key0, a.key1);
-    T.d0 = philox10(gen, (uint32_t)i, 3u, 0u, a.key0, a.key1);   // redraws
-    T.d1 = philox10(gen, (uint32_t)i, 4u, 0u, a.key0, a.key1);
+    return {oa, ob, oc};
 }
 
-// Its searched coordinates into t[0 .. dim) and the network's input row into
-// in[16] (trials, fixed inputs, zeros).
-__device__ __forceinline__ void trial_finish(const DeArgs& a, const Trial& T, int best, float* t,
-                                             float (&in)[16])
+// A coordinate of the trial: mutant, crossover, and the redraw of one outside [-1, 1].
+__device__ __forceinline__ float trial_coord(const DeArgs& a, float xi, float x0, float x1, float x2,
+                                             float xb, bool always, uint32_t uc, uint32_t ud)
 {
+    const float m = x0 + a.F * (xb - x0) + a.F * (x1 - x2);
+    const float v = unit_f(uc) < a.CR || always ? m : xi;
+    return v < -1.0f || v > 1.0f ? 2.0f * unit_f(ud) - 1.0f : v;
+}
+
+// The trial of member i by one lane, for the layered form: its searched coordinates into
+// t[0 .. dim) and the network's input row into in[16] (trials, fixed inputs, zeros).
+__device__ __forceinline__ void propose_member(const DeArgs& a, int i, int best, uint32_t gen,
+                                               float* t, float (&in)[16])
+{
+    const uint32_t P = (uint32_t)a.pop;
+    const u32x4 r = philox10(gen, (uint32_t)i, 0u, 0u, a.key0, a.key1);
+    const Partners o = partners(r.x, r.y, r.z, P);
+    const int jr = (int)below(r.w, (uint32_t)a.dim);     // it always crosses over
+    const float* xi = a.x + (int64_t)i * a.dim;
+    const float* x0 = a.x + (int64_t)((i + o.a) % P) * a.dim;
+    const float* x1 = a.x + (int64_t)((i + o.b) % P) * a.dim;
+    const float* x2 = a.x + (int64_t)((i + o.c) % P) * a.dim;
     const float* xb = a.x + (int64_t)best * a.dim;
+    const u32x4 c0 = philox10(gen, (uint32_t)i, 1u, 0u, a.key0, a.key1);   // crossover
+    const u32x4 c1 = philox10(gen, (uint32_t)i, 2u, 0u, a.key0, a.key1);
+    const u32x4 d0 = philox10(gen, (uint32_t)i, 3u, 0u, a.key0, a.key1);   // redraws
+    const u32x4 d1 = philox10(gen, (uint32_t)i, 4u, 0u, a.key0, a.key1);
     float tv[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
         tv[j] = 0.0f;
         if (j >= a.dim) continue;
-        const float m = T.x0[j] + a.F * (xb[j] - T.x0[j]) + a.F * (T.x1[j] - T.x2[j]);
-        const uint32_t uc = j < 4 ? pick_word(T.c0, j) : pick_word(T.c1, j - 4);
-        const bool cross = unit_f(uc) < a.CR || j == T.jr;
-        float v = cross ? m : T.xi[j];
-        if (v < -1.0f || v > 1.0f) {
-            const uint32_t ud = j < 4 ? pick_word(T.d0, j) : pick_word(T.d1, j - 4);
-            v = 2.0f * unit_f(ud) - 1.0f;
-        }
-        tv[j] = v;
-        t[j] = v;
+        tv[j] = trial_coord(a, xi[j], x0[j], x1[j], x2[j], xb[j], j == jr,
+                            j < 4 ? pick_word(c0, j) : pick_word(c1, j - 4),
+                            j < 4 ? pick_word(d0, j) : pick_word(d1, j - 4));
+        t[j] = tv[j];
     }
 #pragma unroll
     for (int k = 0; k < 16; ++k)
         in[k] = k < a.dim ? tv[k & 7] : (k < a.n_in ? a.fixed[k - a.dim] : 0.0f);
 }
 
-__device__ __forceinline__ void propose_member(const DeArgs& a, int i, int best, uint32_t gen,
-                                               float* t, float (&in)[16])
+// The same trial with a lane a coordinate, eight lanes a member, for the fused kernel: each
+// lane draws one Philox block, and the words it needs come from its member's lanes.
+struct CoordTrial {
+    uint32_t uc, ud;            // crossover and redraw words of the coordinate
+    int jr;                     // the coordinate that always crosses over
+    float xi, x0, x1, x2;
+};
+
+// threads that form trials: whole waves, so that every lane of a shuffle is there
+template <int M>
+constexpr int kTrialThreads = 8 * M < 64 ? 64 : 8 * M;
+
+__device__ __forceinline__ uint32_t word_of(const u32x4& o, int src, int word)
 {
-    Trial T;
-    trial_fetch(a, i, gen, T);
-    trial_finish(a, T, best, t, in);
+    const u32x4 v{(uint32_t)__shfl((int)o.x, src, 64), (uint32_t)__shfl((int)o.y, src, 64),
+                  (uint32_t)__shfl((int)o.z, src, 64), (uint32_t)__shfl((int)o.w, src, 64)};
+    return pick_word(v, word);
+}
+
+// (i < pop; lanes with j past the last coordinate repeat it)
+__device__ __forceinline__ void coord_fetch(const DeArgs& a, int i, int j, uint32_t gen, CoordTrial& T)
+{
+    const int jc = j < a.dim ? j : a.dim - 1;
+    const uint32_t P = (uint32_t)a.pop;
+    const int g = (int)(threadIdx.x & 56u);          // the member's first lane of the wave
+    // blocks: 0 the partners and the crossing coordinate, 1 and 2 crossover, 3 and 4 redraws
+    const u32x4 o = philox10(gen, (uint32_t)i, (uint32_t)(j < 4 ? j : 4), 0u, a.key0, a.key1);
+    const uint32_t rx = (uint32_t)__shfl((int)o.x, g, 64), ry = (uint32_t)__shfl((int)o.y, g, 64);
+    const uint32_t rz = (uint32_t)__shfl((int)o.z, g, 64), rw = (uint32_t)__shfl((int)o.w, g, 64);
+    T.uc = word_of(o, g + 1 + (j >> 2), j & 3);
+    T.ud = word_of(o, g + 3 + (j >> 2), j & 3);
+    const Partners p = partners(rx, ry, rz, P);
+    T.jr = (int)below(rw, (uint32_t)a.dim);
+    auto row = [&](uint32_t off) {                   // coordinate j of member (i + off) mod P
+        const uint32_t m = (uint32_t)i + off;
+        return a.x[(int64_t)(m >= P ? m - P : m) * a.dim + jc];
+    };
+    T.xi = row(0u);
+    T.x0 = row(p.a);
+    T.x1 = row(p.b);
+    T.x2 = row(p.c);
 }
 
 // Objective of one network output row y [n_out], reduced over the wave (every
@@ -211,7 +240,7 @@ __device__ __forceinline__ void select_member(const DeArgs& a, int i, float ft, 
 
 __global__ __launch_bounds__(256) void de_propose_kernel(DeArgs a, uint32_t gen)
 {
-    const int best = population_argmin<256>(a);     // of the previous generation
+    const int best = population_argmin<256>(a, first_key(a));     // of the previous generation
     const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     if (i >= a.pop) return;
     float in[16];
@@ -318,14 +347,16 @@ __device__ __forceinline__ const bf16* tile_fragments(const DeLayer& L, int t, i
     return L.w + ((int64_t)t * (L.kp / 16) * 64 + lane) * 8;
 }
 
-// One whole generation for 32 members per workgroup (see the file comment).
+// One whole generation for M members per workgroup (see the file comment).
 // Dynamic LDS: two activation buffers [32][lda] BF16, the output rows
 // [32][n_out + 4] FP32, the trials [32][8] FP32, the target [n_out], the
 // members' current objectives [32] and rows [32][8] FP32.
 // The fixed network shapes of the unrolled form (the surrogate networks): five
 // layers, 64 padded inputs, hidden layers 512 wide, 256 outputs.
 constexpr int kFixedLayers = 5, kLdaFixed = 512 + 8, kYsFixed = 256 + 4;
-constexpr int kAheadDe = 1;     // chunks in flight ahead of the products (4 KB a wave)
+constexpr int kAheadDe = 2;     // chunks in flight ahead of the products (4 KB a wave each; 150
+                                // generations of 64 members 3.87 ms with 1, 3.79 with 2, and
+                                // 4.08 with 3, at 126 registers)
 
 // The fixed shapes as one stream of weight chunks (four K steps, 4 KB per wave):
 // chunk 0 is layer 0's only chunk (K = 64), chunks 1 + 8 (l - 1) .. + 7 are layer
@@ -337,6 +368,16 @@ __device__ __forceinline__ const bf16* stream_chunk(const bf16* const (&wl)[kFix
     return g == 0 ? wl[0] : wl[1 + (g - 1) / kFixedChunks] + ((g - 1) % kFixedChunks) * 2048;
 }
 
+// The tile row of member u of a workgroup's M.  Accumulator r of a lane holds row 8 (r / 4) +
+// 4 (lane / 32) + r % 4, and the members' rows are those of r < M / 2: 0-15, 0-7, or 0, 1, 4
+// and 5, so that both halves of the wave share an epilogue evenly.
+template <int M>
+__device__ __forceinline__ int member_row(int u)
+{
+    static_assert(M == 16 || M == 8 || M == 4, "rows of M members");
+    return M == 4 ? (u & 1) + 4 * (u >> 1) : u;
+}
+
 // Layer L of the fixed shapes (bn: the bias of the lane's output column, loaded at
 // the kernel's start), its products unrolled over the chunk stream: chunk
 // g sits in buf[g % D] and is fetched D - 1 chunks ahead of its products, across
@@ -346,7 +387,7 @@ __device__ __forceinline__ const bf16* stream_chunk(const bf16* const (&wl)[kFix
 // so the wait before each chunk's products counts exactly the loads issued after
 // it (the output layer's eight idle waves skip it whole).  The same products in
 // the same K order as layer_products.
-template <int L, int D, int LDA, int YS>
+template <int L, int M, int D, int LDA, int YS>
 __device__ __forceinline__ void fixed_layer(const bf16* const (&wl)[kFixedLayers], float bn,
                                             bf16x8 (&buf)[D][4], bf16*& cur, bf16*& nxt,
                                             float* yrow, int t, int lane)
@@ -382,10 +423,8 @@ __device__ __forceinline__ void fixed_layer(const bf16* const (&wl)[kFixedLayers
                 if (!next_last || t < 8) fetch(gf);
             }
         }
-        // accumulator r holds row 8 (r / 4) + 4 (lane / 32) + r % 4: the members'
-        // rows 0-15 are r < 8
 #pragma unroll
-        for (int r = 0; r < 8; ++r) {
+        for (int r = 0; r < M / 2; ++r) {          // the members' rows
             const int m = 8 * (r / 4) + 4 * (lane >> 5) + (r % 4);
             if constexpr (kLastL) {
                 yrow[m * YS + n] = acc[r] + bn;
@@ -405,7 +444,7 @@ __device__ __forceinline__ void fixed_layer(const bf16* const (&wl)[kFixedLayers
 // fixed shapes, laid out by a fully unrolled forward), so that the epilogue's LDS
 // addresses are one base and immediate offsets; 0: any shape the fused kernel
 // takes, net.lda and n_out + 4 at run time.
-template <int LDA, int YS>
+template <int M, int LDA, int YS>
 __global__ __launch_bounds__(kFusedThreads) void de_generation_kernel(DeArgs a, DeNet net,
                                                                       uint32_t gen)
 {
@@ -419,13 +458,34 @@ __global__ __launch_bounds__(kFusedThreads) void de_generation_kernel(DeArgs a, 
     float* fcur = tgt + a.n_out;              // [kRows] the members' current objectives
     float* xown = fcur + kRows;               // [kRows][8] the members' current rows
     const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int row0 = (int)blockIdx.x * kMembers;
+    const int row0 = (int)blockIdx.x * M;
     constexpr int kChunk = 4;                // K steps per weight chunk
     const int t = wave;                      // the wave's output tile in every layer
     __builtin_assume(t < kFusedThreads / 64);   // every wave has a tile of a hidden layer
 
+    // every argument is asked for at once: one trip to memory, not one at each first use
+    asm volatile("" ::"s"(a.keys), "s"(a.target), "s"(a.f), "s"(a.x), "s"(a.x_next),
+                 "s"(a.keys_next), "s"(a.pop), "s"(a.n_out), "s"(a.dim), "s"(a.key0), "s"(a.key1), "s"(gen));
+    if constexpr (LDA > 0) {
+#pragma unroll
+        for (int l = 0; l < kFixedLayers; ++l) asm volatile("" ::"s"(net.L[l].w), "s"(net.L[l].b));
+    }
+    // the keys, the target, the members' current objectives and the trials' draws and
+    // partner rows go out first of all, so that their latencies overlap; a lane takes
+    // coordinate j of member u
+    const uint64_t key = first_key(a);
+    // (unconditional loads, clamped: a load under a branch is waited for at its end)
+    const float tg = a.target[tid < a.n_out ? tid : 0];
+    const float fc = a.f[tid < M && row0 + tid < a.pop ? row0 + tid : row0];
+    const int u = tid >> 3, j = tid & 7;
+    const bool own = u < M && row0 + u < a.pop;
+    const bool coord = own && j < a.dim;
+    CoordTrial T;
+    if (tid < kTrialThreads<M>) coord_fetch(a, own ? row0 + u : row0, j, gen, T);
+    __builtin_amdgcn_sched_barrier(0);
     // the fixed shapes: the wave's tiles of every layer, and a ring of kAheadDe + 1
-    // chunk buffers over the stream whose first chunks go out first of all
+    // chunk buffers over the stream, whose first chunks go out behind the loads above (loads return in
+    // order, so the trials do not wait for weights)
     constexpr int D = kAheadDe + 1;
     const bf16* wl[kFixedLayers];
     float bl[kFixedLayers];                  // the lane's output-column bias of every layer
@@ -434,7 +494,7 @@ __global__ __launch_bounds__(kFusedThreads) void de_generation_kernel(DeArgs a, 
 #pragma unroll
         for (int l = 0; l < kFixedLayers; ++l) {
             const int tl = l + 1 == kFixedLayers ? (t & 7) : t;
-            wl[l] = tile_fragments(net.L[l], tl, lane);
+            wl[l] = net.L[l].w + ((int64_t)tl * (l == 0 ? 4 : 32) * 64 + lane) * 8;
             bl[l] = net.L[l].b[32 * tl + (lane & 31)];
         }
 #pragma unroll
@@ -445,34 +505,31 @@ __global__ __launch_bounds__(kFusedThreads) void de_generation_kernel(DeArgs a, 
         }
     }
 
-    // the trials' draws and partner rows, the target and the members' current
-    // objectives go out before the argmin, so their latencies overlap
-    Trial T;
-    if (tid < kMembers && row0 + tid < a.pop) trial_fetch(a, row0 + tid, gen, T);
-    for (int b = tid; b < a.n_out; b += kFusedThreads) tgt[b] = a.target[b];
-    if (tid < kMembers) fcur[tid] = row0 + tid < a.pop ? a.f[row0 + tid] : 0.0f;
-    // the padding rows of both activation buffers hold zeros (16-byte stores; the
+    __builtin_amdgcn_sched_barrier(0);
+    // the other rows of both activation buffers hold zeros (16-byte stores; the
     // row stride lda is a multiple of 8)
-    for (int e = tid; e < (kRows - kMembers) * lda / 8; e += kFusedThreads) {
-        reinterpret_cast<uint4*>(act0 + kMembers * lda)[e] = make_uint4(0u, 0u, 0u, 0u);
-        reinterpret_cast<uint4*>(act1 + kMembers * lda)[e] = make_uint4(0u, 0u, 0u, 0u);
+    constexpr int kFirstZero = M == 4 ? 2 : M;
+    for (int e = tid; e < (kRows - kFirstZero) * lda / 8; e += kFusedThreads) {
+        reinterpret_cast<uint4*>(act0 + kFirstZero * lda)[e] = make_uint4(0u, 0u, 0u, 0u);
+        reinterpret_cast<uint4*>(act1 + kFirstZero * lda)[e] = make_uint4(0u, 0u, 0u, 0u);
     }
-    const int best = population_argmin<kFusedThreads>(a);   // of the previous generation
-    if (tid < kMembers) {
-        const int i = row0 + tid;
-        float in[16];
-        if (i < a.pop) {
-            trial_finish(a, T, best, trial + tid * 8, in);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) xown[tid * 8 + j] = T.xi[j];
-        } else {
-#pragma unroll
-            for (int k = 0; k < 16; ++k) in[k] = 0.0f;   // padding rows
+    if (tid < a.n_out) tgt[tid] = tg;                 // n_out <= 512
+    if (tid < M) fcur[tid] = fc;
+    const int best = population_argmin<kFusedThreads>(a, key);   // of the previous generation
+    if (u < M) {
+        float t_j = 0.0f;
+        if (coord)
+            t_j = trial_coord(a, T.xi, T.x0, T.x1, T.x2, a.x[(int64_t)best * a.dim + j], j == T.jr,
+                              T.uc, T.ud);
+        if (coord) {
+            trial[8 * u + j] = t_j;
+            xown[8 * u + j] = T.xi;
         }
-        bf16* r = act0 + tid * lda;
-#pragma unroll
-        for (int k = 0; k < 16; ++k) r[k] = (bf16)in[k];
-        for (int k = 16; k < net.L[0].kp; ++k) r[k] = (bf16)0.0f;
+        // the network's input row: trial, fixed inputs, zeros
+        bf16* r = act0 + member_row<M>(u) * lda;
+        r[j] = (bf16)(coord ? t_j : (own && j < a.n_in ? a.fixed[j - a.dim] : 0.0f));
+        for (int k = 8 + j; k < (LDA > 0 ? 64 : net.L[0].kp); k += 8)
+            r[k] = (bf16)(own && k < a.n_in ? a.fixed[k - a.dim] : 0.0f);
     }
     // wave w computes output tile w of every layer that is that wide.  The layer
     // loop is unrolled (layer l's descriptor at a fixed kernel-argument offset:
@@ -484,11 +541,11 @@ __global__ __launch_bounds__(kFusedThreads) void de_generation_kernel(DeArgs a, 
     if constexpr (LDA > 0) {
         lds_barrier();
         static_assert(kFixedLayers == 5, "the unrolled form is written for five layers");
-        fixed_layer<0, D, LDA, YS>(wl, bl[0], buf, cur, nxt, yrow, t, lane);
-        fixed_layer<1, D, LDA, YS>(wl, bl[1], buf, cur, nxt, yrow, t, lane);
-        fixed_layer<2, D, LDA, YS>(wl, bl[2], buf, cur, nxt, yrow, t, lane);
-        fixed_layer<3, D, LDA, YS>(wl, bl[3], buf, cur, nxt, yrow, t, lane);
-        fixed_layer<4, D, LDA, YS>(wl, bl[4], buf, cur, nxt, yrow, t, lane);
+        fixed_layer<0, M, D, LDA, YS>(wl, bl[0], buf, cur, nxt, yrow, t, lane);
+        fixed_layer<1, M, D, LDA, YS>(wl, bl[1], buf, cur, nxt, yrow, t, lane);
+        fixed_layer<2, M, D, LDA, YS>(wl, bl[2], buf, cur, nxt, yrow, t, lane);
+        fixed_layer<3, M, D, LDA, YS>(wl, bl[3], buf, cur, nxt, yrow, t, lane);
+        fixed_layer<4, M, D, LDA, YS>(wl, bl[4], buf, cur, nxt, yrow, t, lane);
     } else {
         bf16x8 pre[1][kChunk], alt[1][kChunk];
         if (t < net.L[0].out / 32) {
@@ -518,7 +575,7 @@ __global__ __launch_bounds__(kFusedThreads) void de_generation_kernel(DeArgs a, 
                 in_alt = layer_products<kChunk, 1>(cur, lda, w, L.kp, acc, pre, alt, wn, next);
                 const bool last = l + 1 == net.n_layers;
 #pragma unroll
-                for (int r = 0; r < 8; ++r) {      // the members' rows 0-15
+                for (int r = 0; r < M / 2; ++r) {      // the members' rows
                     const int m = 8 * (r / 4) + 4 * (lane >> 5) + (r % 4);
                     if (last) {
                         yrow[m * ys + n] = acc[0][r] + bn;
@@ -536,14 +593,28 @@ __global__ __launch_bounds__(kFusedThreads) void de_generation_kernel(DeArgs a, 
     }
 
     // objectives and selection: wave w takes member w of the workgroup
-    constexpr int kPerWave = kMembers / (kFusedThreads / 64);
-#pragma unroll
-    for (int q = 0; q < kPerWave; ++q) {
-        const int r = wave * kPerWave + q, i = row0 + r;
-        if (i >= a.pop) continue;
-        const float ft = member_objective(a, yrow + r * ys, tgt, lane);
-        select_member(a, i, ft, fcur[r], trial + r * 8, xown + r * 8, lane);
+    static_assert(M <= kFusedThreads / 64, "a wave a member");
+    if (wave < M && row0 + wave < a.pop) {
+        const float ft = member_objective(a, yrow + member_row<M>(wave) * ys, tgt, lane);
+        select_member(a, row0 + wave, ft, fcur[wave], trial + wave * 8, xown + wave * 8, lane);
     }
+}
+
+// Members of a workgroup for a population: as few as keep to 128 workgroups, half the CUs.
+// Every CU streams the whole weight set either way, and the epilogues are the members' share
+// of it; with all 256 CUs streaming the L2s are the limit.  150 generations: 1,024 members 3.96
+// ms at 8 a workgroup, 4.46 at 4 (256 workgroups), 4.38 at 16; 64 members 3.87 at 4, 4.26 at
+// 16; 2,048 members 4.44 at 16, 4.79 at 8.
+constexpr int kGroups = 128;
+int members_per_group(int pop) { return pop <= 4 * kGroups ? 4 : pop <= 8 * kGroups ? 8 : 16; }
+
+template <int M>
+hipError_t launch_fixed(const DeArgs& a, const DeNet& net, uint32_t gen, int lds_bytes,
+                        hipStream_t stream)
+{
+    hipLaunchKernelGGL((de_generation_kernel<M, kLdaFixed, kYsFixed>), dim3((unsigned)((a.pop + M - 1) / M)),
+                       dim3(kFusedThreads), (unsigned)lds_bytes, stream, a, net, gen);
+    return hipGetLastError();
 }
 
 }  // namespace
@@ -587,12 +658,13 @@ int de_fused_lds(const DeNet& net, int n_out)
 
 hipError_t de_fused_prepare(int lds_bytes)
 {
-    hipError_t e = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(de_generation_kernel<kLdaFixed, kYsFixed>),
-        hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
-    if (e == hipSuccess)
-        e = hipFuncSetAttribute(reinterpret_cast<const void*>(de_generation_kernel<0, 0>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
+    hipError_t e = hipSuccess;
+    for (const void* f : {reinterpret_cast<const void*>(de_generation_kernel<4, kLdaFixed, kYsFixed>),
+                          reinterpret_cast<const void*>(de_generation_kernel<8, kLdaFixed, kYsFixed>),
+                          reinterpret_cast<const void*>(de_generation_kernel<16, kLdaFixed, kYsFixed>),
+                          reinterpret_cast<const void*>(de_generation_kernel<kMembers, 0, 0>)})
+        if (e == hipSuccess)
+            e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
     return e;
 }
 
@@ -610,13 +682,16 @@ bool de_fixed_shapes(const DeNet& net, int n_out)
 hipError_t de_generation_fused(const DeArgs& a, const DeNet& net, uint32_t gen, int lds_bytes,
                                hipStream_t stream)
 {
-    const dim3 grid((unsigned)(a.pop_pad / kMembers)), block(kFusedThreads);
-    if (de_fixed_shapes(net, a.n_out))
-        hipLaunchKernelGGL((de_generation_kernel<kLdaFixed, kYsFixed>), grid, block,
-                           (unsigned)lds_bytes, stream, a, net, gen);
-    else
-        hipLaunchKernelGGL((de_generation_kernel<0, 0>), grid, block, (unsigned)lds_bytes, stream,
-                           a, net, gen);
+    if (de_fixed_shapes(net, a.n_out)) {
+        switch (members_per_group(a.pop)) {
+        case 4: return launch_fixed<4>(a, net, gen, lds_bytes, stream);
+        case 8: return launch_fixed<8>(a, net, gen, lds_bytes, stream);
+        default: return launch_fixed<16>(a, net, gen, lds_bytes, stream);
+        }
+    }
+    hipLaunchKernelGGL((de_generation_kernel<kMembers, 0, 0>), 
+                       dim3((unsigned)((a.pop + kMembers - 1) / kMembers)),
+                       dim3(kFusedThreads), (unsigned)lds_bytes, stream, a, net, gen);
     return hipGetLastError();
 }
 
