@@ -111,7 +111,7 @@ int         mcl_set_stream(void* ctx, void* hip_stream);
  * event-mode runs take larger clusters, up to 32768 (fixed-dt) or 65535 (event)
  * electrons and 65534 holes, in a global-memory form: holes and cell starts in a
  * scratch slice per resident workgroup (16 B per hole slot, 4 B per cell),
- * electrons in LDS while 16 B each fit; same results, lower speed.  Lab runs and
+ * electrons in LDS while they fit; same results, lower speed.  Lab runs and
  * mcl_run_fixed_dt_noalloc stay within this limit. */
 int         mcl_cluster_limits(const void* ctx, int32_t* max_electrons, int32_t* max_holes);
 /* Kernel tuning knobs of a context, applied to plans made afterwards.  Keys:

@@ -1453,11 +1453,13 @@ int mcl_run_fixed_dt_noalloc(void* ctx, const mcl_run_params* runs, int32_t n_ru
     const int g_cap = ((max_cells + 1 + 3) / 4) * 4;
     const int lds =
         mcl::cluster_lds_bytes(h_cap, g_cap, mcl::fixed_dt_electron_bytes(e_cap));
-    if (lds > c->max_lds)
+    // accepted at 16 B an electron (mcl_cluster_limits), though the layout takes fewer
+    const int counted = mcl::cluster_lds_bytes(h_cap, g_cap, 16 * e_cap);
+    if (counted > c->max_lds)
         return fail(c, MCL_ERANGE,
                     "cluster of %d electrons / %d holes needs %d B of LDS; a workgroup has %d B "
                     "(larger clusters run in global memory: use mcl_run_fixed_dt)",
-                    max_e, max_h, lds, c->max_lds);
+                    max_e, max_h, counted, c->max_lds);
     // descriptors and cluster map through a fixed host staging block, one chunk
     // at a time (each copied and waited for before the block is refilled)
     alignas(64) unsigned char stage[16384];
