@@ -39,6 +39,13 @@
 // slice, the electron arrays in LDS while they fit (e_lds) or after cstart in the
 // slice, persistent workgroups over a ticket; the wave's fences widen to
 // workgroup scope so its global stores complete before its lanes read them.
+//
+// What bounds it: the dependent chain of an event (the removal and its searches 34 % of a
+// cluster's cycles, rates and K 22 %, the selection 9 %) at two waves a SIMD (234 registers, 19.7
+// KB of LDS at 400 electrons), vector units busy 55 %.  Steps that are certainly capped are three
+// quarters of a ramp and are taken up to 64 at a time.  4096 x 400 electrons on the TL12 ramp: 3.52
+// ms with every step taken by itself, 2.92-2.99 now; 737 x 44 electrons 0.74 -> 0.26.  For three waves a
+// SIMD it spills 57 registers: 3.45 ms.
 #include "mc_common.h"
 
 namespace mcl {
