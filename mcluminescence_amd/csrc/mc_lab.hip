@@ -41,15 +41,18 @@
 //
 // The chain of steps bounds this kernel: one cluster issues some 300 vector instructions a
 // step, and it takes several waves on a SIMD to keep it busy.  So whatever depends on an index
-// only is evaluated for 64 steps or pairs at once, a lane each (the step draws, the pairs'
-// coordinates), the channel draws once per Philox block and not for each of its four steps, and
-// a step's independent exponentials and quotients in one evaluation, a lane each.  Holes and
-// electrons are arrays of coordinates, 12 bytes a hole slot and 18 an electron, without a table
-// for packing the slots again: 18 clusters a CU instead of 12 at 100 electrons.  45,056
-// clusters of 100 electrons (88 steps each): 4.37 ms with a Philox block per electron and step
-// and two per pair; 3.11 with the draws batched; 2.70 with the smaller layout (the vector
-// units then issue 95 % of the time).  Held to 96 registers for a fifth wave a SIMD it spills
-// and measures the same.
+// only is evaluated for many steps or pairs at once, a lane each: the step draws 64 at a time, the
+// channel draws once per Philox block and not for each of its four steps, a step's independent
+// exponentials and quotients in one evaluation.  Pairs are prepared 32 at a time, two lanes each:
+// coordinates and the electron's nearest hole, which then follows the holes (a new one is
+// compared with all pairs to come at once, a removed one searched for again) instead of one wave
+// scan and one w per pair.  Holes and electrons are arrays of coordinates, 12 bytes a hole slot
+// and 18 an electron, without a table for packing the slots again: 18 clusters a CU instead of
+// 12 at 100 electrons (16 by registers).  45,056 clusters of 100 electrons (88 steps each), whole
+// call: 4.37 ms with a Philox block per electron and step and two per pair; 3.11 with the draws
+// batched; 2.73 with the smaller layout; 2.59 with the pairs' searches batched (the vector units
+// then issue 92 % of the time).  Held to 96 registers for a fifth wave a SIMD it spilled and
+// measured the same.
 #include "mc_common.h"
 
 namespace mcl {
@@ -58,6 +61,10 @@ namespace {
 
 constexpr uint32_t kFillCtr = 0xFFFFFFFEu;
 constexpr uint32_t kSharedChanCtr = 0xFFFFFFFDu;
+
+// Pairs whose electrons' nearest holes are searched at once, two lanes each (of 77 pairs a
+// cluster 16 lanes of the last batch stay unused on average; with 64, a lane each, 32).
+constexpr int kFillBatch = 32;
 
 
 __device__ __forceinline__ double lab_exp1(uint32_t u)
@@ -197,9 +204,13 @@ __device__ __forceinline__ void run_cluster_lab(const LabArgs& a, const int c,
     constexpr int kChanRows = 8;
     uint32_t l_chan = 0u, ch_blk = 0xFFFFFFFFu;
     int ch_row0 = 0, ch_rows = 0;
-    // Lane j holds the coordinates of the pair of fill fb_base + j.
-    int fb_base = -kWave;
+    // Lanes j and j + 32 hold the pair of fill fb_base + j: its coordinates, and for its electron
+    // the nearest of the holes there are now (squared distance, slot, w), which follow the holes
+    // until the pair is used.
+    int fb_base = -kFillBatch;
     float f_ex = 0.f, f_ey = 0.f, f_ez = 0.f, f_hx = 0.f, f_hy = 0.f, f_hz = 0.f;
+    float f_d2 = __builtin_inff(), f_w = 0.f;
+    uint32_t f_at = kNoHole;
     const double dose = R.D / R.D0;
     const double T0 = R.T0_K, T_rate = R.T_rate, k_b = R.k_b;
     const bool no_dose = R.D == 0.0;
@@ -284,6 +295,9 @@ __device__ __forceinline__ void run_cluster_lab(const LabArgs& a, const int c,
                         hy[q] = vy;
                         hz[q] = vz;
                     }
+                    const int fn = (int)f_at - s0;
+                    if (fn >= 0 && fn < kWave && f_at != kNoHole)
+                        f_at = (uint32_t)(base + __popcll(m & ((1ull << fn) - 1)));
                     for (int e = lane; e < n_e; e += kWave) {
                         const int nn = (int)enn[e] - s0;
                         if (nn >= 0 && nn < kWave && enn[e] != kNoHole)
@@ -295,8 +309,8 @@ __device__ __forceinline__ void run_cluster_lab(const LabArgs& a, const int c,
                 n_hs = base;
                 if (n_hs >= h_cap) return false;
             }
-            if (fills - fb_base >= kWave) {
-                const uint32_t f = (uint32_t)(fills + lane);
+            if (fills - fb_base >= kFillBatch) {
+                const uint32_t f = (uint32_t)(fills + (lane & (kFillBatch - 1)));
                 const u32x4 oe = philox10(f, kFillCtr, prun, psim | MCL_TAG_GEOM_E, k0, k1);
                 const u32x4 oh = philox10(f, kFillCtr, prun, psim | MCL_TAG_GEOM_H, k0, k1);
                 f_ex = unit_coord(oe.x, R.side_nm);
@@ -306,6 +320,23 @@ __device__ __forceinline__ void run_cluster_lab(const LabArgs& a, const int c,
                 f_hy = unit_coord(oh.y, R.side_b_nm);
                 f_hz = unit_coord(oh.z, R.side_b_nm);
                 fb_base = fills;
+                // each of a pair's two lanes takes every other hole (its slots ascend, so a strictly
+                // smaller distance is the smaller key)
+                f_d2 = __builtin_inff();
+                f_at = kNoHole;
+                for (int s = lane / kFillBatch; s < n_hs; s += 2) {
+                    const float dx = hx[s] - f_ex, dy = hy[s] - f_ey, dz = hz[s] - f_ez;
+                    const float d2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
+                    const bool closer = d2 < f_d2;         // (a removed hole's is infinite)
+                    f_d2 = closer ? d2 : f_d2;
+                    f_at = closer ? (uint32_t)s : f_at;
+                }
+                const float od2 = __shfl_xor(f_d2, kFillBatch, kWave);
+                const uint32_t oat = (uint32_t)__shfl_xor((int)f_at, kFillBatch, kWave);
+                const bool other = od2 < f_d2 || (od2 == f_d2 && oat < f_at);
+                f_d2 = other ? od2 : f_d2;
+                f_at = other ? oat : f_at;
+                f_w = f_at == kNoHole ? 0.0f : w_of(__float_as_uint(f_d2), alpha_f);
             }
             const int jf = fills - fb_base;
             const float px = lane_value(f_ex, jf), py = lane_value(f_ey, jf),
@@ -313,17 +344,30 @@ __device__ __forceinline__ void run_cluster_lab(const LabArgs& a, const int c,
             const float nx = lane_value(f_hx, jf), ny = lane_value(f_hy, jf),
                         nz = lane_value(f_hz, jf);
             const int hs = n_hs;
+            // the new electron's nearest hole: before the new hole (reference) or all
+            uint32_t slot = lane_value(f_at, jf);
+            float w = lane_value(f_w, jf);
+            // the new hole (the last slot: it wins only when strictly closer)
             if (lane == jf) {
                 hx[hs] = f_hx;
                 hy[hs] = f_hy;
                 hz[hs] = f_hz;
             }
             wave_lds_fence();
-            // the new electron's nearest hole: before the new hole (reference) or all
-            const uint64_t key = lab_nearest(hole, exact ? hs + 1 : hs, px, py, pz, lane);
-            uint32_t slot;
-            float w;
-            nn_from_key(key, alpha_f, slot, w);
+            {
+                const float dx = nx - f_ex, dy = ny - f_ey, dz = nz - f_ez;
+                const float d2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
+                const bool closer = d2 < f_d2;
+                if (ballot(closer) != 0) {
+                    f_d2 = closer ? d2 : f_d2;
+                    f_at = closer ? (uint32_t)hs : f_at;
+                    f_w = closer ? w_of(__float_as_uint(d2), alpha_f) : f_w;
+                }
+            }
+            if (exact) {
+                slot = lane_value(f_at, jf);
+                w = lane_value(f_w, jf);
+            }
             if (exact) {
                 // existing electrons: the new hole wins only when strictly closer
                 for (int e = lane; e < n_e; e += kWave) {
@@ -465,6 +509,19 @@ __device__ __forceinline__ void run_cluster_lab(const LabArgs& a, const int c,
                     }
                 }
             }
+            // and so are the pairs to come
+            uint64_t mf = ballot(f_at == hw && (lane & (kFillBatch - 1)) >= fills - fb_base) &
+                          ((1ull << kFillBatch) - 1);
+            while (mf != 0) {
+                const int j = (int)__builtin_ctzll(mf);
+                mf &= mf - 1;
+                const uint64_t key = lab_nearest(hole, n_hs, lane_value(f_ex, j), lane_value(f_ey, j),
+                                                 lane_value(f_ez, j), lane);
+                if ((lane & (kFillBatch - 1)) == j) {
+                    f_d2 = __uint_as_float((uint32_t)(key >> 32));
+                    nn_from_key(key, alpha_f, f_at, f_w);
+                }
+            }
             wave_lds_fence();
             // legacy retrapping: a new pair after the recombination
             if (retrap && (uint64_t)lane_value(l_rw, js) < R.retrap_thr && !add_pair(true)) {
@@ -491,7 +548,7 @@ __device__ __forceinline__ void run_cluster_lab(const LabArgs& a, const int c,
     }
 }
 
-__global__ __launch_bounds__(64) void lab_kernel(LabArgs a)
+__global__ __launch_bounds__(64, 4) void lab_kernel(LabArgs a)
 {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     if ((int)blockIdx.x < a.n_clusters) run_cluster_lab(a, (int)blockIdx.x, lds_raw);
