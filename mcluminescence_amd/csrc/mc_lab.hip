@@ -50,7 +50,7 @@
 // and 18 an electron, without a table for packing the slots again: 18 clusters a CU instead of
 // 12 at 100 electrons (16 by registers).  45,056 clusters of 100 electrons (88 steps each), whole
 // call: 4.37 ms with a Philox block per electron and step and two per pair; 3.11 with the draws
-// batched; 2.73 with the smaller layout; 2.59 with the pairs' searches batched (the vector units
+// batched; 2.73 with the smaller layout; 2.50 with the pairs' searches batched (the vector units
 // then issue 92 % of the time).  Held to 96 registers for a fifth wave a SIMD it spilled and
 // measured the same.
 #include "mc_common.h"
@@ -324,6 +324,7 @@ __device__ __forceinline__ void run_cluster_lab(const LabArgs& a, const int c,
                 // smaller distance is the smaller key)
                 f_d2 = __builtin_inff();
                 f_at = kNoHole;
+#pragma unroll 4        // (four trips' reads in flight)
                 for (int s = lane / kFillBatch; s < n_hs; s += 2) {
                     const float dx = hx[s] - f_ex, dy = hy[s] - f_ey, dz = hz[s] - f_ez;
                     const float d2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
