@@ -18,7 +18,7 @@
 //                        (kNever: in none)
 //   lst        [e_cap + 64]  slots gathered from their rows: each wave's from its own
 //                        rows' first entry on, a light step's in the last 64
-//   xch        [2 NW + 5] (NW > 1) per-wave values exchanged between the waves, the
+//   xch        [4 NW + 5] (NW > 1) per-wave values exchanged between the waves, the
 //                        persistent launch's ticket, and what wave 0 publishes
 //
 // A cluster too large for that (GM: the global-memory form) keeps hole and
@@ -135,9 +135,11 @@ __device__ __forceinline__ void wave_sync()
 // Simulate cluster c from its geometry to its last step with NW wavefronts, all
 // state in lds_raw (GM: holes and cell starts, and the electron arrays unless
 // a.e_lds, in the workgroup's scratch slice).  Every branch that holds a
-// workgroup barrier depends only on values all waves share (the window, n_live,
-// n_slots, what wave 0 publishes, and results of the exchanges).  WIDE: the build
-// that searches wider blocks before every hole (far_search_wave).
+// workgroup barrier depends only on values all waves share: launch constants, results
+// of the exchanges, what wave 0 publishes, and what follows from these alone (the window,
+// n_live, n_slots, steps).  rowm is none of them: other waves write it while a wave
+// reads it.  WIDE: the build that searches wider blocks before every hole
+// (far_search_wave).
 template <int NW, bool GM, bool WIDE>
 __device__ __forceinline__ void run_cluster(const LaunchArgs& a, const int c,
                                             unsigned char* lds_raw)
@@ -408,12 +410,22 @@ __device__ __forceinline__ void run_cluster(const LaunchArgs& a, const int c,
         return (uint64_t)pick_word(rr, word) * To < (Tn << 32);
     };
     // Per-wave values between the waves (NW > 1): lane 0 of each wave publishes
-    // v, one workgroup barrier, then every wave reads all NW values.  Consecutive
-    // exchanges alternate between two slots of xch and each holds a barrier, so a
-    // slot is rewritten only after every wave has read it.
+    // v (exchange2: and v2, at NW), one workgroup barrier, then every wave reads all NW
+    // values.  Consecutive exchanges alternate between two slots of xch and each holds
+    // a barrier, so a slot is rewritten only after every wave has read it.
     int xph = 0;
+    auto exchange2 = [&](uint32_t v, uint32_t v2) -> const uint32_t* {
+        uint32_t* slot = xch + (xph & 1) * (2 * NW);
+        if (lane == 0) {
+            slot[wv] = v;
+            slot[NW + wv] = v2;
+        }
+        __syncthreads();
+        ++xph;
+        return slot;
+    };
     auto exchange = [&](uint32_t v) -> const uint32_t* {
-        uint32_t* slot = xch + (xph & 1) * NW;
+        uint32_t* slot = xch + (xph & 1) * (2 * NW);
         if (lane == 0) slot[wv] = v;
         __syncthreads();
         ++xph;
@@ -716,7 +728,7 @@ __device__ __forceinline__ void run_cluster(const LaunchArgs& a, const int c,
 
     // ---- windows (the step loop, simulate.py:51-92) ------------------------------
     // (NW > 1) what wave 0 publishes: {heavy step or kNever, n_live, steps (two words)}
-    uint32_t* const pub = xch + 2 * NW + 1;
+    uint32_t* const pub = xch + 4 * NW + 1;
     while (nb0 < step_limit && n_live > 0) {
         const int w_len = min(kWindow, step_limit - nb0);
         if (nb0 == 0 || ramp || w_len != len) {
@@ -749,6 +761,7 @@ __device__ __forceinline__ void run_cluster(const LaunchArgs& a, const int c,
             __syncthreads();
         }
         // scan: rows wv, wv + NW, ...
+        uint64_t steps = 0;              // steps of the window that may have candidates
         for (int r = wv; r < rows; r += NW) {
             const int p = r * kWave + lane;
             const uint32_t st = p < n_slots ? est[p] : kDeadSlot;
@@ -758,26 +771,39 @@ __device__ __forceinline__ void run_cluster(const LaunchArgs& a, const int c,
                 first_fire(st != kDeadSlot && (st >> 16) != kNoHole, st & 0xFFFFu, w, 0, f);
             nf[p] = (uint8_t)f;
             if (lane == 0) rowm[r] = m;
+            steps |= m;
         }
-        if constexpr (NW == 1) wave_sync<GM>();
-        else __syncthreads();
+        if constexpr (NW == 1) {
+            wave_sync<GM>();
+        } else {
+            // (each wave's from its own rows: a read of the others' rowm here would race with
+            // their searches ahead, and with the next window's scan when this one has no events)
+            const uint32_t* x = exchange2((uint32_t)steps, (uint32_t)(steps >> 32));
+            uint32_t lo = 0, hi = 0;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) {
+                lo |= x[w];
+                hi |= x[NW + w];
+            }
+            steps = ((uint64_t)uniform(hi) << 32) | uniform(lo);
+        }
 
         // Sub-windows of kSub steps.  While wave 0 takes the events of one, the others
         // search ahead for the next one with events (they touch only electrons that
         // fire there, wave 0 only those that fire now).
-        uint64_t steps = 0;              // steps of the window that may have candidates
+        // (wave 0, whose steps takes in what the other waves' searches add to rowm)
         auto all_rows = [&](int above) {
             uint64_t s = 0;
             for (int r = lane; r < rows; r += kWave) s |= (uint64_t)rowm[r];
             steps = ((uint64_t)wave_or_u32((uint32_t)(s >> 32)) << 32) | wave_or_u32((uint32_t)s);
             steps &= above >= kWindow ? 0ull : ~0ull << above;
         };
-        all_rows(0);
         uint32_t searched = 0;           // sub-windows searched ahead
         for (int j = 0; j < kWindow / kSub && n_live > 0; ++j) {
             const uint64_t sub = ((1ull << kSub) - 1ull) << (j * kSub);
             if ((steps & sub) == 0) continue;
-            // (from steps, which every wave has alike here: searched decides on a barrier)
+            // (from steps, which every wave has alike here: the exchange's at first, then what
+            // wave 0 published; searched decides on a barrier)
             int next = -1;               // the next sub-window with events, to search ahead
             if constexpr (NW > 1) {
                 const uint64_t rest = j + 1 < kWindow / kSub ? steps & (~0ull << ((j + 1) * kSub)) : 0ull;
@@ -981,7 +1007,7 @@ __global__ __launch_bounds__(NW * 64, 2) void fixed_dt_mw_kernel(LaunchArgs a)
     uint32_t* const ticket =
         (GM ? (uint32_t*)lds_raw
             : (uint32_t*)(lds_raw + 16 * a.h_cap + 4 * a.g_cap +
-                          fixed_dt_electron_bytes(a.e_cap))) + 2 * NW;
+                          fixed_dt_electron_bytes(a.e_cap))) + 4 * NW;
     for (;;) {
         if (threadIdx.x == 0) *ticket = atomicAdd(a.queue, 1u);
         __syncthreads();

@@ -167,11 +167,11 @@ inline int grid_dim(int n_h, double holes_per_cell)
 constexpr int kWideGrid = 9;
 
 // LDS beyond cluster_lds_bytes for a workgroup of `waves` wavefronts: the
-// per-wave exchange slots (2 x waves words), the persistent ticket and the four
+// per-wave exchange slots (2 x 2 x waves words), the persistent ticket and the four
 // words wave 0 publishes.
 __host__ __device__ constexpr int fixed_dt_waves_lds(int waves)
 {
-    return waves > 1 ? ((4 * (2 * waves + 5) + 15) / 16) * 16 : 0;
+    return waves > 1 ? ((4 * (4 * waves + 5) + 15) / 16) * 16 : 0;
 }
 
 // waves = wavefronts per cluster (1, 2, 4 or 8); lds_bytes = cluster_lds_bytes of the
