@@ -553,21 +553,27 @@ int mcl_mlp_create(void* ctxp, const mcl_mlp_desc* desc, void** out)
         TRY(dalloc(m, &m->loss_tmp, 1));
         HIP_TRY(c, hipEventCreate(&m->ev0));
         HIP_TRY(c, hipEventCreate(&m->ev1));
-        // the fused kernels' copies of the weights
+        // the fused kernels' copies of the weights, zeros as the masters are
         if (m->fused_ok) {
             int64_t nwf = 0;
             for (const Layer& s : m->L) nwf += (int64_t)s.out * s.kp;
             TRY(dalloc(m, &m->wf, nwf));
+            HIP_TRY(c, hipMemset(m->wf, 0, nwf * sizeof(bf16)));
             int64_t off = 0;
             for (size_t l = 0; l < m->L.size(); ++l) {
                 const Layer& s = m->L[l];
                 m->fnet.L[l].w = m->wf + off;
                 off += (int64_t)s.out * s.kp;
                 bf16* wtf = nullptr;
-                if (m->train_fused && l > 0) TRY(dalloc(m, &wtf, (int64_t)s.out * s.kp));
+                if (m->train_fused && l > 0) {
+                    TRY(dalloc(m, &wtf, (int64_t)s.out * s.kp));
+                    HIP_TRY(c, hipMemset(wtf, 0, (int64_t)s.out * s.kp * sizeof(bf16)));
+                }
                 m->wtf.push_back(wtf);
             }
         }
+        // (the first call may be on a stream that does not wait for the null stream's fills)
+        HIP_TRY(c, hipStreamSynchronize(nullptr));
         (void)hipGetLastError();
         return MCL_OK;
     };
