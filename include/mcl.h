@@ -194,7 +194,9 @@ int  mcl_plan_info_get(const void* plan, mcl_plan_info* info);
 int  mcl_plan_launch(void* plan, uint32_t* counts_dev, uint64_t* live_steps_dev);
 
 /* Work done by the last launch of a plan, summed over its clusters (waits for
- * the launch): the algorithmic units behind throughput and roofline figures. */
+ * the launch): the algorithmic units behind throughput and roofline figures.  The
+ * same launch counts the same work every time; distance_evals alone depends on the
+ * knobs too (the hole grid, the wavefronts of a cluster). */
 typedef struct mcl_work {
     uint64_t live_electron_steps;  /* live electrons summed over every simulated step   */
     uint64_t distance_evals;       /* electron-hole squared distances evaluated          */

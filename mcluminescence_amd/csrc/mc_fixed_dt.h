@@ -57,12 +57,20 @@
 //             without a workgroup barrier.  (Sharing steps of more than 12 or of more
 //             than one among the waves measured slower: 1000 x 1500 decays 2.12 ms at
 //             64, 2.28 at 12, 2.65 at 1; 250 x 8000 in scratch memory 14.9, 16.2, 18.2.)
-//   ahead     while wave 0 takes the events of a sub-window (8 steps), the other waves
-//             search for the electrons that fire in the next one with events and whose
-//             hole is gone already, so that few searches are left to the steps
-//             themselves (32 x 2000 glow 2.63 -> 2.27 ms, 64 x 1000 tunnelling ramps 2.40
-//             -> 1.92).  One wave alone has nothing to overlap (the decay measured 2 %
-//             slower with it) and leaves every search to its step.
+//   together  with several waves, the electrons that fire in the next steps with events and
+//             whose hole is gone already are searched by all waves, each its own rows, between
+//             two barriers, so that few searches are left to the steps themselves.  Such a
+//             search keeps wave 0 waiting about as long as two steps that search for
+//             themselves, so it is made every 11 / v steps with candidates, v the stale ones
+//             of a step as the steps before and the share of the holes that are gone let
+//             expect (11 / sqrt(v) above one, where a step's own search takes several
+//             passes; at least every 4).  16 x 500 glow 1.14 ms, 64 x 1000 tunnelling ramps 1.86,
+//             500 uneven sets 1.96, 32 x 2000 glow 3.12, 64 isothermal curves 1.94; every 8
+//             steps with candidates 1.17, 2.07, 2.03, 3.09 and 1.95; by the other waves beside
+//             wave 0's events, none waiting, 1.13, 1.91, 1.81, 2.87 and 2.03, but then the
+//             waves' timing decides which searches are made, and with it the number of distances
+//             evaluated.  One wave alone leaves every search to its step (the decay measured
+//             2 % slower with them).
 //   heavy     a step with more candidates: every wave takes the candidates of its
 //             own rows, gathered 64 to a chunk, and they meet at barriers (winners,
 //             each retry round).
@@ -112,7 +120,11 @@ namespace mcl {
 
 constexpr int kWindow = 64;            // steps of a window (a multiple of 4; rowm's bits)
 constexpr uint32_t kNever = 255u;      // nf: no firing step in the window
-constexpr int kLogSub = 3, kSub = 1 << kLogSub;   // steps of a sub-window (searched ahead)
+constexpr uint32_t kSearch = 254u;     // published in place of a heavy step: search all rows
+// Steps with candidates between two searches of all rows (see "together" above): at first, at
+// least, and the numerator of the rule.
+constexpr int kFirstEvents = 8, kMinEvents = 4;
+constexpr float kEventsPerStale = 11.0f;
 // Rows with at most this many live electrons are scanned four electrons at a time,
 // 16 lanes each, instead of one electron a lane.
 constexpr int kGroupMax = 16;
@@ -351,27 +363,24 @@ __device__ __forceinline__ void run_cluster(const LaunchArgs& a, const int c,
         if (__popcll(m) <= kGroupMax) return group_scan(m, o, w, from, f);
         return lane_scan(live, o, w, from, f);
     };
-    // The slots of rows [r_lo, r_hi) that fire in the 2^lg steps from rel on (a multiple
-    // of 2^lg), to out (at most cap of them); returns how many.  A lane reads eight
-    // slots' nf at once, so one trip covers eight rows, and the row masks skip eight
-    // rows without one.
-    auto gather = [&](int rel, int lg, int r_lo, int r_hi, uint16_t* out, int cap) -> int {
-        const uint32_t bits = (1u << (1 << lg)) - 1u;          // lg <= 3
-        const uint32_t keep = ((0xFFu << lg) & 0xFFu) * 0x01010101u;
-        const uint32_t pat = (uint32_t)rel * 0x01010101u;
+    // The slots of rows [r_lo, r_hi) that fire in the n steps from rel on, to out (at most
+    // cap of them); returns how many.  A lane reads eight slots' nf at once, so one trip
+    // covers eight rows, and the row masks skip eight rows without one.
+    auto gather = [&](int rel, int n, int r_lo, int r_hi, uint16_t* out, int cap) -> int {
+        const uint64_t bits = (~0ull >> (kWindow - n)) << rel;
         int k = 0;
         for (int r0 = r_lo; r0 < r_hi; r0 += kWave) {
             const uint64_t rm = r0 + lane < r_hi ? (uint64_t)rowm[r0 + lane] : 0ull;
-            const uint64_t ev = ballot(((uint32_t)(rm >> rel) & bits) != 0u);
+            const uint64_t ev = ballot((rm & bits) != 0ull);
             for (int r8 = 0; r8 < kWave && (ev >> r8) != 0; r8 += 8) {
                 if (((ev >> r8) & 0xFFull) == 0) continue;
                 const int p0 = (r0 + r8) * kWave + 8 * lane;
                 const uint2 v = p0 < r_hi * kWave ? *(const uint2*)(nf + p0)
                                                   : make_uint2(~0u, ~0u);      // (kNever bytes)
-                const uint32_t xa = (v.x ^ pat) & keep, xb = (v.y ^ pat) & keep;
 #pragma unroll
                 for (int t = 0; t < 8; ++t) {
-                    const bool is = (((t < 4 ? xa : xb) >> (8 * (t & 3))) & 0xFFu) == 0u;
+                    const uint32_t f = ((t < 4 ? v.x : v.y) >> (8 * (t & 3))) & 0xFFu;
+                    const bool is = f - (uint32_t)rel < (uint32_t)n;
                     const uint64_t m = ballot(is);
                     if (m == 0) continue;
                     const int q = k + lanes_below(m);
@@ -574,7 +583,7 @@ __device__ __forceinline__ void run_cluster(const LaunchArgs& a, const int c,
             nr = min(rows, r_lo + per) - r_lo;
         }
         uint16_t* const my = lst + r_lo * kWave;
-        const int k = gather(rel, 0, r_lo, r_lo + nr, my, nr * kWave);
+        const int k = gather(rel, 1, r_lo, r_lo + nr, my, nr * kWave);
         nr = (k + kWave - 1) / kWave;    // chunks from here on
         uint64_t cand = 0;               // per chunk: this lane's candidate claims a hole
         uint32_t wins = 0, step_wins = 0;
@@ -687,14 +696,14 @@ __device__ __forceinline__ void run_cluster(const LaunchArgs& a, const int c,
         return step_wins;
     };
 
-    // The electrons of rows [r_lo, r_hi) that fire in sub-window j and whose nearest hole
-    // is gone already: searched now, together, instead of one step after the other.
-    // Exact: the hole found is no farther than the one a search in the firing step
+    // The electrons of rows [r_lo, r_hi) that fire in the n steps from rel0 on and whose
+    // nearest hole is gone already: searched now, together, instead of one step after the
+    // other.  Exact: the hole found is no farther than the one a search in the firing step
     // would find, and is that one if it still lives then (else it is searched again
     // there); an electron whose draw fails against the new threshold is scanned again.
-    auto pre_search = [&](int j, int r_lo, int r_hi) {
+    auto pre_search = [&](int rel0, int n_rel, int r_lo, int r_hi) {
         uint16_t* const my = lst + r_lo * kWave;
-        const int k = gather(j * kSub, kLogSub, r_lo, r_hi, my, (r_hi - r_lo) * kWave);
+        const int k = gather(rel0, n_rel, r_lo, r_hi, my, (r_hi - r_lo) * kWave);
         for (int c0 = 0; c0 < k; c0 += kWave) {
             const bool is = c0 + lane < k;
             const int p = is ? (int)my[c0 + lane] : 0;
@@ -727,8 +736,10 @@ __device__ __forceinline__ void run_cluster(const LaunchArgs& a, const int c,
     };
 
     // ---- windows (the step loop, simulate.py:51-92) ------------------------------
-    // (NW > 1) what wave 0 publishes: {heavy step or kNever, n_live, steps (two words)}
+    // (NW > 1) what wave 0 publishes: {heavy step, kSearch or kNever (the window is done),
+    // n_live, and the first step and end of the search; at a window's end `events`}
     uint32_t* const pub = xch + 4 * NW + 1;
+    int events = kFirstEvents;           // steps with candidates between searches of all rows
     while (nb0 < step_limit && n_live > 0) {
         const int w_len = min(kWindow, step_limit - nb0);
         if (nb0 == 0 || ramp || w_len != len) {
@@ -760,9 +771,10 @@ __device__ __forceinline__ void run_cluster(const LaunchArgs& a, const int c,
             rows = (n_slots + kWave - 1) / kWave;
             __syncthreads();
         }
-        // scan: rows wv, wv + NW, ...
+        // scan: the wave's own rows
+        const int per = (rows + NW - 1) / NW, my_lo = min(rows, wv * per), my_hi = min(rows, my_lo + per);
         uint64_t steps = 0;              // steps of the window that may have candidates
-        for (int r = wv; r < rows; r += NW) {
+        for (int r = my_lo; r < my_hi; ++r) {
             const int p = r * kWave + lane;
             const uint32_t st = p < n_slots ? est[p] : kDeadSlot;
             const float w = p < n_slots ? ew[p] : 0.0f;
@@ -777,7 +789,7 @@ __device__ __forceinline__ void run_cluster(const LaunchArgs& a, const int c,
             wave_sync<GM>();
         } else {
             // (each wave's from its own rows: a read of the others' rowm here would race with
-            // their searches ahead, and with the next window's scan when this one has no events)
+            // the next window's scan when this one has no events)
             const uint32_t* x = exchange2((uint32_t)steps, (uint32_t)(steps >> 32));
             uint32_t lo = 0, hi = 0;
 #pragma unroll
@@ -788,89 +800,88 @@ __device__ __forceinline__ void run_cluster(const LaunchArgs& a, const int c,
             steps = ((uint64_t)uniform(hi) << 32) | uniform(lo);
         }
 
-        // Sub-windows of kSub steps.  While wave 0 takes the events of one, the others
-        // search ahead for the next one with events (they touch only electrons that
-        // fire there, wave 0 only those that fire now).
-        // (wave 0, whose steps takes in what the other waves' searches add to rowm)
+        // The events: wave 0 takes the steps one after another; the other waves wait until it
+        // publishes a heavy step or a search of all rows, and take part in it.  (steps is
+        // wave 0's alone from here on.)
         auto all_rows = [&](int above) {
             uint64_t s = 0;
             for (int r = lane; r < rows; r += kWave) s |= (uint64_t)rowm[r];
             steps = ((uint64_t)wave_or_u32((uint32_t)(s >> 32)) << 32) | wave_or_u32((uint32_t)s);
             steps &= above >= kWindow ? 0ull : ~0ull << above;
         };
-        uint32_t searched = 0;           // sub-windows searched ahead
-        for (int j = 0; j < kWindow / kSub && n_live > 0; ++j) {
-            const uint64_t sub = ((1ull << kSub) - 1ull) << (j * kSub);
-            if ((steps & sub) == 0) continue;
-            // (from steps, which every wave has alike here: the exchange's at first, then what
-            // wave 0 published; searched decides on a barrier)
-            int next = -1;               // the next sub-window with events, to search ahead
-            if constexpr (NW > 1) {
-                const uint64_t rest = j + 1 < kWindow / kSub ? steps & (~0ull << ((j + 1) * kSub)) : 0ull;
-                if (rest != 0) next = (int)__builtin_ctzll(rest) / kSub;
-                if (next >= 0 && ((searched >> next) & 1u) != 0u) next = -1;
-            }
-            if (NW > 1 && ((searched >> j) & 1u) == 0u) {
-                const int per = (rows + NW - 1) / NW;
-                const int lo = min(rows, wv * per);
-                pre_search(j, lo, min(rows, lo + per));
-                if constexpr (NW > 1) __syncthreads();
-                if (wv == 0) all_rows(j * kSub);
-            }
-            bool ahead = false;
-            for (;;) {
-                uint32_t heavy = kNever;
+        // the step after the next `events` of the mask
+        auto events_end = [&](uint64_t m) -> int {
+            for (int i = 0; i < events && m != 0; ++i) m &= m - 1;
+            return m != 0 ? (int)__builtin_ctzll(m) : kWindow;
+        };
+        int n_ev = 0, n_cand = 0;        // light steps and candidates since the last search
+        auto next_events = [&]() {
+            if (n_ev == 0) return;
+            const float v = (float)n_cand * (float)(n_e0 - n_live) / ((float)n_ev * (float)n_h);
+            events = (int)fminf(fmaxf(kEventsPerStale / (v < 1.0f ? v : __builtin_sqrtf(v)),
+                                      (float)kMinEvents), (float)kWindow);
+            n_ev = 0;
+            n_cand = 0;
+        };
+        uint32_t todo = steps != 0 ? kSearch : kNever;
+        int from = steps != 0 ? (int)__builtin_ctzll(steps) : 0, to = events_end(steps);
+        while (todo != kNever) {
+            if (todo != kSearch) {
+                const uint32_t w = heavy_step((int)todo);
                 if (wv == 0) {
-                    while ((steps & sub) != 0) {
-                        const int rel = __builtin_ctzll(steps);
-                        const int k = gather(rel, 0, 0, rows, lst + e_cap, kWave);
-                        if (k > kWave) {
-                            heavy = (uint32_t)rel;
-                            break;
-                        }
-                        steps &= steps - 1;
-                        if (k == 0) continue;
-                        steps |= light_step(rel, lane < k, lane < k ? (int)lst[e_cap + lane] : 0);
-                        if (n_live == 0) {
-                            steps = 0;
-                            break;
-                        }
-                    }
-                } else if (!ahead && next >= 0) {
-                    const int per = (rows + NW - 2) / (NW > 1 ? NW - 1 : 1);
-                    const int lo = min(rows, (wv - 1) * per);
-                    pre_search(next, lo, min(rows, lo + per));
-                }
-                ahead = true;
-                if constexpr (NW > 1) {
-                    if (tid == 0) {
-                        pub[0] = heavy;
-                        pub[1] = (uint32_t)n_live;
-                    }
-                    __syncthreads();
-                    heavy = uniform(pub[0]);
-                    n_live = (int)uniform(pub[1]);
-                }
-                if (heavy == kNever) break;
-                const uint32_t w = heavy_step((int)heavy);
-                if (wv == 0) {
-                    finish_step(nb0 + (int)heavy, w);
-                    all_rows((int)heavy + 1);
+                    finish_step(nb0 + (int)todo, w);
+                    all_rows((int)todo + 1);
                     if (n_live == 0) steps = 0;
                 }
+            } else if constexpr (NW > 1) {
+                pre_search(from, to - from, my_lo, my_hi);
+                __syncthreads();
+                if (wv == 0) all_rows(from);
             }
-            if constexpr (NW > 1) {
-                if (next >= 0) searched |= 1u << next;
-                // the steps left, with what the searches ahead moved
-                if (wv == 0) {
-                    all_rows((j + 1) * kSub);
-                    if (lane == 0) {
-                        pub[2] = (uint32_t)steps;
-                        pub[3] = (uint32_t)(steps >> 32);
+            todo = kNever;
+            if (wv == 0) {
+                while (steps != 0) {
+                    const int rel = __builtin_ctzll(steps);
+                    if (NW > 1 && rel >= to) {
+                        next_events();
+                        todo = kSearch;
+                        from = rel;
+                        to = events_end(steps);
+                        break;
+                    }
+                    const int k = gather(rel, 1, 0, rows, lst + e_cap, kWave);
+                    if (k > kWave) {
+                        todo = (uint32_t)rel;
+                        break;
+                    }
+                    steps &= steps - 1;
+                    n_ev += 1;
+                    n_cand += k;
+                    if (k == 0) continue;
+                    steps |= light_step(rel, lane < k, lane < k ? (int)lst[e_cap + lane] : 0);
+                    if (n_live == 0) {
+                        steps = 0;
+                        break;
                     }
                 }
+            }
+            if constexpr (NW > 1) {
+                if (todo == kNever) {    // the window is done: `events` for the next one
+                    next_events();
+                    to = events;
+                }
+                if (tid == 0) {
+                    pub[0] = todo;
+                    pub[1] = (uint32_t)n_live;
+                    pub[2] = (uint32_t)from;
+                    pub[3] = (uint32_t)to;
+                }
                 __syncthreads();
-                steps = ((uint64_t)uniform(pub[3]) << 32) | uniform(pub[2]);
+                todo = uniform(pub[0]);
+                n_live = (int)uniform(pub[1]);
+                from = (int)uniform(pub[2]);
+                to = (int)uniform(pub[3]);
+                if (todo == kNever) events = to;
             }
         }
         nb0 += len;

@@ -1,7 +1,7 @@
 """The fixed-dt kernels with several waves a cluster, whatever order the waves run in: their own
 source on the CPU (wave_model), with one wave far behind or far ahead of the others, or in a
 random order.  The workgroup barriers must meet at the same place in every wave, and counts and
-live steps must be those of the replay harness."""
+live steps must be those of the replay harness; the work counted must not depend on the order."""
 import numpy as np
 import pytest
 
@@ -72,3 +72,18 @@ def test_wider_blocks(model, waves):
             assert error == ""
             np.testing.assert_array_equal(got, ref)
             np.testing.assert_array_equal(live, ref_live)
+
+
+@pytest.mark.parametrize("kind", ["sparse", "tail", "many", "two_channel"])
+@pytest.mark.parametrize("waves", [2, 4, 8])
+@pytest.mark.parametrize("form", [wm.LDS, wm.SCRATCH_ALL])
+def test_work_does_not_depend_on_the_order(model, kind, waves, form):
+    runs = _runs(kind)
+    ref = None
+    for schedule, seed in _schedules(waves):
+        _, _, work, error = model.run(runs, waves, form=form, persistent=form != wm.LDS,
+                                      schedule=schedule, schedule_seed=seed)
+        assert error == ""
+        if ref is None:
+            ref = work
+        np.testing.assert_array_equal(work, ref, err_msg=f"schedule {schedule} (seed {seed})")
