@@ -32,7 +32,8 @@ struct Ctx {
     double quiet_window = 1.0;
     double fixed_thresholds = 1.0;
     double waves_per_cluster = 0.0; // wavefronts per fixed-dt cluster: 1, 2, 4, 8 or 0 (chosen per launch)
-    double mlp_fused = 1.0;        // surrogate inference as one kernel (1) or per layer (0)
+    double mlp_fused = 1.0;        // surrogate inference as one kernel (1) or per layer (0);
+                                   // a network made at 0 also trains layer by layer
     double global_memory = 0.0;    // fixed-dt clusters in the global-memory form: 0 when
                                    // they exceed LDS, 1 always
     std::string err;

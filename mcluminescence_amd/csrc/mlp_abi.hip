@@ -506,7 +506,8 @@ int mcl_mlp_create(void* ctxp, const mcl_mlp_desc* desc, void** out)
         m->fused_lds = M::infer_fused_lds(m->fnet);
         m->fused_ok = M::infer_fused_ok(m->fnet) && m->fused_lds <= c->max_lds &&
                       M::infer_fused_prepare(m->fused_lds) == hipSuccess;
-        m->train_fused = m->fused_ok && M::train_fused_ok(m->fnet, c->max_lds) &&
+        m->train_fused = m->fused_ok && c->mlp_fused != 0.0 &&
+                         M::train_fused_ok(m->fnet, c->max_lds) &&
                          M::train_fused_prepare() == hipSuccess;
         (void)hipGetLastError();
         for (Layer& s : m->L) {
