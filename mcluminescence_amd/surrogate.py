@@ -264,6 +264,7 @@ class Network:
                   "mcl_mlp_create")
         self.handle = h
         self._torch_stream = None
+        self._entered = False              # the context is set to the network's stream
         self.n_params = int(self.lib.mcl_mlp_param_count(h))
         self.set_params(default_params(self.desc, seed) if params is None else params)
 
@@ -298,21 +299,31 @@ class Network:
     @contextlib.contextmanager
     def _on_stream(self, *tensors):
         """Run library calls on the network's own torch stream, ordered after the
-        caller's current stream and before its later work."""
+        caller's current stream and before its later work.  Calls made inside (the steps
+        of an epoch) are on that stream already and make no handshake of their own."""
         import torch
         if self._torch_stream is None:
             self._torch_stream = torch.cuda.Stream()
         caller = torch.cuda.current_stream()
         s = self._torch_stream
+        if self._entered and caller == s:
+            for t in tensors:
+                if t is not None:
+                    t.record_stream(s)
+            self.ctx.set_stream(s.cuda_stream)   # (another network's call may have reset it)
+            yield
+            return
         s.wait_stream(caller)
         for t in tensors:
             if t is not None:
                 t.record_stream(s)
         self.ctx.set_stream(s.cuda_stream)
+        self._entered = True
         try:
             with torch.cuda.stream(s):
                 yield
         finally:
+            self._entered = False
             self.ctx.set_stream(None)
             caller.wait_stream(s)
 
@@ -404,6 +415,10 @@ def train(net: Network, x, t, cfg: TrainConfig = TrainConfig(),
     gen = torch.Generator(device="cpu").manual_seed(cfg.seed)
     loss_buf = torch.zeros(total, dtype=torch.float32, device=x.device)
     hp = AdamW(cfg.lr, cfg.beta1, cfg.beta2, cfg.eps, cfg.weight_decay, 0)
+    # (the library's own step without the lifetimes and handshake that the epoch's cover, 5 us of
+    # host time a step; a train_step of the caller's is called as it is)
+    own = getattr(net.train_step, "__func__", None) is Network.train_step
+    take_step = net._step if own else net.train_step
     step = 0
     t0 = time.time()
     ms = []
@@ -421,7 +436,7 @@ def train(net: Network, x, t, cfg: TrainConfig = TrainConfig(),
                     lr = cfg.lr_min + 0.5 * (cfg.lr - cfg.lr_min) * (1.0 + math.cos(math.pi * f))
                 hp.lr = lr
                 hp.step = step
-                net._step(x, t, perm[b * cfg.batch:(b + 1) * cfg.batch], hp, loss_buf[step - 1:step])
+                take_step(x, t, perm[b * cfg.batch:(b + 1) * cfg.batch], hp, loss_buf[step - 1:step])
         ms.append(net.last_ms())
         if log and (ep % max(1, cfg.epochs // 10) == 0 or ep == cfg.epochs - 1):
             torch.cuda.synchronize()
