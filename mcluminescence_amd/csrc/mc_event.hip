@@ -121,7 +121,7 @@ __device__ __forceinline__ void run_cluster_event(const EventArgs& a, const int 
     uint32_t* cstart = (uint32_t*)(hole + h_cap);
     uint32_t* est = (uint32_t*)ebase;
     float* ew = (float*)(est + e_cap);
-    double* rtot = (double*)(ew + e_cap);            // row sums (the ethr words)
+    double* rtot = (double*)(ew + e_cap);            // [e_cap / 64] row sums (in e_cap words)
     uint32_t* rq = (uint32_t*)(ew + e_cap) + e_cap;
 
     const uint32_t k0 = a.key0, k1 = a.key1;
